@@ -378,18 +378,111 @@ __global__ void cg_xclear_kernel(CGState* __restrict__ st) { st->xfrom = st->ite
 
 // --- fused iteration forms (CSR operator, P = I or Jacobi) ------------------
 // Form 1 keeps the four-kernel order but computes partial(p.u) in the SpMM
-// epilogue (cg_dir_spmm_kernel with FORM = false), saving the separate p.u pass.
-// Form 2 has two vector kernels per iteration instead of four:
-//   K1 (cg_dir_spmm_kernel):  p = z + beta p_prev;  u = A p;  partial(p.u)
-//   K2 (cg_step_kernel):      x += alpha p;  r -= alpha u;  partial(r.z)
+// epilogue (cg_spmm_kernel), saving the separate p.u pass.
+// Form 2 is two kernels per iteration and nothing between them:
+//   K1 (cg_dir_spmm_kernel):  rho = r.z, beta, stop test;  p = z + beta p_prev;  u = A p;
+//                             partial(p.u)
+//   K2 (cg_step_kernel):      alpha = rho / p.u;  x += alpha p;  r -= alpha u;  partial(r.z)
 // with z = r (P = I) or z = d r (Jacobi) formed where it is needed and never
-// stored.  p is double-buffered by the parity of the iteration count: K1 of
+// stored.  p is double-buffered by the parity of the iteration: K1 of
 // iteration t writes p[t & 1] and reads p[(t - 1) & 1]; p[1] is zero before the
 // first iteration, where beta = 0, so p = z exactly as after the reference's
 // copy (ConjugateGradient.hpp:247-253).  A row needs p of the rows its columns
 // name, which other workgroups write in the same launch; it recomputes them from
 // z and p_prev with the same fused multiply-add, so the values are bitwise those
 // the owners store and no workgroup reads what another writes.
+// The scalars: every workgroup adds the previous kernel's workgroup partials itself, in
+// one fixed order (block_totals), so all of them hold the same alpha, beta and stop
+// decision; workgroup 0 of K1 keeps rho of iteration t in rho slot t & 1, which K2 and the
+// next K1 read.  The first K1 of a block of iterations takes beta and rho from the state
+// (the host's hook may have changed them); cg_rho2_kernel closes a block.
+// What bounds the iteration of such a small system is the latency of its kernels: with a
+// one-workgroup kernel for alpha and one for rho between them (4.4 us each) an iteration
+// of a 45^3 grid with one right-hand side took 21.3 us.
+
+struct FusedScalars {
+    const double* rz;   // r.z partials of the previous K2 ...
+    int rzB;            // ... of this many workgroups
+    double* slots;      // rho of the last two iterations, 2 x k
+    int par;            // parity of this iteration
+    int first;          // 1: first iteration of a block (beta and rho from the state)
+};
+
+// Stop test and beta of K1 into LDS; true when the solve has stopped (for every thread of
+// every workgroup alike).  Workgroup 0 records rho, the iteration count and a stop.
+__device__ __forceinline__ bool fused_beta(const FusedScalars& F, int k, int kpad, double* be, double* scratch,
+                                           CGState* st) {
+    const int c = threadIdx.x;
+    const int done = st->done, guard = st->guard;
+    if (F.first) {
+        if (done) return true;
+        if (c < k) {
+            be[c] = st->beta[c];
+            if (blockIdx.x == 0) F.slots[(int64_t)F.par * k + c] = st->rho[c];
+        }
+        __syncthreads();
+        return false;
+    }
+    __shared__ int going;
+    if (threadIdx.x == 0) going = 0;
+    double rz = 0.0, old = 0.0, beta = 0.0, lim = 0.0;
+    if (c < k) {  // in flight with the partials
+        old = F.slots[(int64_t)(F.par ^ 1) * k + c];
+        lim = st->TOL[c];
+    }
+    block_totals(F.rz, F.rzB, k, kpad, be, scratch);
+    if (done) return true;
+    if (c < k) {
+        rz = be[c];
+        beta = (guard && !(old != 0.0)) ? 0.0 : rz / old;  // guard: a column whose r vanished
+        if (!(fabs(rz) <= lim)) going = 1;
+        be[c] = beta;
+    }
+    __syncthreads();
+    const bool stop = !going;
+    if (blockIdx.x == 0) {
+        if (c < k) {
+            F.slots[(int64_t)F.par * k + c] = rz;
+            if (stop) {
+                st->rho_old[c] = old;
+                st->rho[c] = rz;
+                st->beta[c] = beta;
+            }
+        }
+        if (threadIdx.x == 0) {
+            st->iter += 1;
+            if (stop) {
+                st->succeeded = 1;
+                st->done = 1;  // the workgroups that see it at their start stop for the same reason
+            }
+        }
+    }
+    return stop;
+}
+
+// After the last K2 of a block: rho, beta, the stop test and the count of its iteration
+// into the state, as the next K1 would have found them.
+__global__ __launch_bounds__(kBlock) void cg_rho2_kernel(int k, int kpad, FusedScalars F, CGState* __restrict__ st) {
+    if (st->done) return;
+    __shared__ double tot[kMaxCols], scratch[kBlock];
+    __shared__ int going;
+    if (threadIdx.x == 0) going = 0;
+    block_totals(F.rz, F.rzB, k, kpad, tot, scratch);
+    const int c = threadIdx.x;
+    if (c < k) {
+        const double rz = tot[c], old = F.slots[(int64_t)F.par * k + c];
+        st->rho_old[c] = old;
+        st->rho[c] = rz;
+        st->beta[c] = (st->guard && !(old != 0.0)) ? 0.0 : rz / old;
+        if (!(fabs(rz) <= st->TOL[c])) going = 1;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        st->succeeded = going ? 0 : 1;
+        st->iter += 1;
+        st->done = (!going || st->iter >= st->max_iter) ? 1 : 0;
+    }
+}
 
 // One row per lane group of G lanes; each lane holds V consecutive columns of a
 // G*V-column tile (k > G*V only for G = 64: further tiles).  The workgroup's p.u
@@ -402,21 +495,24 @@ __global__ void cg_xclear_kernel(CGState* __restrict__ st) { st->xfrom = st->ite
 // panels before and after, which the workgroups of the same XCD (contiguous
 // offsets after xcd_swizzle) work on at about the same time, so p rows are reused
 // from the L2 instead of being fetched again for each neighbouring plane.
-// FORM = false is the plain "u = A p, partial(p.u)" step of the three-pass
-// iteration (p formed by cg_p_kernel in ring slot iter % xdefer from p0 on, pstride
-// elements apart; r, d, p1 unused).
-template <typename T, typename RP, int G, int V, bool FORM, bool HAS_D>
-__global__ __launch_bounds__(kBlock) void cg_dir_spmm_kernel(int n, int k, const RP* __restrict__ rp,
+// p was formed by cg_p_kernel in ring slot iter % xdefer (p0 = slot 0, pstride elements
+// apart).
+// A lane holds PER of its group's (column, value) pairs, so that narrow groups (k = 1: a
+// lane per row) still load eight of them at once and gather four at a time; their lanes
+// read a cache line in several loads, so it must not be fetched non-temporally (form 2 on
+// 100^3, k = 1: 83 us a call with it, 33 us without).
+template <typename T, typename RP, int G, int V>
+__global__ __launch_bounds__(kBlock) void cg_spmm_kernel(int n, int k, const RP* __restrict__ rp,
                                                              const int32_t* __restrict__ ci, const T* __restrict__ a,
-                                                             const T* __restrict__ r, const T* __restrict__ d,
-                                                             T* __restrict__ p0, T* __restrict__ p1,
-                                                             int64_t pstride, T* __restrict__ u,
+                                                             const T* __restrict__ p0, int64_t pstride, T* __restrict__ u,
                                                              double* __restrict__ partial,
                                                              const CGState* __restrict__ st, int panel) {
     if (st->done) return;
     constexpr int S = kWave / G;  // rows in flight per wave
     constexpr int KT = G * V;     // columns per tile
     constexpr int WAVES = kBlock / kWave;
+    constexpr int PER = G >= 8 ? 1 : 8 / G;  // pairs per lane of a chunk
+    constexpr int CH = G * PER;              // pairs per chunk
     // gathers in flight per lane and round (8 measured slower on the 128^3
     // Laplacian: 86 VGPRs and 5 waves per SIMD instead of 56 and 8)
     constexpr int U = 4;
@@ -442,10 +538,7 @@ __global__ __launch_bounds__(kBlock) void cg_dir_spmm_kernel(int n, int k, const
         sw = 1;
         cnt = (int)((int64_t)n * (lb + 1) / B) - first;
     }
-    const bool odd = FORM && (st->iter & 1) != 0;
-    // FORM: written by the previous iteration; else ring slot iter % xdefer (p0 = slot 0)
-    const T* __restrict__ pp = FORM ? (odd ? p0 : p1) : p0 + (int64_t)(st->iter % st->xdefer) * pstride;
-    T* __restrict__ pn = odd ? p1 : p0;
+    const T* __restrict__ pp = p0 + (int64_t)(st->iter % st->xdefer) * pstride;
     for (int qb = wave * S; qb < cnt; qb += WAVES * S) {
         const int q = qb + s;
         const int row = P > 0 ? first + (q / sw) * P + q % sw : first + q;
@@ -455,34 +548,39 @@ __global__ __launch_bounds__(kBlock) void cg_dir_spmm_kernel(int n, int k, const
         int wmax = len;  // longest row of the wave (uniform loop bound)
 #pragma unroll
         for (int off = G; off < kWave; off <<= 1) wmax = max(wmax, __shfl_xor(wmax, off, kWave));
-        const T di = (HAS_D && rok) ? d[row] : T(1);
         for (int c0 = 0; c0 < k; c0 += KT) {
             const int col = c0 + g * V;
             const bool colok = col < k;
             const int colc = colok ? col : 0;
-            T be[V];
-#pragma unroll
-            for (int i = 0; i < V; ++i) be[i] = FORM ? (T)st->beta[colc + i] : T(0);
             T acc[V];
 #pragma unroll
             for (int i = 0; i < V; ++i) acc[i] = T(0);
-            // the row's own r and p_prev (p for FORM = false), issued before the
-            // gathers so they are in flight with them (clamped to a valid row)
-            const int64_t own = (int64_t)(rok ? row : first) * k + colc;
-            T rv_own[V], pv_own[V];
-            if constexpr (FORM) load_vec<T, V>(r + own, rv_own);
-            load_vec<T, V>(pp + own, pv_own);
-            for (int base = 0; base < wmax; base += G) {
-                const int e = base + g;
-                int32_t myc = 0;
-                T mya = T(0);
-                if (e < len) {
-                    myc = __builtin_nontemporal_load(ci + lo + e);
-                    mya = a ? __builtin_nontemporal_load(a + lo + e) : T(1);
+            // the row's own p, issued before the gathers so that it is in flight with them
+            // (clamped to a valid row)
+            T pv_own[V];
+            load_vec<T, V>(pp + (int64_t)(rok ? row : first) * k + colc, pv_own);
+            for (int base = 0; base < wmax; base += CH) {
+                int32_t myc[PER];
+                T mya[PER];
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    const int e = base + g + q * G;
+                    if constexpr (PER > 1) {  // clamped: some row of the wave has a nonzero, so 0 is valid
+                        const RP at = max(lo + min(e, len - 1), RP(0));
+                        myc[q] = ci[at];
+                        mya[q] = a ? a[at] : T(1);
+                    } else {
+                        myc[q] = 0;
+                        mya[q] = T(0);
+                        if (e < len) {
+                            myc[q] = __builtin_nontemporal_load(ci + lo + e);
+                            mya[q] = a ? __builtin_nontemporal_load(a + lo + e) : T(1);
+                        }
+                    }
                 }
-                const int cnt = min(G, len - base);  // this group's pairs in the chunk
-                const int wcnt = min(G, wmax - base);
-                for (int u0 = 0; u0 < wcnt; u0 += U) {
+                const int cnt = min(CH, len - base);  // this group's pairs in the chunk
+                const int wcnt = min(CH, wmax - base);
+                auto round = [&](int u0) {
                     // U (column, value) pairs from the group's lanes, then all their
                     // gathers in flight together, then the arithmetic
                     int cj[U];
@@ -491,48 +589,39 @@ __global__ __launch_bounds__(kBlock) void cg_dir_spmm_kernel(int n, int k, const
 #pragma unroll
                     for (int uu = 0; uu < U; ++uu) {
                         const int j = u0 + uu;
-                        const int src = s * G + (j < G ? j : 0);
-                        const int32_t c = __shfl(myc, src, kWave);
-                        av[uu] = __shfl(mya, src, kWave);
+                        int32_t c;
+                        if constexpr (G == 1) {
+                            c = myc[j % PER];
+                            av[uu] = mya[j % PER];
+                        } else {  // pair j is in lane j % G's slot j / G
+                            const int src = s * G + (PER > 1 ? j % G : (j < G ? j : 0));
+                            c = __shfl(myc[PER == 1 ? 0 : (j / G) % PER], src, kWave);
+                            av[uu] = __shfl(mya[PER == 1 ? 0 : (j / G) % PER], src, kWave);
+                        }
                         live[uu] = (j < cnt) && colok;
                         cj[uu] = live[uu] ? c : 0;
                     }
-                    T rv[U][V], pv[U][V], dj[U];
+                    T pv[U][V];
 #pragma unroll
-                    for (int uu = 0; uu < U; ++uu) {
-                        const int64_t o = (int64_t)cj[uu] * k + colc;
-                        if constexpr (FORM) load_vec<T, V>(r + o, rv[uu]);
-                        load_vec<T, V>(pp + o, pv[uu]);
-                        dj[uu] = HAS_D ? d[cj[uu]] : T(1);
-                    }
+                    for (int uu = 0; uu < U; ++uu) load_vec<T, V>(pp + (int64_t)cj[uu] * k + colc, pv[uu]);
 #pragma unroll
                     for (int uu = 0; uu < U; ++uu) {
 #pragma unroll
-                        for (int i = 0; i < V; ++i) {
-                            T pj = pv[uu][i];
-                            if constexpr (FORM) {
-                                const T z = HAS_D ? dj[uu] * rv[uu][i] : rv[uu][i];
-                                pj = fma_t(be[i], pv[uu][i], z);
-                            }
-                            acc[i] += live[uu] ? av[uu] * pj : T(0);
-                        }
+                        for (int i = 0; i < V; ++i) acc[i] += live[uu] ? av[uu] * pv[uu][i] : T(0);
                     }
+                };
+                if constexpr (PER > 1) {  // CH = 8: two rounds, so that a pair's slot is a constant
+                    round(0);
+                    if (wcnt > U) round(U);
+                } else {
+                    for (int u0 = 0; u0 < wcnt; u0 += U) round(u0);
                 }
             }
             if (rok && colok) {
                 const int64_t o = (int64_t)row * k + col;
-                T pi[V];
                 double* shs = sh + (int64_t)slot * k + col;
 #pragma unroll
-                for (int i = 0; i < V; ++i) {
-                    pi[i] = pv_own[i];
-                    if constexpr (FORM) {
-                        const T z = HAS_D ? di * rv_own[i] : rv_own[i];
-                        pi[i] = fma_t(be[i], pv_own[i], z);
-                    }
-                    shs[i] += (double)pi[i] * (double)acc[i];
-                }
-                if constexpr (FORM) store_vec<T, V>(pn + o, pi);
+                for (int i = 0; i < V; ++i) shs[i] += (double)pv_own[i] * (double)acc[i];
                 store_vec<T, V>(u + o, acc);
             }
         }
@@ -546,32 +635,249 @@ __global__ __launch_bounds__(kBlock) void cg_dir_spmm_kernel(int n, int k, const
     for (int c = threadIdx.x; c < k; c += kBlock) partial[(int64_t)lb * k + c] = sh[c];
 }
 
-// x = (first ? 0 : x) + alpha p;  r -= alpha u;  partial(r.z), z = r or d r
+// K1: cg_spmm_kernel's lanes, pairs and row order, with p formed of the row and of its
+// neighbours, and the scalars in front; a group's p.u of its columns stays in registers
+// (G < 64), its first row's pairs are loaded before the totals.
+template <typename T, typename RP, int G, int V, bool HAS_D>
+__global__ __launch_bounds__(kBlock) void cg_dir_spmm_kernel(int n, int k, const RP* __restrict__ rp,
+                                                             const int32_t* __restrict__ ci, const T* __restrict__ a,
+                                                             const T* __restrict__ r, const T* __restrict__ d,
+                                                             T* __restrict__ p0, T* __restrict__ p1, T* __restrict__ u,
+                                                             double* __restrict__ partial,
+                                                             CGState* __restrict__ st, int panel, int kpad,
+                                                             FusedScalars F) {
+    constexpr int S = kWave / G;  // rows in flight per wave
+    constexpr int KT = G * V;     // columns per tile
+    constexpr int WAVES = kBlock / kWave;
+    constexpr int PER = G >= 8 ? 1 : 8 / G;  // pairs per lane of a chunk
+    constexpr int CH = G * PER;              // pairs per chunk
+    constexpr int U = 4;  // gathers in flight per lane and round
+
+    __shared__ double sh[WAVES * kWave * 4];  // WAVES * k <= 1024, and kBlock for the totals
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int s = lane / G, g = lane % G;
+    const int B = gridDim.x;
+    const int lb = xcd_swizzle(blockIdx.x, B);
+    // rows: q in [0, cnt) -> first + (q / sw) * P + q % sw (panel order) or first + q
+    int first, sw, cnt, P;
+    if (panel > 0) {
+        P = panel;
+        first = (int)((int64_t)P * lb / B);
+        sw = (int)((int64_t)P * (lb + 1) / B) - first;
+        cnt = sw * ((n + P - 1) / P);
+    } else {
+        P = 0;
+        first = (int)((int64_t)n * lb / B);
+        sw = 1;
+        cnt = (int)((int64_t)n * (lb + 1) / B) - first;
+    }
+    // a group's row of pass qb: its nonzeros, and the longest row of the wave
+    int row, len, wmax;
+    bool rok;
+    RP lo;
+    auto load_row = [&](int qb) {
+        const int q = qb + s;
+        row = P > 0 ? first + (q / sw) * P + q % sw : first + q;
+        rok = q < cnt && row < n;
+        const RP r0 = rok ? rp[row] : RP(0), r1 = rok ? rp[row + 1] : RP(0);
+        lo = r0;
+        len = (int)(r1 - r0);
+        wmax = len;
+#pragma unroll
+        for (int off = G; off < kWave; off <<= 1) wmax = max(wmax, __shfl_xor(wmax, off, kWave));
+    };
+    int32_t myc[PER];
+    T mya[PER];
+    auto load_pairs = [&](int base) {  // wmax > base: the wave has a nonzero, so position 0 is valid
+#pragma unroll
+        for (int q = 0; q < PER; ++q) {
+            const RP at = max(lo + min(base + g + q * G, len - 1), RP(0));
+            // narrow groups read a cache line in several loads: it has to stay
+            myc[q] = PER > 1 ? ci[at] : __builtin_nontemporal_load(ci + at);
+            mya[q] = !a ? T(1) : PER > 1 ? a[at] : __builtin_nontemporal_load(a + at);
+        }
+    };
+    // the first row's pairs are on their way while the previous kernel's partials are added
+    load_row(wave * S);
+    if (wmax > 0) load_pairs(0);
+    __shared__ double sbe[kMaxCols];
+    if (fused_beta(F, k, kpad, sbe, sh, st)) return;
+    double pu[V];  // this lane's columns' p.u (G < 64: all columns in one tile); else in sh
+#pragma unroll
+    for (int i = 0; i < V; ++i) pu[i] = 0.0;
+    if constexpr (G == 64) {
+        for (int i = threadIdx.x; i < WAVES * k; i += kBlock) sh[i] = 0.0;
+        __syncthreads();
+    }
+    const T* __restrict__ pp = F.par ? p0 : p1;
+    T* __restrict__ pn = F.par ? p1 : p0;
+    for (int qb = wave * S; qb < cnt; qb += WAVES * S) {
+        const bool later = qb != wave * S;
+        if (later) load_row(qb);
+        const T di = (HAS_D && rok) ? d[row] : T(1);
+        for (int c0 = 0; c0 < k; c0 += KT) {
+            const int col = c0 + g * V;
+            const bool colok = col < k;
+            const int colc = colok ? col : 0;
+            T be[V];
+#pragma unroll
+            for (int i = 0; i < V; ++i) be[i] = (T)sbe[colc + i];
+            T acc[V];
+#pragma unroll
+            for (int i = 0; i < V; ++i) acc[i] = T(0);
+            // the row's own r and p_prev, issued before the
+            // gathers so they are in flight with them (clamped to a valid row)
+            const int64_t own = (int64_t)(rok ? row : first) * k + colc;
+            T rv_own[V], pv_own[V];
+            load_vec<T, V>(r + own, rv_own);
+            load_vec<T, V>(pp + own, pv_own);
+            for (int base = 0; base < wmax; base += CH) {
+                if (later || base > 0 || c0 > 0) load_pairs(base);
+                const int cnt = min(CH, len - base);  // this group's pairs in the chunk
+                const int wcnt = min(CH, wmax - base);
+                auto round = [&](int u0) {
+                    // U (column, value) pairs from the group's lanes, then all their
+                    // gathers in flight together, then the arithmetic
+                    int cj[U];
+                    T av[U];
+                    bool live[U];
+#pragma unroll
+                    for (int uu = 0; uu < U; ++uu) {
+                        const int j = u0 + uu;  // pair j is in lane j % G's slot j / G
+                        int32_t c;
+                        if constexpr (G == 1) {
+                            c = myc[j % PER];
+                            av[uu] = mya[j % PER];
+                        } else {
+                            const int src = s * G + j % G;
+                            c = __shfl(myc[PER == 1 ? 0 : (j / G) % PER], src, kWave);
+                            av[uu] = __shfl(mya[PER == 1 ? 0 : (j / G) % PER], src, kWave);
+                        }
+                        live[uu] = (j < cnt) && colok;
+                        cj[uu] = live[uu] ? c : 0;
+                    }
+                    T rv[U][V], pv[U][V], dj[U];
+#pragma unroll
+                    for (int uu = 0; uu < U; ++uu) {
+                        const int64_t o = (int64_t)cj[uu] * k + colc;
+                        load_vec<T, V>(r + o, rv[uu]);
+                        load_vec<T, V>(pp + o, pv[uu]);
+                        dj[uu] = HAS_D ? d[cj[uu]] : T(1);
+                    }
+#pragma unroll
+                    for (int uu = 0; uu < U; ++uu) {
+#pragma unroll
+                        for (int i = 0; i < V; ++i) {
+                            const T z = HAS_D ? dj[uu] * rv[uu][i] : rv[uu][i];
+                            const T pj = fma_t(be[i], pv[uu][i], z);
+                            acc[i] += live[uu] ? av[uu] * pj : T(0);
+                        }
+                    }
+                };
+                if constexpr (PER > 1) {  // CH = 8: two rounds, so that a pair's slot is a constant
+                    round(0);
+                    if (wcnt > U) round(U);
+                } else {
+                    for (int u0 = 0; u0 < wcnt; u0 += U) round(u0);
+                }
+            }
+            if (rok && colok) {
+                const int64_t o = (int64_t)row * k + col;
+                T pi[V];
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    const T z = HAS_D ? di * rv_own[i] : rv_own[i];
+                    pi[i] = fma_t(be[i], pv_own[i], z);
+                    const double t = (double)pi[i] * (double)acc[i];
+                    if constexpr (G == 64)
+                        sh[(int64_t)wave * k + col + i] += t;
+                    else
+                        pu[i] += t;
+                }
+                store_vec<T, V>(pn + o, pi);
+                store_vec<T, V>(u + o, acc);
+            }
+        }
+    }
+    if constexpr (G < 64) {
+        // the lane groups of the wave in a fixed tree, then the waves
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+#pragma unroll
+            for (int off = kWave / 2; off >= G; off >>= 1) pu[i] += shfl_xor(pu[i], off);
+        }
+        __syncthreads();  // sh may still be read (totals)
+        if (lane < G) {
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+                if (g * V + i < k) sh[wave * k + g * V + i] = pu[i];
+        }
+    }
+    __syncthreads();
+    for (int c = threadIdx.x; c < k; c += kBlock) {
+        double t = sh[c];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) t += sh[w * k + c];
+        partial[(int64_t)lb * k + c] = t;
+    }
+}
+
+// alpha = rho / p.u from K1's partials;  x += alpha p;  r -= alpha u;  partial(r.z), z = r
+// or d r.  x is zero (or the guess) before the first iteration.  Loads of kRowsInFlight
+// rows first, at clamped rows, as in the r update, and the first ones before the totals.
 template <typename T, bool HAS_D>
-__global__ __launch_bounds__(kBlock) void cg_step_kernel(int n, int k, int kpad, const T* __restrict__ p0,
-                                                         const T* __restrict__ p1, const T* __restrict__ u,
-                                                         const T* __restrict__ d, T* __restrict__ x,
-                                                         T* __restrict__ r, double* __restrict__ partial,
+__global__ __launch_bounds__(kBlock) void cg_step_kernel(int n, int k, int kpad, const T* __restrict__ p,
+                                                         const T* __restrict__ u, const T* __restrict__ d,
+                                                         T* __restrict__ x, T* __restrict__ r,
+                                                         const double* __restrict__ pu, int puB,
+                                                         const double* __restrict__ rho, double* __restrict__ partial,
                                                          const CGState* __restrict__ st) {
-    if (st->done) return;
+    __shared__ double tot[kMaxCols], scratch[kBlock];
     int i0, i1;
     block_row_range(n, i0, i1);
     const Lanes L = lanes_of(kpad);
-    const T* __restrict__ p = (st->iter & 1) ? p1 : p0;
-    const bool first = (st->iter == 0) && !st->use_guess;
+    const int c = L.c < k ? L.c : 0;
+    T xv[kRowsInFlight], pv[kRowsInFlight], rv[kRowsInFlight], uv[kRowsInFlight], dv[kRowsInFlight];
+    int64_t e[kRowsInFlight];
+    auto load = [&](int ib) {
+#pragma unroll
+        for (int q = 0; q < kRowsInFlight; ++q) {
+            const int i = max(min(ib + q * L.rows, i1 - 1), 0);
+            e[q] = (int64_t)i * k + c;
+            xv[q] = x[e[q]];
+            pv[q] = p[e[q]];
+            rv[q] = r[e[q]];
+            uv[q] = u[e[q]];
+            dv[q] = HAS_D ? d[i] : T(1);
+        }
+    };
+    // the first rows, the flag and the partials are all in flight together: a round trip
+    // to memory is most of such a kernel's time
+    const int done = st->done, guard = st->guard;
+    const double rh = rho[c];
+    load(i0 + L.ro);
+    block_totals(pu, puB, k, kpad, tot, scratch);
+    if (done) return;
     double acc = 0.0;
     if (L.c < k) {
-        const T al = (T)st->alpha[L.c];
-        for (int i = i0 + L.ro; i < i1; i += L.rows) {
-            const int64_t e = (int64_t)i * k + L.c;
-            x[e] = x_step(first, x[e], al, p[e]);
-            const T rv = r[e] - al * u[e];
-            r[e] = rv;
-            const T zv = HAS_D ? d[i] * rv : rv;
-            acc += (double)rv * (double)zv;
+        // guard: a column whose direction has vanished stops moving, as in cg_alpha_kernel
+        const double t = tot[c];
+        const T al = (T)((guard && !(t > 0.0)) ? 0.0 : rh / t);
+        for (int ib = i0 + L.ro; ib < i1; ib += kRowsInFlight * L.rows) {
+            if (ib != i0 + L.ro) load(ib);
+#pragma unroll
+            for (int q = 0; q < kRowsInFlight; ++q) {
+                if (ib + q * L.rows < i1) {
+                    x[e[q]] = fma_t(al, pv[q], xv[q]);
+                    const T rn = rv[q] - al * uv[q];
+                    r[e[q]] = rn;
+                    const T zv = HAS_D ? dv[q] * rn : rn;
+                    acc += (double)rn * (double)zv;
+                }
+            }
         }
     }
-    column_partial(acc, L, k, kpad, partial);
+    column_partial_wave(acc, k, kpad, scratch, partial);
 }
 
 template <typename T>
@@ -632,10 +938,10 @@ size_t cg_workspace_bytes(int32_t n, int32_t k, size_t vs, int prec_kind, int sl
 // Iteration form for CSR operators with P = I or Jacobi, short rows (mean length
 // <= 16) and no column slabs ("cg_fused"): 0 = four vector kernels after the
 // SpMM; 1 = p.u in the SpMM epilogue (kSpmmDot); 2 = direction, SpMM and p.u in
-// one kernel (kFormDir); 3 = default (form 2 up to 2^20 entries n * nrhs, form 1
-// above).  On the 128^3 Laplacian with 32 right-hand sides form 1 measured fastest in
+// one kernel (kFormDir); 3 = default (form 2 up to 2^20 entries n * nrhs, and up to 2^21
+// with at most 4 right-hand sides; form 1 above).  On the 128^3 Laplacian with 32 right-hand sides form 1 measured fastest in
 // FP64 and FP32: gathering both z and p_prev per nonzero (form 2) cost more than
-// streaming p once; on small blocks form 2's one launch less per iteration wins.  Other
+// streaming p once; on small blocks form 2's two launches instead of five win.  Other
 // operators always take form 0.
 enum CgForm : int { kFourKernels = 0, kSpmmDot = 1, kFormDir = 2, kFormAuto = 3 };
 static int g_cg_fused = kFormAuto;
@@ -684,18 +990,19 @@ int32_t cg_tune_get(const char* key) {
 template <typename T, typename RP, int V>
 static int launch_dir_v(int G, int form, bool has_d, hipStream_t s, int n, int k, const RP* rp, const int32_t* ci,
                         const T* a, const T* r, const T* d, T* p0, T* p1, int64_t pstride, T* u, double* partial,
-                        const CGState* st, int panel) {
-#define TG_DIRK(GG, FORM, HD)                                                                                  \
-    hipLaunchKernelGGL((cg_dir_spmm_kernel<T, RP, GG, V, FORM, HD>), dim3(kFusedBlocks), dim3(kBlock), 0, s, n, k, \
-                       rp, ci, a, r, d, p0, p1, pstride, u, partial, st, panel)
-#define TG_DIR(GG)                     \
-    case GG:                           \
-        if (form != kFormDir)          \
-            TG_DIRK(GG, false, false); \
-        else if (has_d)                \
-            TG_DIRK(GG, true, true);   \
-        else                           \
-            TG_DIRK(GG, true, false);  \
+                        CGState* st, int panel, int blocks, int kpad, const FusedScalars& F) {
+#define TG_DIRK(GG, HD)                                                                                          \
+    hipLaunchKernelGGL((cg_dir_spmm_kernel<T, RP, GG, V, HD>), dim3(blocks), dim3(kBlock), 0, s, n, k, rp, ci, a, \
+                       r, d, p0, p1, u, partial, st, panel, kpad, F)
+#define TG_DIR(GG)                                                                                                  \
+    case GG:                                                                                                        \
+        if (form != kFormDir)                                                                                       \
+            hipLaunchKernelGGL((cg_spmm_kernel<T, RP, GG, V>), dim3(blocks), dim3(kBlock), 0, s, n, k, rp, ci, a, p0, \
+                               pstride, u, partial, (const CGState*)st, panel);                                     \
+        else if (has_d)                                                                                             \
+            TG_DIRK(GG, true);                                                                                      \
+        else                                                                                                        \
+            TG_DIRK(GG, false);                                                                                     \
         break;
     switch (G) {
         TG_DIR(1)
@@ -715,30 +1022,44 @@ static int launch_dir_v(int G, int form, bool has_d, hipStream_t s, int n, int k
 
 // The SpMM kernel of forms 1 and 2: V columns per lane (16-byte loads where k
 // allows), G = enough lanes for all k columns (at most 64; then k / (64 V) tiles).
+static void dir_shape(int k, size_t vs, int& V, int& G) {
+    if (vs == 8)
+        V = (k % 2 == 0) ? 2 : 1;  // 4 doubles per lane measured slower on the 128^3 Laplacian
+    else
+        V = (k % 4 == 0) ? 4 : (k % 2 == 0) ? 2 : 1;
+    G = 1;
+    while (G < 64 && G * V < k) G *= 2;
+}
+
+// Workgroups of form 2's kernels: one pass over the rows each where that gives few
+// enough, and at most 1024 and 8192 / k (each workgroup adds all of the other kernel's
+// partials, B k values, before it starts).
+static int fused_blocks(int n, int k, size_t vs) {
+    int V, G;
+    dir_shape(k, vs, V, G);
+    const int per = kBlock / G;
+    const int most = std::min(kFusedBlocks / 2, std::max(256, 4096 / k));
+    return std::max(1, std::min(most, (n + per - 1) / per));
+}
+
 template <typename T, typename RP>
 static int launch_dir(int form, hipStream_t s, int n, int k, const RP* rp, const int32_t* ci, const T* a,
                       const T* r, const T* d, T* p0, T* p1, int64_t pstride, T* u, double* partial,
-                      const CGState* st, int panel) {
-    int V = 1;
-    if (sizeof(T) == 8) {
-        V = (k % 2 == 0) ? 2 : 1;  // 4 doubles per lane measured slower on the 128^3 Laplacian
-    } else {
-        V = (k % 4 == 0) ? 4 : (k % 2 == 0) ? 2 : 1;
-    }
-    int G = 1;
-    while (G < 64 && G * V < k) G *= 2;
+                      CGState* st, int panel, int blocks, int kpad, const FusedScalars& F) {
+    int V, G;
+    dir_shape(k, sizeof(T), V, G);
     const bool has_d = d != nullptr;
     switch (V) {
         case 1:
             return launch_dir_v<T, RP, 1>(G, form, has_d, s, n, k, rp, ci, a, r, d, p0, p1, pstride, u, partial, st,
-                                                  panel);
+                                                  panel, blocks, kpad, F);
         case 2:
             return launch_dir_v<T, RP, 2>(G, form, has_d, s, n, k, rp, ci, a, r, d, p0, p1, pstride, u, partial, st,
-                                                  panel);
+                                                  panel, blocks, kpad, F);
         default:
             if constexpr (sizeof(T) == 4)
                 return launch_dir_v<T, RP, 4>(G, form, has_d, s, n, k, rp, ci, a, r, d, p0, p1, pstride, u, partial, st,
-                                                  panel);
+                                                  panel, blocks, kpad, F);
             return fail(TG_ERR_INVALID, "internal: bad vector width");
     }
 }
@@ -796,27 +1117,38 @@ int cg_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d, co
     const bool csr_ok = !host_ops && Aop.csr && n > 0 && Ac.m == n && Ac.n == n && Ac.nnz <= 16 * (int64_t)n &&
                         !spmm_uses_slabs(Ac, k) && Ac.rp && (Ac.nnz == 0 || Ac.ci) &&
                         Ac.val_type == (sizeof(T) == 8 ? TG_F64 : TG_F32);
-    // auto: form 2 (four launches per iteration) for blocks of up to 2^20 entries, where
-    // an iteration is bound by the kernels' fixed costs (22^3 and 45^3 Laplacians: 12 %
-    // faster), form 1 above (its SpMM gathers one vector instead of two)
-    int form = g_cg_fused == kFormAuto ? ((int64_t)n * k <= (int64_t(1) << 20) ? kFormDir : kSpmmDot) : g_cg_fused;
+    // auto: form 2 (two launches per iteration) for small blocks, where an iteration is
+    // bound by the kernels' latency; form 1 (five, its SpMM gathers one vector instead of
+    // two) above.  Measured, form 2 / form 1 a solve: 45^3 x 8 16.1 / 18.8 ms, 90^3 x 2
+    // 15.5 / 17.7, 110^3 x 1 22.5 / 27.3, 80^3 x 4 17.7 / 18.0, 64^3 x 8 37.8 / 36.6, 45^3 x 16
+    // 14.9 / 13.0, 128^3 x 1 (2^21 entries) 31.9 / 35.6.
+    const int64_t entries = (int64_t)n * k;
+    const bool small = entries <= (int64_t(1) << 20) || (k <= 4 && entries <= (int64_t(1) << 21));
+    int form = g_cg_fused == kFormAuto ? (small ? kFormDir : kSpmmDot) : g_cg_fused;
     if (!csr_ok) form = kFourKernels;
     const bool fused = form == kFormDir;
     // deferred x update: form 1 only (form 0's operator reads p at a fixed address, form 2
     // updates x in its step kernel)
     const int xdefer = form == kSpmmDot ? std::min(g_cg_xdefer, slots) : 1;
-    // panel order for the SpMM kernel of forms 1 / 2 (cg_dir_spmm_kernel): panels of
+    // panel order for the SpMM kernel of forms 1 / 2: panels of
     // one band, when that gives every workgroup at least 4 rows per panel and the
     // matrix at least 4 panels (the band as the caller measured it; none measured: off)
     int panel = 0;
     if (form != kFourKernels && g_cg_panel && Ac.band >= 4 * (int64_t)kFusedBlocks && (int64_t)n >= 4 * Ac.band)
         panel = (int)Ac.band;
-    auto dir_spmm_on = [&](hipStream_t ss) -> int {
+    // form 2: p.u partials in the lower half of `partial`, r.z partials in the upper; the
+    // two rho slots in the alpha history, which only the deferred x update uses
+    const int fb = fused ? fused_blocks(n, k, sizeof(T)) : kFusedBlocks;
+    double* rz_partial = partial + (size_t)(kPartialBlocks / 2) * k;
+    auto scalars = [&](int par, bool first) {
+        return FusedScalars{(const double*)rz_partial, fb, ahist, par, first ? 1 : 0};
+    };
+    auto dir_spmm_on = [&](hipStream_t ss, const FusedScalars& F) -> int {
         if (Ac.rp_type == TG_I64)
             return launch_dir<T, int64_t>(form, ss, n, k, (const int64_t*)Ac.rp, Ac.ci, (const T*)Ac.val, r, dd, p,
-                                          p1, pstride, u, partial, st, panel);
+                                          p1, pstride, u, partial, st, panel, fb, kpad, F);
         return launch_dir<T, int32_t>(form, ss, n, k, (const int32_t*)Ac.rp, Ac.ci, (const T*)Ac.val, r, dd, p, p1,
-                                      pstride, u, partial, st, panel);
+                                      pstride, u, partial, st, panel, fb, kpad, F);
     };
 
     // z = P r by callback, then partial(r.z) -- the external-preconditioner step
@@ -898,25 +1230,27 @@ int cg_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d, co
             TG_HIP(hipStreamSynchronize(s));
         }
     }
-    // One iteration's launches on stream ss (every kernel returns at once when `done` is set).
-    auto one_iteration = [&](hipStream_t ss) -> int {
+    // One iteration's launches on stream ss (every kernel returns at once when `done` is
+    // set); `at`: its position in a block of iterations, which ends with close_block, `t`:
+    // an iteration number of its parity.
+    auto one_iteration = [&](hipStream_t ss, int at, int t) -> int {
         if (fused) {
-            int rc1 = dir_spmm_on(ss);
+            const int par = t & 1;
+            int rc1 = dir_spmm_on(ss, scalars(par, at == 0));
             if (rc1) return rc1;
-            hipLaunchKernelGGL(cg_alpha_kernel, dim3(1), dim3(kFinalThreads), 0, ss, k, kpad, kFusedBlocks,
-                               (const double*)partial, ahist, st);
+            const T* pt = par ? p1 : p;
             if (dd)
-                hipLaunchKernelGGL((cg_step_kernel<T, true>), dim3(B), dim3(kBlock), 0, ss, n, k, kpad, (const T*)p,
-                                   (const T*)p1, (const T*)u, dd, x, r, partial, (const CGState*)st);
+                hipLaunchKernelGGL((cg_step_kernel<T, true>), dim3(fb), dim3(kBlock), 0, ss, n, k, kpad, pt,
+                                   (const T*)u, dd, x, r, (const double*)partial, fb,
+                                   (const double*)(ahist + (size_t)par * k), rz_partial, (const CGState*)st);
             else
-                hipLaunchKernelGGL((cg_step_kernel<T, false>), dim3(B), dim3(kBlock), 0, ss, n, k, kpad, (const T*)p,
-                                   (const T*)p1, (const T*)u, dd, x, r, partial, (const CGState*)st);
-            hipLaunchKernelGGL(cg_rho_kernel, dim3(1), dim3(kFinalThreads), 0, ss, k, kpad, B, (const double*)partial,
-                               st);
+                hipLaunchKernelGGL((cg_step_kernel<T, false>), dim3(fb), dim3(kBlock), 0, ss, n, k, kpad, pt,
+                                   (const T*)u, dd, x, r, (const double*)partial, fb,
+                                   (const double*)(ahist + (size_t)par * k), rz_partial, (const CGState*)st);
             return TG_OK;
         }
         if (form == kSpmmDot) {  // u = A p and partial(p.u) in one kernel
-            int rc1 = dir_spmm_on(ss);
+            int rc1 = dir_spmm_on(ss, FusedScalars{});
             if (rc1) return rc1;
             hipLaunchKernelGGL(cg_alpha_kernel, dim3(1), dim3(kFinalThreads), 0, ss, k, kpad, kFusedBlocks,
                                (const double*)partial, ahist, st);
@@ -939,6 +1273,11 @@ int cg_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d, co
                            (const double*)ahist, (const CGState*)st);
         return TG_OK;
     };
+    // `next`: a number of the parity of the iteration after the block's last
+    auto close_block = [&](hipStream_t ss, int next) {
+        if (fused)
+            hipLaunchKernelGGL(cg_rho2_kernel, dim3(1), dim3(kBlock), 0, ss, k, kpad, scalars((next + 1) & 1, false), st);
+    };
     // Blocks of kCgGraphIters iterations as one captured hipGraph (the CSR forms, whose
     // launches never allocate), captured after the first batch and replayed; batches
     // run as whole blocks where they can, the rest eagerly.  The same kernels in the
@@ -955,11 +1294,12 @@ int cg_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d, co
     } ig;
     while (!hflag[1] && launched < max_iter) {
         int todo = std::min(batch, max_iter - launched);
-        if (graphs && launched >= 4 && todo >= kCgGraphIters) {
+        if (graphs && launched >= 4 && launched % 2 == 0 && todo >= kCgGraphIters) {  // captured at an even iteration
             if (!ig.ex) {
                 if (!ig.cs) TG_HIP(hipStreamCreateWithFlags(&ig.cs, hipStreamNonBlocking));
                 TG_HIP(hipStreamBeginCapture(ig.cs, hipStreamCaptureModeThreadLocal));
-                for (int it = 0; it < kCgGraphIters && rc == TG_OK; ++it) rc = one_iteration(ig.cs);
+                for (int it = 0; it < kCgGraphIters && rc == TG_OK; ++it) rc = one_iteration(ig.cs, it, it);
+                if (rc == TG_OK) close_block(ig.cs, kCgGraphIters);
                 hipGraph_t g = nullptr;
                 const hipError_t ec = hipStreamEndCapture(ig.cs, &g);
                 if (rc) {
@@ -977,7 +1317,11 @@ int cg_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d, co
             for (; todo >= kCgGraphIters; todo -= kCgGraphIters, launched += kCgGraphIters)
                 TG_HIP(hipGraphLaunch(ig.ex, s));
         }
-        for (; todo > 0 && rc == TG_OK; --todo, ++launched) rc = one_iteration(s);
+        if (todo > 0) {
+            for (int at = 0; at < todo && rc == TG_OK; ++at) rc = one_iteration(s, at, launched + at);
+            launched += todo;
+            close_block(s, launched);
+        }
         if (rc) break;
         if (!fused) {  // x complete before the host looks at the state
             hipLaunchKernelGGL((cg_xfinish_kernel<T>), dim3(B), dim3(kBlock), 0, s, n, k, kpad, (const T*)p, pstride,

@@ -41,6 +41,22 @@ __device__ __forceinline__ void column_partial(double v, const Lanes& L, int k, 
     if (L.ro == 0 && L.c < k) partial[(int64_t)blockIdx.x * k + L.c] = sh[L.c];
 }
 
+// column_partial with the row lanes of a wave combined by cross-lane adds and the waves
+// through LDS (two barriers instead of up to nine): for kernels that are short enough for
+// the tree's barriers to show.  sh: kBlock doubles of LDS.
+__device__ __forceinline__ void column_partial_wave(double v, int k, int kpad, double* sh, double* partial) {
+    for (int off = kWave / 2; off >= kpad; off >>= 1) v += shfl_xor(v, off);
+    __syncthreads();  // sh may still be read
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    const int step = kpad > kWave ? kpad : kWave;
+    if (threadIdx.x < k) {
+        double t = sh[threadIdx.x];
+        for (int q = step; q < kBlock; q += step) t += sh[q + threadIdx.x];
+        partial[(int64_t)blockIdx.x * k + threadIdx.x] = t;
+    }
+}
+
 // Threads of the one-workgroup kernels that finish a reduction.
 constexpr int kFinalThreads = 1024;
 
@@ -75,6 +91,39 @@ __device__ __forceinline__ double column_total(const double* partial, int B, int
     const double t = sh[c];
     __syncthreads();
     return t;
+}
+
+// Totals of B workgroup partials per column, in a fixed order, by a workgroup of kBlock
+// threads that needs them itself: out[0 .. k) in LDS (scratch: kBlock doubles of LDS).
+// Thread (c, j) adds partials j, j + J, ... into four running sums, the lanes of a wave
+// and then the waves are combined in a fixed tree, so every workgroup that calls it gets
+// bitwise the same totals.  Saves the one-workgroup kernel between two passes where B k
+// is small enough (a few thousand values) for every workgroup to read.
+__device__ __forceinline__ void block_totals(const double* __restrict__ partial, int B, int k, int kpad, double* out,
+                                             double* scratch) {
+    const int c = threadIdx.x % kpad, j = threadIdx.x / kpad, J = kBlock / kpad;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    if (c < k) {
+        int b = j;
+        for (; b + 3 * J < B; b += 4 * J) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) s[q] += partial[(int64_t)(b + q * J) * k + c];
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q)  // fewer than 4 left
+            if (b + q * J < B) s[q] += partial[(int64_t)(b + q * J) * k + c];
+    }
+    double t = (s[0] + s[1]) + (s[2] + s[3]);
+    for (int off = kWave / 2; off >= kpad; off >>= 1) t += shfl_xor(t, off);
+    scratch[threadIdx.x] = t;
+    __syncthreads();
+    const int step = kpad > kWave ? kpad : kWave;
+    if (threadIdx.x < k) {
+        double v = scratch[threadIdx.x];
+        for (int q = step; q < kBlock; q += step) v += scratch[q + threadIdx.x];
+        out[threadIdx.x] = v;
+    }
+    __syncthreads();
 }
 
 }  // namespace tg

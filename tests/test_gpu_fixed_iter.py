@@ -90,6 +90,48 @@ def test_cg_fixed_iterations_3d_wide(cuda, steps):
     assert res_err(cg.Residuals(), ar_o, ar_o / rr_o) <= TOL
 
 
+@pytest.mark.parametrize("n,k", [(1, 1), (7, 5), (255, 1), (257, 2), (5003, 4), (3001, 7), (1999, 16), (777, 100),
+                                 (300001, 1), (262147, 3)])
+@pytest.mark.parametrize("prec", [False, True], ids=["identity", "jacobi"])
+def test_cg_two_kernel_form_ragged_rows(cuda, fused_knob, n, k, prec):
+    """The two-kernel iteration (every workgroup adds the partials itself) on rows of 1 to
+    about 25 nonzeros: chunks of eight pairs and their remainders, blocks of one and of
+    several passes over the rows, fewer rows than a workgroup has lanes.  tol = 0, 21 steps
+    (several blocks of iterations, the last of odd length), at the bar of this file.  The
+    iterates of two correct implementations differ by about steps * cond * 2^-53, so the
+    matrix is scaled to a condition number of at most 3 (2 I + a symmetric part of norm <=
+    1): 21 * 3 * 1.1e-16 = 7e-15, against 1e-12.  (Unscaled, the long rows' diagonals are
+    60 times the short ones', cond is about 500, the same estimate 1.2e-12 and the measured
+    difference 1.7e-12.)"""
+    rng = np.random.default_rng(n * 131 + k)
+    m = n * 2
+    i = rng.integers(0, n, m)
+    j = np.where(rng.random(m) < 0.1, i // 64 * 64, (i + rng.integers(1, 40, m)) % n)  # some rows much longer
+    v = rng.uniform(-1, 1, m) * (i != j)
+    off = sp.coo_matrix((v, (i, j)), shape=(n, n)).tocsr()
+    off = (off + off.T).tocsr()
+    w = sp.diags(1.0 / np.sqrt(np.maximum(np.asarray(abs(off).sum(1)).ravel(), 1e-3)))
+    A = (w @ off @ w + 2.0 * sp.identity(n)).tocsr()  # |w off w| <= 1: w off w is similar to a matrix of row sums <= 1
+    A.sort_indices()
+    rp, ci, val = A.indptr.astype(np.int64), A.indices.astype(np.int32), A.data
+    assert A.nnz <= 16 * n
+    d = 1.0 / A.diagonal() if prec else None
+    B = gen.uniform(77 + k, n * k).reshape(n, k)
+    fused_knob(2)
+    steps = 21
+    Xo = np.zeros((n, k))
+    _, it_o, rr_o, _ = oracle.cg_ex(n, rp, ci, val, B, Xo, k, steps, 0.0, prec_diag=d, threads=8)
+    cg = ConjugateGradient(n, steps, k)
+    Xd = torch.zeros(n, k, dtype=torch.float64, device=cuda)
+    cg(MatrixCSR(rp if k % 2 else rp.astype(np.int32), ci, val, n, n), None if d is None else dev(d, cuda), 1.0,
+       dev(B, cuda), 0.0, Xd, 0.0)
+    if n == 1:  # exact after one step, then 0 / 0 (as the reference's recurrences give)
+        return
+    assert cg.IterationCount() == it_o == steps
+    assert rel_err(Xd.cpu().numpy(), Xo) <= TOL
+    assert res_err(cg.RelativeResiduals(), rr_o) <= TOL
+
+
 @pytest.fixture
 def panel_knob():
     before = int(capi.lib().tg_tune_get(b"cg_panel"))

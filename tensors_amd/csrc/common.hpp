@@ -51,6 +51,38 @@ __device__ __forceinline__ void load_vec(const T* __restrict__ p, T (&out)[V]) {
     }
 }
 
+// The same at any element's address: global vector loads and stores need 4-byte alignment
+// only, so rows of an odd number of values are read in vectors too.
+template <typename T, int V>
+struct VecAt {
+    typedef T type __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+};
+
+template <typename T, int V>
+__device__ __forceinline__ void load_vec_at(const T* __restrict__ p, T* out) {
+    if constexpr (V == 1) {
+        out[0] = *p;
+    } else {
+        using VT = typename VecAt<T, V>::type;
+        const VT v = *reinterpret_cast<const VT*>(p);
+#pragma unroll
+        for (int i = 0; i < V; ++i) out[i] = v[i];
+    }
+}
+
+template <typename T, int V>
+__device__ __forceinline__ void store_vec_at(T* __restrict__ p, const T* in) {
+    if constexpr (V == 1) {
+        *p = in[0];
+    } else {
+        using VT = typename VecAt<T, V>::type;
+        VT v;
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[i] = in[i];
+        *reinterpret_cast<VT*>(p) = v;
+    }
+}
+
 template <typename T, int V>
 __device__ __forceinline__ void store_vec(T* __restrict__ p, const T (&in)[V]) {
     if constexpr (V == 1) {

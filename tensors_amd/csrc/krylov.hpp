@@ -33,6 +33,7 @@ struct CsrView {
     const void* val = nullptr;  // null: binary matrix
     tg_dtype val_type = TG_F64;
     int64_t band = -1;          // max |column - row| if known (csr_band), else -1
+    int32_t max_row = -1;       // nonzeros of the longest row if known (plans), else -1
     const LongRows* longr = nullptr;  // split-off long rows (plan path), or none
 };
 

@@ -49,29 +49,39 @@ __device__ __forceinline__ T fma_rn(T a, T b, T c) {
         return __builtin_fmaf(a, b, c);
 }
 
+// The first `skip` entries are left alone (another lane's columns).
 template <typename T, int V>
 __device__ __forceinline__ void epilogue(T* __restrict__ yp, const T (&z)[V], bool empty, T alpha,
-                                         int alpha_one, T beta, int beta_mode) {
+                                         int alpha_one, T beta, int beta_mode, int skip = 0) {
 #pragma clang fp contract(off)
     T out[V];
+    auto store = [&]() {
+        if (V == 1 || skip == 0) {
+            store_vec_at<T, V>(yp, out);
+        } else {
+#pragma unroll
+            for (int i = 1; i < V; ++i)
+                if (i >= skip) yp[i] = out[i];
+        }
+    };
     if (empty) {
         if (beta_mode == kBetaOne) return;
         if (beta_mode == kBetaZero) {
 #pragma unroll
             for (int i = 0; i < V; ++i) out[i] = T(0);
         } else {
-            load_vec<T, V>(yp, out);
+            load_vec_at<T, V>(yp, out);
 #pragma unroll
             for (int i = 0; i < V; ++i) out[i] = beta * out[i];
         }
-        store_vec<T, V>(yp, out);
+        store();
         return;
     }
 #pragma unroll
     for (int i = 0; i < V; ++i) out[i] = alpha_one ? z[i] : alpha * z[i];
     if (beta_mode != kBetaZero) {
         T yv[V];
-        load_vec<T, V>(yp, yv);
+        load_vec_at<T, V>(yp, yv);
         if (beta_mode == kBetaOne) {
 #pragma unroll
             for (int i = 0; i < V; ++i) out[i] = out[i] + yv[i];
@@ -80,7 +90,7 @@ __device__ __forceinline__ void epilogue(T* __restrict__ yp, const T (&z)[V], bo
             for (int i = 0; i < V; ++i) out[i] = fma_rn(beta, yv[i], out[i]);
         }
     }
-    store_vec<T, V>(yp, out);
+    store();
 }
 
 __device__ __forceinline__ void block_rows(int m, const int32_t* __restrict__ job_ptr, int rows_per_block,
@@ -132,32 +142,72 @@ __global__ __launch_bounds__(kBlock) void spmv_team_kernel(
     }
 }
 
-// nrhs == 1, streaming form: the workgroup walks its nonzeros in chunks of
+// K <= 4 consecutive entries of an X row, at most 16 bytes a load.
+template <typename T, int K>
+__device__ __forceinline__ void load_cols(const T* __restrict__ p, T* out) {
+    if constexpr (sizeof(T) == 4 || K <= 2) {
+        load_vec_at<T, K>(p, out);
+    } else {
+        load_vec_at<T, 2>(p, out);
+        load_vec_at<T, K - 2>(p + 2, out + 2);
+    }
+}
+
+// Sum of p[l K] for l = lb, lb + TEAM, ... < le, in four running sums: four reads in
+// flight, and a rounding error that grows with a quarter of the terms.
+template <typename T, int TEAM, int K>
+__device__ __forceinline__ T lds_sum(const T* p, int lb, int le) {
+    T s[4] = {T(0), T(0), T(0), T(0)};
+    int l = lb;
+    for (; l + 3 * TEAM < le; l += 4 * TEAM)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] += p[(l + j * TEAM) * K];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+        if (l + j * TEAM < le) s[j] += p[(l + j * TEAM) * K];
+    return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
+// nrhs = K <= 4, streaming form: the workgroup walks its nonzeros in chunks of
 // kBlock * ELEMS.  Every lane loads ELEMS (column, value) pairs of the chunk
 // with coalesced loads and gathers the x entries -- all independent, so a wave
 // keeps 2*ELEMS loads in flight instead of one dependent rp -> ci -> x chain
 // per row -- and leaves the products in LDS.  Teams of TEAM lanes then sum each
-// row's segment out of LDS (strided, butterfly); rows that span chunks
+// (row, column)'s segment out of LDS (strided, butterfly); rows that span chunks
 // accumulate in LDS.  Rows are taken RMAX at a time.
-template <typename T, typename RP, int ELEMS, int TEAM>
+// SPLIT: the re-laid layout of a plan -- rp holds the 8m + 1 row pointers of all column
+// slices, slice after slice; workgroup b works on slice b % 8 (the XCD it runs on), whose
+// rows' runs are one contiguous range of ci and a, and leaves the row sums in
+// part[slice][row][column].  (Finding each position's row by binary search, as the
+// cut-based slices have to, took 283 us of a 305 us product; the product takes 203 us so:
+// 1e6 rows, 32 nonzeros each, FP64, one column.)
+template <typename T, typename RP, int ELEMS, int TEAM, int K, bool SPLIT>
 __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(
     int m, const RP* __restrict__ rp, const int32_t* __restrict__ ci, const T* __restrict__ a, T alpha,
     const T* __restrict__ x, int64_t ldx, T beta, T* __restrict__ y, int64_t ldy, int alpha_one, int beta_mode,
-    const int32_t* __restrict__ job_ptr, int rows_per_block, const int* __restrict__ skip) {
+    const int32_t* __restrict__ job_ptr, int rows_per_block, const int* __restrict__ skip, T* __restrict__ part) {
     if (skip && *skip) return;
     constexpr int CAP = kBlock * ELEMS;
-    constexpr int RMAX = 1024;
+    constexpr int RMAX = 1024 / (K == 3 ? 4 : K);
     constexpr int TEAMS = kBlock / TEAM;
-    __shared__ T prod[CAP];
+    __shared__ T prod[CAP * K];
     __shared__ RP srp[RMAX + 1];
-    __shared__ T racc[RMAX];
+    __shared__ T racc[RMAX * K];
     int r0, r1;
-    block_rows(m, job_ptr, rows_per_block, r0, r1);
+    if constexpr (SPLIT) {
+        const int b = blockIdx.x, sl = b % kXcds;
+        r0 = min(m, (b / kXcds) * rows_per_block);
+        r1 = min(m, r0 + rows_per_block);
+        rp += (int64_t)sl * m;
+        part += (int64_t)sl * m * K;
+    } else {
+        block_rows(m, job_ptr, rows_per_block, r0, r1);
+    }
     const int lt = threadIdx.x % TEAM, team = threadIdx.x / TEAM;
     for (int rs = r0; rs < r1; rs += RMAX) {
         const int nr = min(RMAX, r1 - rs);
         for (int i = threadIdx.x; i <= nr; i += kBlock) srp[i] = rp[rs + i];
-        for (int i = threadIdx.x; i < nr; i += kBlock) racc[i] = T(0);
+        for (int i = threadIdx.x; i < nr * K; i += kBlock) racc[i] = T(0);
         __syncthreads();
         const RP L0 = srp[0], L1 = srp[nr];
         for (RP cs = L0; cs < L1; cs += CAP) {
@@ -176,28 +226,36 @@ __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(
             }
             // gathers unconditionally (c = 0 for the lanes past the chunk, a valid
             // entry) so that all ELEMS are in flight together; only the store is masked
-            T xv[ELEMS];
+            T xv[ELEMS][K];
 #pragma unroll
-            for (int j = 0; j < ELEMS; ++j) xv[j] = x[(int64_t)c[j] * ldx];
+            for (int j = 0; j < ELEMS; ++j) load_cols<T, K>(x + (int64_t)c[j] * ldx, xv[j]);
 #pragma unroll
             for (int j = 0; j < ELEMS; ++j) {
                 const int e = threadIdx.x + j * kBlock;
-                if (e < cnt) prod[e] = av[j] * xv[j];
+                if (e < cnt)
+#pragma unroll
+                    for (int q = 0; q < K; ++q) prod[e * K + q] = av[j] * xv[j][q];
             }
             __syncthreads();
-            for (int i = team; i < nr; i += TEAMS) {
+            for (int t = team; t < nr * K; t += TEAMS) {
+                const int i = t / K, q = t % K;
                 const RP lb = srp[i] > cs ? srp[i] : cs;
                 const RP le = srp[i + 1] < cs + cnt ? srp[i + 1] : cs + cnt;
-                T sum = T(0);
-                for (RP l = lb + lt; l < le; l += TEAM) sum += prod[l - cs];
+                T sum = lds_sum<T, TEAM, K>(prod + q, (int)(lb - cs) + lt, (int)(le - cs));
                 sum = group_sum<TEAM>(sum);
-                if (lt == 0 && le > lb) racc[i] += sum;
+                if (lt == 0 && le > lb) racc[t] += sum;
             }
             __syncthreads();
         }
-        for (int i = threadIdx.x; i < nr; i += kBlock) {
-            T zz[1] = {racc[i]};
-            epilogue<T, 1>(y + (int64_t)(rs + i) * ldy, zz, srp[i + 1] == srp[i], alpha, alpha_one, beta, beta_mode);
+        for (int t = threadIdx.x; t < nr * K; t += kBlock) {
+            const int i = t / K, q = t % K;
+            if constexpr (SPLIT) {
+                part[(int64_t)rs * K + t] = racc[t];
+            } else {
+                T zz[1] = {racc[t]};
+                epilogue<T, 1>(y + (int64_t)(rs + i) * ldy + q, zz, srp[i + 1] == srp[i], alpha, alpha_one, beta,
+                               beta_mode);
+            }
         }
         __syncthreads();
     }
@@ -294,14 +352,17 @@ __global__ __launch_bounds__(kBlock) void spmm_wave_kernel(
     }
 }
 
-// spmm_rows<G,V>: short rows (grid and FEM matrices, a few nonzeros per row) with
-// many right-hand sides.  Splitting one such row over a whole wave leaves most
-// lanes idle and makes every row a chain of dependent loads; here each of the
-// 64/G lane groups of a wave owns its own row: the group loads G (column, value)
-// pairs of the row at once, hands them out with cross-lane reads, and gathers the
-// X rows U at a time, so a wave keeps 64/G rows and 4 gathers per lane in flight.
-// A row's sum stays in its group (no butterfly); the summation order is the
-// nonzero order.
+// spmm_rows<G,V>: a row per lane group (short and middling rows) with many right-hand
+// sides.  Splitting such a row over a whole wave leaves lanes idle and makes every row a
+// chain of dependent loads with one row in flight per wave; here each of the 64/G lane
+// groups of a wave owns its own row: the group loads CH (column, value) pairs of the row
+// at once (PER per lane), hands them out with cross-lane reads, and gathers the X rows U
+// at a time, so a wave keeps 64/G rows and U gathers per lane in flight.  A row's sum
+// stays in its group (no butterfly): U nonzeros in a fixed tree, then the next U.
+// Several pairs per lane make narrow groups read a cache line of A in several loads, which
+// therefore are ordinary ones (a non-temporal line would be fetched again for each).
+// V columns per lane at any alignment; where V does not divide nrhs the last lane's vector
+// is moved back to end at the last column and stores only its own columns.
 template <typename T, typename RP, int G, int V>
 __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(
     int m, const RP* __restrict__ rp, const RP* __restrict__ rpe, const int32_t* __restrict__ ci, const T* __restrict__ a, T alpha,
@@ -311,7 +372,9 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(
     constexpr int S = kWave / G;  // rows in flight per wave
     constexpr int KT = G * V;     // columns per tile
     constexpr int WAVES = kBlock / kWave;
-    constexpr int U = 4;
+    constexpr int U = V * sizeof(T) <= 8 ? 8 : 4;
+    constexpr int PER = G >= 16 ? 1 : G == 8 ? 2 : 8 / G;
+    constexpr int CH = G * PER;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int s = lane / G, g = lane % G;
     int r0, r1;
@@ -325,37 +388,77 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(
 #pragma unroll
         for (int off = G; off < kWave; off <<= 1) wmax = max(wmax, __shfl_xor(wmax, off, kWave));
         for (int c0 = 0; c0 < nrhs; c0 += KT) {
-            const int col = c0 + g * V;
-            const bool colok = col < nrhs;
+            const int own = c0 + g * V;
+            const bool colok = own < nrhs;
+            const int col = colok ? min(own, nrhs - V) : 0;  // V <= nrhs
             T acc[V];
 #pragma unroll
             for (int i = 0; i < V; ++i) acc[i] = T(0);
-            for (int base = 0; base < wmax; base += G) {
-                const int e = base + g;
-                int32_t myc = 0;
-                T mya = T(0);
-                if (e < len) {
-                    myc = __builtin_nontemporal_load(ci + lb + e);
-                    mya = a ? __builtin_nontemporal_load(a + lb + e) : T(1);
+            for (int base = 0; base < wmax; base += CH) {
+                int32_t myc[PER];
+                T mya[PER];
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {  // clamped: some row of the wave has a nonzero, so 0 is valid
+                    const RP at = max(lb + min(base + g + q * G, len - 1), RP(0));
+                    myc[q] = ci[at];
+                    mya[q] = a ? a[at] : T(1);
                 }
-                const int cnt = min(G, len - base);  // this group's pairs in the chunk
-                const int wcnt = min(G, wmax - base);
-                for (int u0 = 0; u0 < wcnt; u0 += U) {
+                const int cnt = min(CH, len - base);  // this group's pairs in the chunk
+                const int wcnt = min(CH, wmax - base);
+                auto round = [&](int u0) {
+                    int cj[U];
+                    T av[U];
+                    bool live[U];
 #pragma unroll
                     for (int uu = 0; uu < U; ++uu) {
-                        const int j = u0 + uu;
-                        const int src = s * G + (j < G ? j : 0);
-                        const int32_t c = __shfl(myc, src, kWave);
-                        const T av = __shfl(mya, src, kWave);
-                        const bool live = (j < cnt) && colok;
-                        T xv[V];
-                        load_vec<T, V>(X + (int64_t)(live ? c : 0) * ldX + (live ? col : 0), xv);
-#pragma unroll
-                        for (int i = 0; i < V; ++i) acc[i] += live ? av * xv[i] : T(0);
+                        const int j = u0 + uu;  // pair j is in lane j % G's slot j / G
+                        int32_t c;
+                        if constexpr (G == 1) {
+                            c = myc[j % PER];
+                            av[uu] = mya[j % PER];
+                        } else {
+                            const int src = s * G + (PER > 1 ? j % G : (j < G ? j : 0));
+                            c = __shfl(myc[PER == 1 ? 0 : (j / G) % PER], src, kWave);
+                            av[uu] = __shfl(mya[PER == 1 ? 0 : (j / G) % PER], src, kWave);
+                        }
+                        live[uu] = (j < cnt) && colok;
+                        cj[uu] = live[uu] ? c : 0;
+                        av[uu] = live[uu] ? av[uu] : T(0);
                     }
+                    T xv[U][V];
+#pragma unroll
+                    for (int uu = 0; uu < U; ++uu)
+                        load_vec_at<T, V>(X + (int64_t)cj[uu] * ldX + col, xv[uu]);
+                    // the round's products are added in a tree: a row of one lane would otherwise
+                    // be one chain of roundings
+#pragma unroll
+                    for (int i = 0; i < V; ++i) {
+                        T t[U / 2];
+#pragma unroll
+                        for (int h = 0; h < U / 2; ++h) {
+                            const T x0 = live[2 * h] ? xv[2 * h][i] : T(0), x1 = live[2 * h + 1] ? xv[2 * h + 1][i] : T(0);
+                            t[h] = fma_rn(av[2 * h + 1], x1, av[2 * h] * x0);
+                        }
+#pragma unroll
+                        for (int w = U / 4; w > 0; w /= 2)
+#pragma unroll
+                            for (int h = 0; h < w; ++h) t[h] += t[h + w];
+                        acc[i] += t[0];
+                    }
+                };
+                if constexpr (PER > 1) {  // rounds at constant positions, so that a pair's slot is a constant
+                    static_assert(CH <= 4 * U, "rounds");
+                    round(0);
+                    if (CH > U && wcnt > U) round(U);
+                    if (CH > 2 * U && wcnt > 2 * U) round(2 * U);
+                    if (CH > 3 * U && wcnt > 3 * U) round(3 * U);
+                } else {
+                    for (int u0 = 0; u0 < wcnt; u0 += U) round(u0);
                 }
             }
-            if (rok && colok) epilogue<T, V>(Y + (int64_t)row * ldY + col, acc, le == lb, alpha, alpha_one, beta, beta_mode);
+            if (rok && colok)
+                epilogue<T, V>(Y + (int64_t)row * ldY + col, acc, le == lb, alpha, alpha_one, beta, beta_mode,
+                               own - col);
         }
     }
 }
@@ -463,6 +566,15 @@ static int rows_per_block_for(int32_t m, int64_t nnz, int32_t nrhs) {
     return (kBlock / kWave) * kRowsPerTeam;
 }
 
+// Rounds of `rows` rows each that a workgroup of the nrhs >= 2 kernels makes: as few as
+// give at most 2048 workgroups (eight per CU, no second wave of them), at most
+// kRowsPerTeam.  With a fixed eight a 20 000-row matrix filled 40 workgroups (FP64, 24 per
+// row, 8 columns, a row per lane group: 42 us; 9.3 us so).
+static int rounds_for(int32_t m, int rows) {
+    const int64_t wave = (int64_t)rows * 2048;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(kRowsPerTeam, ((int64_t)m + wave - 1) / wave));
+}
+
 constexpr int kStreamElems = 8;
 constexpr int kStreamCap = kBlock * kStreamElems;
 
@@ -497,10 +609,11 @@ static int launch_spmv(int32_t m, int64_t nnz, const RP* rp, const RP* rpe, cons
         const int grid = job_ptr ? blocks : (m + rpb - 1) / rpb;
         if (grid <= 0) return TG_OK;
         const int steam = std::min(team, 32);
-#define TG_SPMVS(TM)                                                                                          \
-    case TM:                                                                                                  \
-        hipLaunchKernelGGL((spmv_stream_kernel<T, RP, kStreamElems, TM>), dim3(grid), dim3(kBlock), 0, st, m, rp, \
-                           ci, a, alpha, X, ldX, beta, Y, ldY, alpha_one, beta_mode, job_ptr, rpb, skip);      \
+#define TG_SPMVS(TM)                                                                                               \
+    case TM:                                                                                                       \
+        hipLaunchKernelGGL((spmv_stream_kernel<T, RP, kStreamElems, TM, 1, false>), dim3(grid), dim3(kBlock), 0, \
+                           st, m, rp, ci, a, alpha, X, ldX, beta, Y, ldY, alpha_one, beta_mode, job_ptr, rpb, skip, \
+                           (T*)nullptr);                                                                           \
         break;
         switch (steam) {
             TG_SPMVS(1)
@@ -537,14 +650,52 @@ static int launch_spmv(int32_t m, int64_t nnz, const RP* rp, const RP* rpe, cons
     return TG_OK;
 }
 
+// Positions per lane of the streaming kernel for K columns: 16-32 KB of products.
+constexpr int stream_elems(int K) { return K == 1 ? kStreamElems : 4; }
+
+// Lanes that add a row's products and rows per workgroup, for rows cut into S slices.  One
+// lane adds up to 12 products out of LDS (a butterfly would cost more), one chunk of
+// positions holds the workgroup's rows.
+static void stream_shape(int32_t m, int64_t nnz, int S, int K, int& team, int& rpb) {
+    const double avg = m > 0 ? (double)nnz / m / S : 0.0;
+    team = avg <= 12.0 ? 1 : avg <= 64.0 ? 4 : 16;
+    const int rmax = 1024 / (K == 3 ? 4 : K);
+    rpb = std::max(1, std::min(rmax, (int)(kBlock * stream_elems(K) / (avg + 1.0))));
+}
+
+// The streaming kernel for K = 2, 3, 4 columns (plain), or K = 1..4 on the re-laid slices.
+template <typename T, typename RP, int K, bool SPLIT>
+static int launch_stream_k(int32_t m, int64_t nnz, const RP* rp, const int32_t* ci, const T* a, T alpha, const T* X,
+                           int64_t ldX, T beta, T* Y, int64_t ldY, int alpha_one, int beta_mode, const int* skip,
+                           T* part, hipStream_t st) {
+    constexpr int E = stream_elems(K);
+    int team, rpb;
+    stream_shape(m, nnz, SPLIT ? kXcds : 1, K, team, rpb);
+    const int grid = ((m + rpb - 1) / rpb) * (SPLIT ? kXcds : 1);
+    if (grid <= 0) return TG_OK;
+#define TG_STREAM(TM)                                                                                                \
+    hipLaunchKernelGGL((spmv_stream_kernel<T, RP, E, TM, K, SPLIT>), dim3(grid), dim3(kBlock), 0, st, m, rp, \
+                       ci, a, alpha, X, ldX, beta, Y, ldY, alpha_one, beta_mode, (const int32_t*)nullptr, rpb, skip, \
+                       part)
+    if (team == 1)
+        TG_STREAM(1);
+    else if (team == 4)
+        TG_STREAM(4);
+    else
+        TG_STREAM(16);
+#undef TG_STREAM
+    TG_LAUNCH_CHECK();
+    return TG_OK;
+}
+
 template <typename T, typename RP, int V>
-static int launch_spmm_v(int G, bool rows_mode, int32_t m, const RP* rp, const RP* rpe, const int32_t* ci, const T* a,
+static int launch_spmm_v(int G, bool rows, int32_t m, const RP* rp, const RP* rpe, const int32_t* ci, const T* a,
                          T alpha,
                          const T* X, int64_t ldX, T beta, T* Y, int64_t ldY, int32_t nrhs, int alpha_one,
                          int beta_mode, const int32_t* job_ptr, int32_t blocks, const int* skip, hipStream_t st) {
-    if (rows_mode && G < kWave) {
-        // 64/G rows per wave at a time; kRowsPerTeam rounds per wave per block
-        const int rpb = (kBlock / G) * kRowsPerTeam;
+    if (rows && G < kWave) {
+        // 64/G rows per wave at a time
+        const int rpb = (kBlock / G) * rounds_for(m, kBlock / G);
         const int grid = job_ptr ? blocks : (m + rpb - 1) / rpb;
         if (grid <= 0) return TG_OK;
 #define TG_SPMMR(GG)                                                                                          \
@@ -565,7 +716,7 @@ static int launch_spmm_v(int G, bool rows_mode, int32_t m, const RP* rp, const R
         TG_LAUNCH_CHECK();
         return TG_OK;
     }
-    const int rpb = (kBlock / kWave) * kRowsPerTeam;
+    const int rpb = (kBlock / kWave) * rounds_for(m, kBlock / kWave);
     const int grid = job_ptr ? blocks : (m + rpb - 1) / rpb;
     if (grid <= 0) return TG_OK;
 #define TG_SPMM(GG)                                                                                      \
@@ -589,7 +740,7 @@ static int launch_spmm_v(int G, bool rows_mode, int32_t m, const RP* rp, const R
 }
 
 template <typename T, typename RP>
-static int spmm_typed(int32_t m, int64_t nnz, const RP* rp, const int32_t* ci, const T* a, double alpha_d,
+static int spmm_typed(int32_t m, int32_t n, int64_t nnz, int32_t max_row, const RP* rp, const int32_t* ci, const T* a, double alpha_d,
                       const T* X, int64_t ldX, double beta_d, T* Y, int64_t ldY, int32_t nrhs,
                       const int32_t* job_ptr, int32_t blocks, const int* skip, hipStream_t st,
                       const RP* rpe = nullptr) {
@@ -600,34 +751,64 @@ static int spmm_typed(int32_t m, int64_t nnz, const RP* rp, const int32_t* ci, c
     if (nrhs == 1)
         return launch_spmv<T, RP>(m, nnz, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, alpha_one, beta_mode,
                                   job_ptr, blocks, skip, st);
-    // Vector width: 16-byte loads when X and Y rows allow it.
+    const double avg = m > 0 ? (double)nnz / m : 0.0;
+    // Up to three columns, and four of longer rows: the streaming kernel (products of
+    // consecutive nonzeros, added per row out of LDS).  Four columns of 5-7 nonzeros a row
+    // are better a row per lane group: 100^3 grid, streaming / rows: k = 2 28 / 26 us, k = 3
+    // 40 / 41, k = 4 55 / 38 FP64, 27 / 20 FP32; 1e6 x 2e4, 6 a row, k = 2 FP32 33 / 41.
+    if (nrhs <= 4 && g_spmm_rows == 0 && !g_spmm_group && !job_ptr && rpe == rp + 1 && (nrhs < 4 || avg > 16.0)) {
+#define TG_SK(KK)                                                                                                \
+    return launch_stream_k<T, RP, KK, false>(m, nnz, rp, ci, a, alpha, X, ldX, beta, Y, ldY, alpha_one, beta_mode, \
+                                             skip, (T*)nullptr, st)
+        if (nrhs == 2) TG_SK(2);
+        if (nrhs == 3) TG_SK(3);
+        TG_SK(4);
+#undef TG_SK
+    }
+    // A row per lane group for short rows (mean length up to 16), and for middling ones where
+    // the gathers are mostly served by the L2s (X up to 20 MB) and no row is much longer than
+    // the others (a plan knows): a wave then works on 64 / G rows at a time instead of being
+    // a chain of round trips per row.  Gathers that miss the L2s are bound by the rate of
+    // lines instead, and splitting the row keeps its order of requests.  Row per lane group /
+    // per wave: 3e5 x 2.1e5, 21 a row, k = 7 FP32 77 / 104 us; 6e4, 20 a row, FP64, k = 16 (8 MB)
+    // 21 / 30, k = 40 (19 MB) 61 / 64; 3e5, 24 a row, k = 11 (26 MB) 209 / 192; 1e6, 32 a row,
+    // k = 16 (128 MB) 735 / 653.
+    const bool middling = avg <= 64.0 && max_row >= 0 && max_row <= 8 * avg &&
+                          (int64_t)n * nrhs * (int64_t)sizeof(T) <= (20ll << 20);
+    const bool rows_mode = g_spmm_rows == 2 || (g_spmm_rows == 0 && (avg <= 16.0 || middling));
+    // Vector width: up to 16 bytes.  The row-per-wave kernel needs X and Y rows aligned for it.
     const auto aligned = [&](int bytes) {
         return ((uintptr_t)X % bytes == 0) && ((uintptr_t)Y % bytes == 0) &&
                ((ldX * (int64_t)sizeof(T)) % bytes == 0) && ((ldY * (int64_t)sizeof(T)) % bytes == 0);
     };
-    int V = 1;
-    if (sizeof(T) == 8) {
-        if (nrhs % 2 == 0 && aligned(16)) V = 2;
-    } else {
-        if (nrhs % 4 == 0 && aligned(16))
-            V = 4;
-        else if (nrhs % 2 == 0 && aligned(8))
-            V = 2;
+    auto lanes_for = [&](int v) { return g_spmm_group ? g_spmm_group : std::min(64, pow2ceil((nrhs + v - 1) / v)); };
+    // As wide as the columns allow, but groups of at least 8 lanes for longer rows: narrower
+    // ones read A in pieces (21 a row, k = 7 FP32: V = 4 / 1 94 / 77 us; 32 a row, k = 5 58 / 45).
+    int Vr = sizeof(T) == 4 && nrhs >= 4 ? 4 : nrhs >= 2 ? 2 : 1;
+    while (Vr > 1 && avg > 12.0 && lanes_for(Vr) < 8) Vr /= 2;
+    const bool rows = rows_mode && lanes_for(Vr) < kWave;
+    int V = rows ? Vr : 1;
+    if (!rows) {
+        if (sizeof(T) == 8) {
+            if (nrhs % 2 == 0 && aligned(16)) V = 2;
+        } else {
+            if (nrhs % 4 == 0 && aligned(16))
+                V = 4;
+            else if (nrhs % 2 == 0 && aligned(8))
+                V = 2;
+        }
     }
-    const int G = g_spmm_group ? g_spmm_group : std::min(64, pow2ceil((nrhs + V - 1) / V));
-    // short rows: one row per lane group (auto: mean row length up to 16)
-    const double avg = m > 0 ? (double)nnz / m : 0.0;
-    const bool rows_mode = g_spmm_rows == 2 || (g_spmm_rows == 0 && avg <= 16.0);
+    const int G = lanes_for(V);
     switch (V) {
         case 1:
-            return launch_spmm_v<T, RP, 1>(G, rows_mode, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
+            return launch_spmm_v<T, RP, 1>(G, rows, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
                                            beta_mode, job_ptr, blocks, skip, st);
         case 2:
-            return launch_spmm_v<T, RP, 2>(G, rows_mode, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
+            return launch_spmm_v<T, RP, 2>(G, rows, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
                                            beta_mode, job_ptr, blocks, skip, st);
         default:
             if constexpr (sizeof(T) == 4)
-                return launch_spmm_v<T, RP, 4>(G, rows_mode, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
+                return launch_spmm_v<T, RP, 4>(G, rows, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
                                                beta_mode, job_ptr, blocks, skip, st);
             return fail(TG_ERR_INVALID, "internal: bad vector width");
     }
@@ -668,12 +849,15 @@ constexpr int kCuts = kXcds - 1;
 template <typename RP>
 __global__ __launch_bounds__(kBlock) void slice_plan_kernel(int m, int n, const RP* __restrict__ rp,
                                                             const int32_t* __restrict__ ci,
-                                                            int32_t* __restrict__ cuts, int* __restrict__ unsorted) {
+                                                            int32_t* __restrict__ cuts, int* __restrict__ unsorted,
+                                                            int* __restrict__ longest) {
+    int most = 0;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < m; i += gridDim.x * kBlock) {
         const int64_t lb = rp[i], le = rp[i + 1];
         bool bad = false;
         for (int64_t l = lb + 1; l < le; ++l) bad |= ci[l] < ci[l - 1];
         if (bad) *unsorted = 1;
+        most = max(most, (int)min(le - lb, (int64_t)0x7fffffff));
         for (int s = 1; s <= kCuts; ++s) {
             const int32_t bound = (int32_t)((int64_t)n * s / kXcds);
             int64_t lo = lb, hi = le;  // first l with ci[l] >= bound
@@ -687,6 +871,9 @@ __global__ __launch_bounds__(kBlock) void slice_plan_kernel(int m, int n, const 
             cuts[(int64_t)(s - 1) * m + i] = (int32_t)(lo - lb);  // offset within the row
         }
     }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off, kWave));
+    if (threadIdx.x % kWave == 0) atomicMax(longest, most);
 }
 
 // Run lengths of the re-laid layout: len[s * m + i] = nonzeros of row i in column
@@ -766,14 +953,9 @@ __device__ __forceinline__ void block_exclusive_scan(int* v, int n) {
 // so loads of a run coalesce), finds its row by binary search in LDS, gathers the
 // X row and leaves the K products in LDS; teams of TEAM lanes then add each row's
 // products (rows spanning chunks accumulate in LDS).
-// SPLIT: the re-laid layout of the plan -- every slice's runs stored as a CSR of
-// their own, slice after slice (srp: the 8m + 1 row pointers of all slices, ci and a
-// the re-laid column indices and values), so a workgroup's runs are one contiguous
-// range and no XCD touches another slice's cache lines of A.  S is 8 then.
-template <typename T, typename RP, int ELEMS, int TEAM, int K, bool SPLIT>
+template <typename T, typename RP, int ELEMS, int TEAM, int K>
 __global__ __launch_bounds__(kBlock) void spmm_slice_stream_kernel(int m, int S, const RP* __restrict__ rp,
                                                                    const int32_t* __restrict__ cuts,
-                                                                   const int32_t* __restrict__ srp,
                                                                    const int32_t* __restrict__ ci,
                                                                    const T* __restrict__ a, const T* __restrict__ X,
                                                                    int64_t ldX, T* __restrict__ part,
@@ -794,15 +976,9 @@ __global__ __launch_bounds__(kBlock) void spmm_slice_stream_kernel(int m, int S,
         const int nr = min(RMAX, r1 - rs);
         for (int i = threadIdx.x; i < nr; i += kBlock) {
             const int row = rs + i;
-            RP lb, le;
-            if constexpr (SPLIT) {
-                lb = srp[(int64_t)s * m + row];
-                le = srp[(int64_t)s * m + row + 1];
-            } else {
-                const RP base = rp[row];
-                lb = s == 0 ? base : base + cuts[(int64_t)(s * step - 1) * m + row];
-                le = s == S - 1 ? rp[row + 1] : base + cuts[(int64_t)((s + 1) * step - 1) * m + row];
-            }
+            const RP base = rp[row];
+            const RP lb = s == 0 ? base : base + cuts[(int64_t)(s * step - 1) * m + row];
+            const RP le = s == S - 1 ? rp[row + 1] : base + cuts[(int64_t)((s + 1) * step - 1) * m + row];
             slo[i] = lb;
             soff[i] = (int)(le - lb);
         }
@@ -836,9 +1012,7 @@ __global__ __launch_bounds__(kBlock) void spmm_slice_stream_kernel(int m, int S,
             }
             T xv[ELEMS][K];  // gathered unconditionally (c = 0 past the chunk) so they overlap
 #pragma unroll
-            for (int j = 0; j < ELEMS; ++j)
-#pragma unroll
-                for (int q = 0; q < K; ++q) xv[j][q] = X[(int64_t)c[j] * ldX + q];
+            for (int j = 0; j < ELEMS; ++j) load_cols<T, K>(X + (int64_t)c[j] * ldX, xv[j]);
 #pragma unroll
             for (int j = 0; j < ELEMS; ++j) {
                 const int e = threadIdx.x + j * kBlock;
@@ -850,16 +1024,10 @@ __global__ __launch_bounds__(kBlock) void spmm_slice_stream_kernel(int m, int S,
             for (int i = team; i < nr; i += TEAMS) {
                 const int lb = max(soff[i], cs), le = min(soff[i + 1], cs + cnt);
                 if (le <= lb) continue;  // team-uniform
-                T sum[K];
-#pragma unroll
-                for (int q = 0; q < K; ++q) sum[q] = T(0);
-                for (int l = lb + lt; l < le; l += TEAM)
-#pragma unroll
-                    for (int q = 0; q < K; ++q) sum[q] += prod[(l - cs) * K + q];
 #pragma unroll
                 for (int q = 0; q < K; ++q) {
-                    sum[q] = group_sum<TEAM>(sum[q]);
-                    if (lt == 0) racc[i * K + q] += sum[q];
+                    const T sum = group_sum<TEAM>(lds_sum<T, TEAM, K>(prod + q, lb - cs + lt, le - cs));
+                    if (lt == 0) racc[i * K + q] += sum;
                 }
             }
             __syncthreads();
@@ -904,6 +1072,8 @@ static bool split_pays(int64_t xbytes) {
     return xbytes > 2 * kMB && xbytes <= 64 * kMB;
 }
 
+constexpr int64_t kBandWindowBytes = 4ll << 20;  // an XCD's L2
+
 static int slice_count(int64_t xbytes) {
     constexpr int64_t kMB = 1ll << 20;
     constexpr int64_t kSliceBytes = 4 * kMB;
@@ -914,24 +1084,20 @@ static int slice_count(int64_t xbytes) {
     return S;
 }
 
-template <typename T, typename RP, int K, bool SPLIT>
+template <typename T, typename RP, int K>
 static void launch_slice_stream(int S, int team, int grid, int m, const RP* rp, const int32_t* cuts,
-                                const int32_t* srp, const int32_t* ci, const T* a, const T* X, int64_t ldX, T* part,
+                                const int32_t* ci, const T* a, const T* X, int64_t ldX, T* part,
                                 int rpb, hipStream_t st) {
-    // ELEMS keeps the product stage at 2048 entries (16 KB in FP64)
-    constexpr int E = K == 1 ? 8 : K == 2 ? 4 : 2;
+    constexpr int E = stream_elems(K);
 #define TG_SLS(TM)                                                                                                \
-    case TM:                                                                                                      \
-        hipLaunchKernelGGL((spmm_slice_stream_kernel<T, RP, E, TM, K, SPLIT>), dim3(grid), dim3(kBlock), 0, st, m, \
-                           S, rp, cuts, srp, ci, a, X, ldX, part, rpb);                                           \
-        break;
-    switch (team) {
-        TG_SLS(2)
-        TG_SLS(4)
-        TG_SLS(8)
-        default:
-            TG_SLS(16)
-    }
+    hipLaunchKernelGGL((spmm_slice_stream_kernel<T, RP, E, TM, K>), dim3(grid), dim3(kBlock), 0, st, m, S, rp, cuts, \
+                       ci, a, X, ldX, part, rpb)
+    if (team == 1)
+        TG_SLS(1);
+    else if (team == 4)
+        TG_SLS(4);
+    else
+        TG_SLS(16);
 #undef TG_SLS
 }
 
@@ -939,19 +1105,18 @@ template <typename T, typename RP>
 static int spmm_sliced_typed(int S, int32_t m, int64_t nnz, const RP* rp, const int32_t* cuts, const int32_t* srp,
                              const int32_t* ci, const T* a, double alpha_d, const T* X, int64_t ldX, double beta_d,
                              T* Y, int64_t ldY, int32_t K, T* part, hipStream_t st) {
-    const double avg = m > 0 ? (double)nnz / m / S : 0.0;  // mean run length per row and slice
-    const int team = std::min(16, std::max(2, pow2ceil((int)std::ceil(avg))));
-    const int cap = kBlock * (K == 1 ? 8 : K == 2 ? 4 : 2);
-    const int rmax = 1024 / (K == 3 ? 4 : K);
-    const int rpb = std::max(1, std::min(rmax, (int)(cap / (avg + 1.0))));
+    int team, rpb;
+    stream_shape(m, nnz, S, K, team, rpb);
     const int row_blocks = (m + rpb - 1) / rpb;
     const int per = kXcds / S;
     const int grid = kXcds * ((row_blocks + per - 1) / per);
-#define TG_SLK(KK)                                                                                              \
-    if (srp)                                                                                                    \
-        launch_slice_stream<T, RP, KK, true>(S, team, grid, m, rp, cuts, srp, ci, a, X, ldX, part, rpb, st);    \
-    else                                                                                                        \
-        launch_slice_stream<T, RP, KK, false>(S, team, grid, m, rp, cuts, srp, ci, a, X, ldX, part, rpb, st);
+    int rc = TG_OK;
+#define TG_SLK(KK)                                                                                                \
+    if (!srp)                                                                                                     \
+        launch_slice_stream<T, RP, KK>(S, team, grid, m, rp, cuts, ci, a, X, ldX, part, rpb, st);                 \
+    else                                                                                                          \
+        rc = launch_stream_k<T, int32_t, KK, true>(m, nnz, srp, ci, a, T(1), X, ldX, T(0), (T*)nullptr, 0, 0, 0,  \
+                                                   (const int*)nullptr, part, st);
     switch (K) {
         case 1: TG_SLK(1) break;
         case 2: TG_SLK(2) break;
@@ -959,6 +1124,7 @@ static int spmm_sliced_typed(int S, int32_t m, int64_t nnz, const RP* rp, const 
         default: TG_SLK(4) break;
     }
 #undef TG_SLK
+    if (rc) return rc;
     const int alpha_one = (alpha_d == 1.0);
     const int beta_mode = (beta_d == 0.0) ? kBetaZero : (beta_d == 1.0) ? kBetaOne : kBetaGeneric;
     const int rgrid = (int)std::min<int64_t>((m + kBlock - 1) / kBlock, 65536);
@@ -1283,22 +1449,22 @@ int spmm_dispatch(const CsrView& A, double alpha, const void* X, int64_t ldX, do
             const double* Xc = (const double*)X + c0;
             double* Yc = (double*)Y + c0;
             if (A.rp_type == TG_I32)
-                rc = spmm_typed<double, int32_t>(m, A.nnz, (const int32_t*)A.rp, A.ci, (const double*)A.val, alpha, Xc,
+                rc = spmm_typed<double, int32_t>(m, n, A.nnz, A.max_row, (const int32_t*)A.rp, A.ci, (const double*)A.val, alpha, Xc,
                                                  ldX, beta, Yc, ldY, kc, job_ptr, blocks, skip, st,
                                                  (const int32_t*)rpe);
             else
-                rc = spmm_typed<double, int64_t>(m, A.nnz, (const int64_t*)A.rp, A.ci, (const double*)A.val, alpha, Xc,
+                rc = spmm_typed<double, int64_t>(m, n, A.nnz, A.max_row, (const int64_t*)A.rp, A.ci, (const double*)A.val, alpha, Xc,
                                                  ldX, beta, Yc, ldY, kc, job_ptr, blocks, skip, st,
                                                  (const int64_t*)rpe);
         } else {
             const float* Xc = (const float*)X + c0;
             float* Yc = (float*)Y + c0;
             if (A.rp_type == TG_I32)
-                rc = spmm_typed<float, int32_t>(m, A.nnz, (const int32_t*)A.rp, A.ci, (const float*)A.val, alpha, Xc,
+                rc = spmm_typed<float, int32_t>(m, n, A.nnz, A.max_row, (const int32_t*)A.rp, A.ci, (const float*)A.val, alpha, Xc,
                                                 ldX, beta, Yc, ldY, kc, job_ptr, blocks, skip, st,
                                                 (const int32_t*)rpe);
             else
-                rc = spmm_typed<float, int64_t>(m, A.nnz, (const int64_t*)A.rp, A.ci, (const float*)A.val, alpha, Xc,
+                rc = spmm_typed<float, int64_t>(m, n, A.nnz, A.max_row, (const int64_t*)A.rp, A.ci, (const float*)A.val, alpha, Xc,
                                                 ldX, beta, Yc, ldY, kc, job_ptr, blocks, skip, st,
                                                 (const int64_t*)rpe);
         }
@@ -1329,6 +1495,7 @@ struct tg_csr_plan_s {
     int32_t* cuts = nullptr;  // kCuts x m row offsets of the 8-way column cut
     int sorted = 0;
     int64_t band = -1;        // max |column - row|
+    int32_t max_row = -1;     // nonzeros of the longest row
     // Re-laid layout (tg_csr_plan_set_values): the 8 slices' runs as CSRs of their own,
     // slice after slice -- row pointers of all slices (8m + 1), column indices, and the
     // values of one registered pointer per value type (0 FP64, 1 FP32).
@@ -1457,28 +1624,29 @@ extern "C" int tg_csr_plan_create(int32_t m, int32_t n, int64_t nnz, const void*
     int* flag = nullptr;
     if (m > 0 && n > 0) {
         if (hipMallocAsync((void**)&P->cuts, (size_t)kCuts * m * sizeof(int32_t), st) != hipSuccess ||
-            hipMallocAsync((void**)&flag, sizeof(int), st) != hipSuccess) {
+            hipMallocAsync((void**)&flag, 2 * sizeof(int), st) != hipSuccess) {
             delete P;
             return fail(TG_ERR_HIP, "tg_csr_plan_create: allocation failed");
         }
-        int zero = 0;
-        (void)hipMemcpyAsync(flag, &zero, sizeof(int), hipMemcpyHostToDevice, st);
+        const int zero[2] = {0, 0};  // unsorted, longest row
+        (void)hipMemcpyAsync(flag, zero, sizeof(zero), hipMemcpyHostToDevice, st);
         const int grid = (int)std::min<int64_t>((m + kBlock - 1) / kBlock, 65536);
         if (rp_type == TG_I32)
             hipLaunchKernelGGL((slice_plan_kernel<int32_t>), dim3(grid), dim3(kBlock), 0, st, m, n, (const int32_t*)rp,
-                               ci, P->cuts, flag);
+                               ci, P->cuts, flag, flag + 1);
         else
             hipLaunchKernelGGL((slice_plan_kernel<int64_t>), dim3(grid), dim3(kBlock), 0, st, m, n, (const int64_t*)rp,
-                               ci, P->cuts, flag);
-        int unsorted = 1;
-        (void)hipMemcpyAsync(&unsorted, flag, sizeof(int), hipMemcpyDeviceToHost, st);
+                               ci, P->cuts, flag, flag + 1);
+        int found[2] = {1, 0};
+        (void)hipMemcpyAsync(found, flag, sizeof(found), hipMemcpyDeviceToHost, st);
         (void)hipFreeAsync(flag, st);
         if (hipStreamSynchronize(st) != hipSuccess || hipGetLastError() != hipSuccess) {
             (void)hipFree(P->cuts);
             delete P;
             return fail(TG_ERR_HIP, "tg_csr_plan_create: plan kernel failed");
         }
-        P->sorted = unsorted ? 0 : 1;
+        P->sorted = found[0] ? 0 : 1;
+        P->max_row = found[1];
         CsrView V;
         V.m = m;
         V.n = n;
@@ -1514,6 +1682,15 @@ extern "C" int tg_csr_plan_destroy(tg_csr_plan_t plan) {
     return TG_OK;
 }
 
+// A banded matrix gathers from a window of X around the current rows, which the L2s keep
+// anyway: column slices would only add their partial blocks.  The line is an XCD's L2: 1e6
+// rows, 16 random columns a row within the band, FP64, sliced / plain: window 0.15 MB (k = 1)
+// 125 / 90 us, 3 MB (k = 1) 120 / 108, (k = 2) 149 / 95, 6 MB (k = 1) 120 / 127, 12 MB (k = 2)
+// 138 / 180; a 100^3 grid 63 / 26 us (k = 1), 182 / 36 (k = 4).
+static bool plan_band_narrow(tg_csr_plan_t plan, int32_t nrhs, int64_t vs) {
+    return plan->band >= 0 && (2 * plan->band + 1) * (int64_t)nrhs * vs <= kBandWindowBytes;
+}
+
 extern "C" int tg_csr_plan_set_values(tg_csr_plan_t plan, const void* a, tg_dtype val_type, void* stream) {
     if (!plan || (val_type != TG_F64 && val_type != TG_F32))
         return fail(TG_ERR_INVALID, "tg_csr_plan_set_values: bad argument");
@@ -1521,6 +1698,8 @@ extern "C" int tg_csr_plan_set_values(tg_csr_plan_t plan, const void* a, tg_dtyp
     std::lock_guard<std::mutex> lk(plan->mu);
     plan->sval_src[vi] = nullptr;
     if (!a || !plan->sorted || plan->m == 0 || plan->n == 0 || plan->nnz == 0) return TG_OK;
+    // a narrow band never takes the layout for up to four columns (plan_slices): no copy
+    if (g_spmm_slices == 0 && plan_band_narrow(plan, 4, val_type == TG_F64 ? 8 : 4)) return TG_OK;
     if (plan->nnz >= (1ll << 31)) return TG_OK;  // int32 offsets of the layout
     hipStream_t st = as_stream(stream);
     const int32_t m = plan->m;
@@ -1587,6 +1766,7 @@ static int plan_slices(tg_csr_plan_t plan, tg_dtype val_type, int32_t nrhs, cons
     if (g_spmm_slices == 1) return 0;
     const int64_t vs = val_type == TG_F64 ? 8 : 4;
     const int64_t xbytes = (int64_t)plan->n * nrhs * vs;
+    if (g_spmm_slices == 0 && plan_band_narrow(plan, nrhs, vs)) return 0;
     const int vi = val_type == TG_F64 ? 0 : 1;
     if (g_spmm_split && a && plan->srp && plan->sval_src[vi] == a && (g_spmm_slices == 0 || g_spmm_slices == kXcds) &&
         (g_spmm_slices == kXcds || split_pays(xbytes))) {
@@ -1627,6 +1807,7 @@ extern "C" int tg_csr_spmm_plan(tg_csr_plan_t plan, const void* a, tg_dtype val_
     A.val = a;
     A.val_type = val_type;
     A.band = plan->band;
+    A.max_row = plan->max_row;
     hipStream_t st = as_stream(stream);
     if (plan->nlong > 0 && (val_type == TG_F64 || val_type == TG_F32) && alpha != 0.0 && X && Y && X != Y &&
         ldX >= nrhs && ldY >= nrhs && nrhs > 0) {

@@ -263,3 +263,80 @@ def test_spmv_kernel_variants(cuda, variant, dtype):
             assert st == 0 and rel_err(Y, Yo) <= tol
     finally:
         L.tg_tune_set(b"spmv_kernel", old)
+
+
+def skewed_csr(m, n, mean, seed, longest):
+    """Rows of 0 to about 2 mean nonzeros (every ninth empty) and one of `longest`."""
+    rng = np.random.default_rng(seed)
+    lens = np.minimum(rng.integers(0, 2 * mean + 1, m), n)
+    lens[::9] = 0
+    lens[m // 2] = min(longest, n)
+    rp = np.zeros(m + 1, np.int64)
+    np.cumsum(lens, out=rp[1:])
+    ci = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens]).astype(np.int32)
+    return rp, ci, rng.integers(-4, 5, int(rp[-1])).astype(np.float64)
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 11, 33, 37])
+@pytest.mark.parametrize("mean,longest", [(3, 40), (20, 3000)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("plan", [False, True], ids=["call", "plan"])
+def test_spmm_kernel_choices_are_exact(cuda, k, mean, longest, dtype, plan):
+    """The streaming kernel (up to 4 columns; a row spans its chunks) and the row per lane
+    group (a last vector moved back where its width does not divide k, groups of every
+    width), with leading dimensions that leave no row aligned, pointers offset by one
+    element, int32 / int64 row pointers, binary matrices, empty rows and every beta rule.
+    Small integers: every sum is exact, so the bits are the oracle's; the columns beyond k
+    and the element before Y stay as they were."""
+    m, n = 700, 3100
+    rp, ci, val = skewed_csr(m, n, mean, 5 * k + mean, longest)
+    if plan and mean == 20:  # no long row: the plan's middling rule
+        rp, ci, val = skewed_csr(m, n, mean, 5 * k + mean, 2 * mean)
+    rng = np.random.default_rng(k)
+    ldx, ldy = k + 3, k + 1
+    X = rng.integers(-3, 4, (n, ldx)).astype(dtype)
+    Y0 = rng.integers(-3, 4, (m, ldy)).astype(dtype)
+    dt = torch.float64 if dtype == np.float64 else torch.float32
+
+    def shifted(a):  # one element past the allocation's alignment
+        flat = torch.zeros(a.size + 1, dtype=dt, device=cuda)
+        flat[0] = 99.0
+        flat[1:] = to_dev(a.reshape(-1), cuda, dt)
+        return flat, flat[1:].view(*a.shape)
+
+    rpd = to_dev(rp if k % 2 else rp.astype(np.int32), cuda)
+    cid, vd = to_dev(ci, cuda), to_dev(val, cuda, dt)
+    for a, alpha, beta in ((vd, 1.0, 0.0), (vd, -2.0, 1.0), (None, 2.0, 2.0), (vd, 1.0, -1.0)):
+        _, Xd = shifted(X)
+        whole, Yd = shifted(Y0)
+        if plan:
+            from tensors_amd.sparse import SlicePlan
+            P = SlicePlan(m, n, len(ci), rpd, cid)
+            assert P.spmm(a, alpha, Xd, ldx, beta, Yd, ldy, k) == 0
+        else:
+            assert spmm_raw(m, n, len(ci), rpd, cid, a, alpha, Xd, ldx, beta, Yd, ldy, k) == 0
+        Yo = Y0.astype(np.float64).copy()
+        oracle.spmm(rp, ci, None if a is None else val, m, n, alpha, X.astype(np.float64), ldx, beta, Yo, ldy, k)
+        assert np.array_equal(Yd.cpu().numpy().astype(np.float64), Yo), (alpha, beta)
+        assert whole[0].item() == 99.0
+
+
+def test_narrow_bands_take_no_slices(cuda):
+    """A banded matrix whose window of X fits an L2 is not sliced and keeps no re-laid copy;
+    the same sizes with scattered columns do and are."""
+    n = 600_000
+    i = np.arange(n)
+    rp = np.arange(0, 3 * n + 1, 3, dtype=np.int64)
+    band = np.stack([(i - 40) % n, i, (i + 40) % n], 1)
+    band[:40, 0], band[-40:, 2] = 80, n - 120  # no wrap-around
+    band = np.sort(band, 1)
+    far = np.sort(np.stack([i, (i * 7919 + 11) % n, (i * 104729 + 5) % n], 1), 1)
+    X = torch.ones(n, 2, dtype=torch.float64, device=cuda)
+    for cols, sliced in ((band, False), (far, True)):
+        A = MatrixCSR(rp, cols.reshape(-1).astype(np.int32), np.arange(3 * n) % 5 - 2.0, n, n)
+        Y = torch.zeros_like(X)
+        assert A.Dot(1.0, X, 0.0, Y) == 0
+        v = A.device_arrays(torch.float64)[2]
+        assert A.Plan().uses_split(v, 2) == sliced and (A.Plan().slices(torch.float64, 2) > 0) == sliced
+        want = (np.arange(3 * n) % 5 - 2.0).reshape(n, 3).sum(1)
+        assert np.array_equal(Y.cpu().numpy(), np.stack([want, want], 1))

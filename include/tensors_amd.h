@@ -218,12 +218,11 @@ int tg_csr_spmm_plan(tg_csr_plan_t plan, const void* a, tg_dtype val_type, doubl
  *                  for restart lengths up to 32 and (2m + 2) * nrhs <= 2048: two
  *                  passes over the basis and five launches per step), 0 = CGS2
  *                  (three passes, eight launches).  Results agree to rounding.
- *   "gmres_split_dots": delayed steps with one right-hand side and more than 16
- *                  basis vectors (FP32: the cycles of tg_gmres_solve_mixed; FP64:
- *                  systems below 2^19 rows): 1 = the dots pass with its u-side and
- *                  v-side dot products on alternate lanes (default: half the
- *                  accumulators per lane), and in FP32 the update pass with its two
- *                  output vectors on alternate lanes; 0 = both on every lane.
+ *   "gmres_split_dots": delayed steps with one right-hand side, 1 = the basis
+ *                  vectors dealt over the waves of a workgroup, two or three
+ *                  kernels a step with the product among them for CSR operators of
+ *                  short rows (default); 0 = every vector on every lane, a kernel
+ *                  each for the product, dots, totals, scalars and update.
  *                  Results agree to rounding.
  *   "bsr_vector":  tg_bsr_spmm with row-major X / Y chunks, 1 = a lane per
  *                  (block row, 1-4 right-hand sides) with vector loads (default),

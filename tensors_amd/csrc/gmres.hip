@@ -42,14 +42,15 @@ constexpr int kGmresMaxM = 63;     // restart length limit (m + 1 basis vectors 
 constexpr int kGB = 512;           // workgroups of the vector kernels (at most; fewer for small n)
 static int g_gmres_graph = 1;      // 1: cycles after the first run as one captured hipGraph
 static int g_gmres_delayed = 1;    // 1: CGS2 with the second pass delayed to the next step (two basis passes per step)
-static int g_gmres_split_dots = 1;  // 1: one-column dots pass of the 32-vector bucket with its two sides on alternate lanes
+static int g_gmres_split_dots = 1;  // 1: one column: the basis dealt over the waves of a workgroup, two or three kernels a step
 
 struct GmresHdr {
     int iter;
     int done;
     int succ;
     int m;
-    int pad[12];
+    int pend;  // one-column steps: the stop found by the step before, which the next one turns into `done`
+    int pad[11];
 };
 
 // Small FP64 arrays (offsets in doubles from the start of the small region).
@@ -355,89 +356,6 @@ __global__ __launch_bounds__(kBlock) void gm_ddots_kernel(int n, int k, int kpad
     dd_partial<NQMAX>(acc, j, k, kpad, partial);
 }
 
-// One column, 32-vector bucket: the dots pass with its two sides on alternate lanes.  Even lanes accumulate a_i = Q_i . u and alpha = u . u, odd lanes b_i = Q_i . v
-// and beta = u . v, over the same rows (the pair's loads of a basis row are one
-// address), so a lane holds NQMAX + 1 FP64 accumulators instead of 2 NQMAX + 2 and the
-// reduce-scatter (over the lanes of one side: two "columns") half the values.  FP32: RU
-// rows per iteration, 1 (111 VGPRs, 4 waves per SIMD) measured faster on systems of 1e4
-// and 9e4 rows, 2 (179 VGPRs, 2 waves) on 1e6 rows.  FP64: 1 (144 VGPRs, 3 waves), below
-// 2^19 rows.
-template <int NQMAX>
-__device__ __forceinline__ void dd_partial_split(double (&v)[NQMAX + 1], int j, double* __restrict__ partial) {
-    extern __shared__ double gm_sh[];
-    const int nv = 2 * j + 2;
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    constexpr int R = NQMAX + 1;
-    {
-        const ScatterOut o = wave_scatter_sum<R>(v, 2);
-        const int side = lane % 2;
-        if ((lane % o.low) < 2)
-#pragma unroll
-            for (int i = 0; i < ScatterSizes<R>::A; ++i) {
-                const int r = o.base + i;
-                const int t = i >= o.count ? -1 : r < NQMAX ? (r < j ? side * j + r : -1) : 2 * j + side;
-                if (t >= 0) gm_sh[wave * nv + t] = v[i];
-            }
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < nv; t += kBlock) {
-        double s = 0.0;
-#pragma unroll
-        for (int w = 0; w < kBlock / kWave; ++w) s += gm_sh[w * nv + t];
-        partial[(int64_t)blockIdx.x * nv + t] = s;
-    }
-}
-
-template <typename T, int NQMAX, int RU>
-__global__ __launch_bounds__(kBlock) void gm_ddots_split_kernel(int n, int j, int finish,
-                                                                const T* __restrict__ Q, int64_t qstride,
-                                                                const T* __restrict__ z,
-                                                                const T* __restrict__ d, T* __restrict__ vslot,
-                                                                double* __restrict__ partial,
-                                                                const GmresHdr* __restrict__ hd) {
-    if (hd->done) return;
-    int i0, i1;
-    grow_range(n, i0, i1);
-    const int side = threadIdx.x & 1, ro = threadIdx.x >> 1, rows = kBlock / 2;
-    double acc[NQMAX + 1];
-#pragma unroll
-    for (int r = 0; r < NQMAX + 1; ++r) acc[r] = 0.0;
-    const T* U = Q + (int64_t)j * qstride;
-    for (int r = i0 + ro; r < i1; r += rows * RU) {
-        T qi[RU][NQMAX], uv[RU], vv[RU];
-        int rr[RU];
-#pragma unroll
-        for (int u = 0; u < RU; ++u) {
-            rr[u] = r + u * rows < i1 ? r + u * rows : r;
-#pragma unroll
-            for (int i = 0; i < NQMAX; ++i) qi[u][i] = Q[(int64_t)max(0, min(i, j - 1)) * qstride + rr[u]];
-            uv[u] = U[rr[u]];
-        }
-#pragma unroll
-        for (int u = 0; u < RU; ++u) {
-            const bool ok = r + u * rows < i1;
-            if (finish) {
-                vv[u] = uv[u];
-            } else if (d) {
-                vv[u] = d[rr[u]] * z[rr[u]];
-                if (ok && side) vslot[rr[u]] = vv[u];
-            } else {
-                vv[u] = vslot[rr[u]];
-            }
-            if (!ok) uv[u] = vv[u] = T(0);
-        }
-#pragma unroll
-        for (int u = 0; u < RU; ++u) {
-            const T w = side ? vv[u] : uv[u];
-#pragma unroll
-            for (int i = 0; i < NQMAX; ++i)
-                if (i < j) acc[i] += (double)qi[u][i] * (double)w;
-            acc[NQMAX] += (double)uv[u] * (double)w;
-        }
-    }
-    dd_partial_split<NQMAX>(acc, j, partial);
-}
-
 // One workgroup: the scalar work of delayed step j (finish: the cycle's last column).
 // The totals, column j - 1 of H and the rotations are staged in LDS; the per-column
 // serial part (|a|^2, a.b, the Givens chain) reads only LDS, everything else is
@@ -610,50 +528,421 @@ __global__ __launch_bounds__(kBlock) void gm_dupdate_kernel(int n, int k, int kp
     }
 }
 
-// One column, 32-vector bucket, FP32: gm_dupdate_kernel with its two outputs on
-// alternate lanes (even: q_j, odd: the next pending vector) over the same rows, the
-// pair's loads of a basis row being one address; each output's operations and order are
-// those of gm_dupdate_kernel (the compiler's contraction of the products may differ, so
-// the vectors agree to rounding).  Mixed GMRES 1e4 / 9e4 / 1e6 rows 1-3 % faster; in FP64
-// the unsplit kernel measured faster on 1e6 rows.
-template <typename T, int NQMAX>
-__global__ __launch_bounds__(kBlock) void gm_dupdate_split_kernel(int n, int j, T* __restrict__ Q, int64_t qstride,
-                                                                  const double* __restrict__ small, GmresLayout L,
-                                                                  const GmresHdr* __restrict__ hd) {
-    if (hd->done && hd->iter != j) return;
-    const bool next = !hd->done;
-    const int side = threadIdx.x & 1;
-    if (side && !next) return;  // no pending vector to form
-    int i0, i1;
-    grow_range(n, i0, i1);
-    const int ro = threadIdx.x >> 1, rows = kBlock / 2;
-    T co[NQMAX];
+// ---------------------------------------------------------------------------
+// One column (nrhs = 1): a delayed step in two kernels (three from kDirectTotals values
+// of partials on), for any n.
+//   gm_one_dots:    v = A u of a tile of rows (CSR operators of short rows; the products of
+//                   consecutive nonzeros through LDS, then a row per thread), and the
+//                   partial sums of a, b, u.u and u.v over the tile
+//   (gm_total_kernel: the 2j + 2 totals)
+//   gm_one_update:  q_j and the next vector; a workgroup of its own does the scalar work
+//                   (column j - 1 of H, its rotation, the stop test), which the vectors
+//                   do not need: their coefficients are a, b, u.u and u.v scaled
+// The basis vectors are dealt over the waves of a workgroup (wave w takes i = w mod 4, NB of
+// them), every wave over the same 256 rows, so that a lane holds 2 NB accumulators instead
+// of 2 j + 2 and no sum crosses waves; u and v come from LDS.  FP64 accumulators as in the
+// other forms.
+// With a kernel each for the product, the dots, the totals, the scalars and the update a
+// step of a 1e4-row system (GMRES(30), FP64) took 30 us, most of it the five kernels'
+// latencies; of a 1e6-row one (FP32 cycles) 61 us, its dots streaming at 3.9 TB/s with two
+// waves per SIMD.  Now 13 and 45 us: solves to 1e-10, 100^2 FP64 13.9 / 7.6 ms, 300^2 31.9 /
+// 19.5, 1000^2 216 / 174; mixed 15.4 / 8.0, 32.6 / 18.9, 169 / 121 ms.  The dots run at
+// 4.6 TB/s (FP64, 1e6 rows, 17-30 vectors and the product: 55 us), the update at 6.
+// A stop is found in gm_one_update, whose other workgroups must not see it: it goes to
+// hd->pend, which the next gm_one_dots reads; that one's first workgroup sets hd->done.
+// ---------------------------------------------------------------------------
+constexpr int kOneVecs = 4;        // the waves that share a tile's rows
+constexpr int kOneRows = 256;      // rows of such a group of waves
+// Values of partials that every workgroup of the update adds itself (32 KB; 9e4 rows with up
+// to 8192: 31.9 -> 25.4 ms a solve, 19.5 so), above that a kernel does.
+constexpr int kDirectTotals = 4096;
+constexpr int kOneRowUpdate = 1 << 17;  // rows up to which the update takes one row per thread: 512 workgroups
+
+// Sums R values per lane over the wave and writes value r to out[at(r)] (at(r) < 0: none).
+template <int R, typename At>
+__device__ __forceinline__ void wave_sums(double (&v)[R], At at, double* out) {
+    const ScatterOut o = wave_scatter_sum<R>(v, 1);
+    if (threadIdx.x % o.low == 0)
 #pragma unroll
-    for (int i = 0; i < NQMAX; ++i) co[i] = i < j ? (T)small[(side ? L.dE : L.dA) + i] : T(0);
-    const T ir = (T)small[L.dsc];
-    const T cj = next ? (T)small[L.dsc + 1] : T(0);
-    T* U = Q + (int64_t)j * qstride;
-    T* V = Q + (int64_t)(j + 1) * qstride;
-    for (int r = i0 + ro; r < i1; r += rows) {
-        T qi[NQMAX];
+        for (int i = 0; i < ScatterSizes<R>::A; ++i)
+            if (i < o.count) {
+                const int t = at(o.base + i);
+                if (t >= 0) out[t] = v[i];
+            }
+}
+
+template <typename T, typename RP, int NB, int TH, bool SPMV>
+__global__ __launch_bounds__(TH, TH == kOneRows ? 1 : 4) void gm_one_dots_kernel(int n, int j, int finish, const RP* __restrict__ rp,
+                                                         const int32_t* __restrict__ ci, const T* __restrict__ a,
+                                                         const T* __restrict__ dl, const T* __restrict__ dr,
+                                                         const T* __restrict__ Q, int64_t qstride,
+                                                         const T* __restrict__ z, T* __restrict__ vslot,
+                                                         double* __restrict__ partial, GmresHdr* __restrict__ hd) {
+    constexpr int EL = 8;  // nonzeros per thread and chunk
+    constexpr int CAP = TH * EL;
+    constexpr int GROUPS = TH / kOneRows;
+    constexpr int RQ = kOneRows / kWave;        // rows per lane
+    constexpr int VB = NB > 4 && TH > kOneRows ? (sizeof(T) == 8 ? 2 : 4) : NB;  // vectors in flight
+    constexpr int R = 2 * NB + 2;
+    __shared__ T prod[SPMV ? CAP : 1];
+    __shared__ RP srp[SPMV ? TH + 1 : 1];
+    __shared__ T sv[TH], su[TH];
+    __shared__ double sums[GROUPS > 1 ? GROUPS * (2 * kDdMaxM + 2) : 1];
+    if (hd->done) return;
+    if (hd->pend) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) hd->done = 1;
+        return;
+    }
+    // wave ids in scalar registers: a basis vector's address is one scalar pair and a lane offset
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int w = wave % kOneVecs, grp = wave / kOneVecs;
+    const int B = gridDim.x, lb = xcd_swizzle(blockIdx.x, B);
+    const int tiles = (n + TH - 1) / TH;
+    const T* U = Q + (int64_t)j * qstride;
+    double acc[R];
 #pragma unroll
-        for (int i = 0; i < NQMAX; ++i) qi[i] = Q[(int64_t)max(0, min(i, j - 1)) * qstride + r];  // loads first
-        const T uv = U[r];
-        T out;
-        if (side) {
-            const T vv = V[r];
-            out = vv * ir - cj * uv;
-        } else {
-            out = uv * ir;
+    for (int r = 0; r < R; ++r) acc[r] = 0.0;
+    for (int t = (int)((int64_t)tiles * lb / B); t < (int)((int64_t)tiles * (lb + 1) / B); ++t) {
+        const int base = t * TH, nr = min(TH, n - base);
+        const int row = base + min((int)threadIdx.x, nr - 1);
+        const T uown = U[row];
+        T qv[VB][RQ];
+        unsigned off[RQ];  // clamped rows
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) off[q] = (unsigned)min(grp * kOneRows + lane + q * kWave, nr - 1);
+        auto load_q = [&](int b0) {  // at clamped vectors
+#pragma unroll
+            for (int b = 0; b < VB; ++b) {
+                const T* qb = Q + (int64_t)max(0, min(w + kOneVecs * (b0 + b), j - 1)) * qstride + base;
+#pragma unroll
+                for (int q = 0; q < RQ; ++q) qv[b][q] = qb[off[q]];
+            }
+        };
+        if constexpr (VB == NB) load_q(0);  // on their way during the product
+        T vown = uown;
+        if (SPMV && !finish) {
+            for (int i = threadIdx.x; i <= nr; i += TH) srp[i] = rp[base + i];
+            __syncthreads();
+            const RP l0 = srp[0], l1 = srp[nr];
+            T sum = T(0);
+            const RP rb = threadIdx.x < nr ? srp[threadIdx.x] : l0, re = threadIdx.x < nr ? srp[threadIdx.x + 1] : l0;
+            for (RP cs = l0; cs < l1; cs += CAP) {
+                const int cnt = (int)((l1 - cs) < (RP)CAP ? (l1 - cs) : (RP)CAP);
+                int32_t c[EL];
+                T av[EL], xv[EL];
+#pragma unroll
+                for (int e = 0; e < EL; ++e) {  // clamped to the chunk's last nonzero
+                    const RP at = cs + min((int)threadIdx.x + e * TH, cnt - 1);
+                    c[e] = __builtin_nontemporal_load(ci + at);
+                    av[e] = a ? __builtin_nontemporal_load(a + at) : T(1);
+                }
+#pragma unroll
+                for (int e = 0; e < EL; ++e) xv[e] = dr ? dr[c[e]] * U[c[e]] : U[c[e]];
+#pragma unroll
+                for (int e = 0; e < EL; ++e) {
+                    const int at = threadIdx.x + e * TH;
+                    if (at < cnt) prod[at] = av[e] * xv[e];
+                }
+                __syncthreads();
+                const int b0 = (int)((rb > cs ? rb : cs) - cs), b1 = (int)((re < cs + cnt ? re : cs + cnt) - cs);
+                for (int l = b0; l < b1; ++l) sum += prod[l];
+                __syncthreads();
+            }
+            vown = dl ? dl[row] * sum : sum;
+            if (threadIdx.x < nr) vslot[row] = vown;
+        } else if (!finish) {
+            if (dl) {
+                vown = dl[row] * z[row];
+                if (threadIdx.x < nr) vslot[row] = vown;
+            } else {
+                vown = vslot[row];
+            }
+        }
+        su[threadIdx.x] = threadIdx.x < nr ? uown : T(0);
+        sv[threadIdx.x] = threadIdx.x < nr ? vown : T(0);
+        __syncthreads();
+        T uv[RQ], vv[RQ];
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            uv[q] = su[grp * kOneRows + lane + q * kWave];
+            vv[q] = sv[grp * kOneRows + lane + q * kWave];
         }
 #pragma unroll
-        for (int i = 0; i < NQMAX; ++i)
-            if (i < j) out -= co[i] * qi[i];
-        if (side)
-            V[r] = out;
-        else if (j > 0)
-            U[r] = out;
+        for (int b0 = 0; b0 < NB; b0 += VB) {
+            if constexpr (VB != NB) load_q(b0);
+#pragma unroll
+            for (int b = 0; b < VB; ++b)
+#pragma unroll
+                for (int q = 0; q < RQ; ++q) {
+                    acc[b0 + b] += (double)qv[b][q] * (double)uv[q];
+                    acc[NB + b0 + b] += (double)qv[b][q] * (double)vv[q];
+                }
+        }
+        if (w == kOneVecs - 1)
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) {
+                acc[2 * NB] += (double)uv[q] * (double)uv[q];
+                acc[2 * NB + 1] += (double)uv[q] * (double)vv[q];
+            }
+        __syncthreads();
     }
+    const int nv = 2 * j + 2;
+    auto at = [&](int r) {  // place of register r among the 2j + 2 values
+        if (r >= 2 * NB) return w == kOneVecs - 1 ? 2 * j + (r - 2 * NB) : -1;
+        const int i = w + kOneVecs * (r < NB ? r : r - NB);
+        return i < j ? (r < NB ? i : j + i) : -1;
+    };
+    double* out = partial + (int64_t)lb * nv;
+    if constexpr (GROUPS == 1) {
+        wave_sums<R>(acc, at, out);
+    } else {
+        wave_sums<R>(acc, at, sums + grp * (2 * kDdMaxM + 2));
+        __syncthreads();
+        for (int i = threadIdx.x; i < nv; i += TH) {
+            double s = 0.0;
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g) s += sums[g * (2 * kDdMaxM + 2) + i];
+            out[i] = s;
+        }
+    }
+}
+
+struct OneScalarLds {
+    double sv[2 * kDdMaxM + 2];                  // the totals
+    double hm[(kDdMaxM + 1) * (kDdMaxM + 1)];    // Hraw, rows 0..j, columns 0..j-1
+    double rot[2 * kDdMaxM];                     // cs, sn of rotations 0..j-2
+    double col[kDdMaxM + 1];                     // column j - 1, rotated
+    double g[kDdMaxM + 1];                       // column j, first pass
+    int conv;
+};
+
+// What gm_dscalar_kernel does, for one column, by a workgroup of kBlock threads.  `stage`
+// runs before the totals are known (its loads are in flight with theirs), `finish_step`
+// after lds.sv holds them and the workgroup has synchronised; it returns whether the cycle
+// stops here.  Wave 0 rotates column j - 1 while the others form column j.
+__device__ __forceinline__ void one_scalar_stage(int j, int m, const double* __restrict__ small, const GmresLayout& L,
+                                                 OneScalarLds& lds) {
+    constexpr int W = kDdMaxM + 1;
+    for (int t = threadIdx.x; t < j * (j + 1); t += kBlock) {
+        const int r = t / j, c = t % j;
+        lds.hm[r * W + c] = r <= c + 1 ? small[L.Hraw + (int64_t)r * m + c] : 0.0;
+    }
+    for (int t = threadIdx.x; t < j - 1; t += kBlock) {
+        lds.rot[t] = small[L.cs + t];
+        lds.rot[kDdMaxM + t] = small[L.sn + t];
+    }
+}
+
+__device__ __forceinline__ bool one_scalar_step(int j, int m, int finish, double* __restrict__ small,
+                                                const GmresLayout& L, const GmresHdr* __restrict__ hd,
+                                                OneScalarLds& lds) {
+    constexpr int W = kDdMaxM + 1;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, jj = j - 1;
+    double* H = small + L.H;
+    double* Hr = small + L.Hraw;
+    // |a|^2 and a.b, by every wave alike
+    double aa = 0.0, ab = 0.0;
+    const double alane = lane < j ? lds.sv[lane] : 0.0;
+    if (lane < j) {
+        aa = alane * alane;
+        ab = alane * lds.sv[j + lane];
+    }
+    aa = group_sum<kWave>(aa);
+    ab = group_sum<kWave>(ab);
+    const double alpha = lds.sv[2 * j], beta = lds.sv[2 * j + 1];
+    // |u - Q a|; at a breakdown (u in the span of Q to rounding) at least 2^-52 |u|
+    const double rho = j > 0 ? sqrt(fmax(alpha - aa, 0x1p-104 * alpha)) : 1.0;
+    const double irho = 1.0 / rho;
+    if (j > 0) {
+        // column jj completed: its second pass and |u - Q a|
+        if (wave == 0 && lane <= j) {
+            const double v = lane < j ? lds.hm[lane * W + jj] + alane : rho;
+            lds.hm[lane * W + jj] = v;
+            lds.col[lane] = v;
+            Hr[(int64_t)lane * m + jj] = v;
+        }
+        __syncthreads();
+    }
+    if (wave == 0) {
+        if (lane == 0 && j > 0) {
+            // Givens on column jj (GMRES.hpp:603-658)
+            const double bj = small[L.beta + jj], lim = small[L.TOL];
+            double xi = lds.col[0];
+#pragma unroll 4
+            for (int i = 0; i < jj; ++i) {
+                const double eta = lds.col[i + 1], co = lds.rot[i], si = lds.rot[kDdMaxM + i];
+                lds.col[i] = co * xi + si * eta;
+                xi = -si * xi + co * eta;
+            }
+            const double eta = lds.col[j];
+            const double r = sqrt(xi * xi + eta * eta);
+            double co, si;
+            if (fabs(xi) <= 2.220446049250313e-16 * r) {
+                co = 0.0;
+                si = 1.0;
+            } else {
+                const double rinv = 1.0 / r;
+                co = fabs(xi) * rinv;
+                si = (xi / fabs(xi)) * eta * rinv;
+            }
+            lds.col[jj] = co * xi + si * eta;
+            lds.col[j] = 0.0;
+            small[L.cs + jj] = co;
+            small[L.sn + jj] = si;
+            small[L.beta + j] = -si * bj;
+            small[L.beta + jj] = co * bj;
+            lds.conv = fabs(-si * bj) <= lim ? 1 : 0;
+        }
+        if (lane == 0 && j == 0) lds.conv = 0;
+    } else if (!finish) {
+        // column j, first pass: g_l = (t_l - (Hraw a)_l) / rho, four lanes to a row
+        const double tj = j > 0 ? (beta - ab) * irho : beta;
+        const int t = threadIdx.x - kWave, part = t % 4;
+        for (int l = t / 4; l <= j; l += (kBlock - kWave) / 4) {
+            double ha = 0.0;
+            for (int i = part; i < j; i += 4) ha += lds.hm[l * W + i] * lds.sv[i];
+            ha += shfl_xor(ha, 1);
+            ha += shfl_xor(ha, 2);
+            if (part == 0) lds.g[l] = ((l < j ? lds.sv[j + l] : tj) - ha) * irho;
+        }
+    }
+    __syncthreads();
+    const bool stop = j > 0 && (lds.conv || j >= hd->m);
+    if (j > 0 && threadIdx.x <= j) H[(int64_t)threadIdx.x * m + jj] = lds.col[threadIdx.x];
+    if (!finish && !stop && threadIdx.x <= j) {
+        Hr[(int64_t)threadIdx.x * m + j] = lds.g[threadIdx.x];
+        H[(int64_t)threadIdx.x * m + j] = lds.g[threadIdx.x];
+    }
+    return stop;
+}
+
+// q_j = u / rho - sum a_i / rho q_i (slot j) and, unless finishing, the next vector (slot
+// j + 1, in place of v); the last workgroup does the scalar work instead.  `parts` > 0:
+// every workgroup adds the partials of that many workgroups itself, else `tot` holds them.
+// RQ rows per thread, VB vectors in flight: 1 and 32 where one row per thread fills few
+// workgroups (a single round trip), else 4 and 8.
+template <typename T, int RQ, int VB>
+__global__ __launch_bounds__(kBlock) void gm_one_update_kernel(int n, int j, int m, int finish, T* __restrict__ Q,
+                                                               int64_t qstride, int parts,
+                                                               const double* __restrict__ partial,
+                                                               const double* __restrict__ tot,
+                                                               double* __restrict__ small, GmresLayout L,
+                                                               GmresHdr* __restrict__ hd) {
+    constexpr int W = kBlock / kWave;
+    __shared__ OneScalarLds lds;
+    __shared__ double wsum[W][2 * kDdMaxM + 2];
+    __shared__ T ca[kDdMaxM], ce[kDdMaxM];
+    const bool scalar = blockIdx.x == gridDim.x - 1;
+    const int nv = 2 * j + 2;
+    const int done = hd->done;
+    const int64_t b0 = (int64_t)blockIdx.x * (kBlock * RQ);
+    T* U = Q + (int64_t)j * qstride + b0;
+    T* V = Q + (int64_t)(j + 1) * qstride + b0;
+    unsigned row[RQ];  // within the workgroup's rows, clamped
+    T uv[RQ], vv[RQ], qv[VB][RQ];
+    auto load_q = [&](int i0) {
+#pragma unroll
+        for (int b = 0; b < VB; ++b) {
+            const T* qb = Q + (int64_t)max(0, min(i0 + b, j - 1)) * qstride + b0;
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) qv[b][q] = qb[row[q]];
+        }
+    };
+    if (!scalar) {  // the first loads are on their way during the totals
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            row[q] = (unsigned)min((int64_t)threadIdx.x + q * kBlock, n - 1 - b0);
+            uv[q] = U[row[q]];
+            vv[q] = finish ? T(0) : V[row[q]];
+        }
+        load_q(0);
+    } else {
+        one_scalar_stage(j, m, small, L, lds);
+    }
+    if (parts > 0) {
+        // lane groups of nvp = 2^ceil(log2 nv) lanes (at most the wave) share a wave's partials
+        const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+        int nvp = 2;
+        while (nvp < nv && nvp < kWave) nvp *= 2;
+        const int sub = lane / nvp, S = W * (kWave / nvp), b1 = wave * (kWave / nvp) + sub;
+        for (int i0 = 0; i0 < nv; i0 += nvp) {
+            const int i = i0 + lane % nvp;
+            double s[4] = {0.0, 0.0, 0.0, 0.0};
+            if (i < nv) {
+                int b = b1;
+                for (; b + 3 * S < parts; b += 4 * S)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) s[q] += partial[(int64_t)(b + q * S) * nv + i];
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    if (b + q * S < parts) s[q] += partial[(int64_t)(b + q * S) * nv + i];
+            }
+            double t = (s[0] + s[1]) + (s[2] + s[3]);
+            for (int off = kWave / 2; off >= nvp; off >>= 1) t += shfl_xor(t, off);
+            if (lane < nvp && i < nv) wsum[wave][i] = t;
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < nv; i += kBlock)
+            lds.sv[i] = (wsum[0][i] + wsum[1][i]) + (wsum[2][i] + wsum[3][i]);
+    } else {
+        for (int i = threadIdx.x; i < nv; i += kBlock) lds.sv[i] = tot[i];
+    }
+    if (done) return;
+    __syncthreads();
+    if (scalar) {
+        const bool stop = one_scalar_step(j, m, finish, small, L, hd, lds);
+        if (threadIdx.x == 0 && j > 0) {
+            hd->iter = j;
+            hd->succ = lds.conv;
+            if (stop) hd->pend = 1;
+        }
+        return;
+    }
+    // rho and a.b as in one_scalar_step, by every wave alike
+    const int lane = threadIdx.x % kWave;
+    double aa = 0.0, ab = 0.0;
+    if (lane < j) {
+        const double ai = lds.sv[lane];
+        aa = ai * ai;
+        ab = ai * lds.sv[j + lane];
+    }
+    aa = group_sum<kWave>(aa);
+    ab = group_sum<kWave>(ab);
+    const double alpha = lds.sv[2 * j], beta = lds.sv[2 * j + 1];
+    const double irho = j > 0 ? 1.0 / sqrt(fmax(alpha - aa, 0x1p-104 * alpha)) : 1.0;
+    const double tj = j > 0 ? (beta - ab) * irho : beta;
+    const double cjd = tj * irho * irho;
+    if (threadIdx.x < j) {
+        ca[threadIdx.x] = (T)(lds.sv[threadIdx.x] * irho);
+        ce[threadIdx.x] = (T)(lds.sv[j + threadIdx.x] * irho - cjd * lds.sv[threadIdx.x]);
+    }
+    __syncthreads();
+    const T ir = (T)irho, cj = (T)cjd;
+    T qo[RQ], no[RQ];
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+        qo[q] = uv[q] * ir;
+        no[q] = vv[q] * ir - cj * uv[q];
+    }
+    for (int i0 = 0; i0 < j; i0 += VB) {
+        if (i0 > 0) load_q(i0);
+#pragma unroll
+        for (int b = 0; b < VB; ++b)
+            if (i0 + b < j) {
+                const T cai = ca[i0 + b], cei = ce[i0 + b];
+#pragma unroll
+                for (int q = 0; q < RQ; ++q) {
+                    qo[q] -= cai * qv[b][q];
+                    no[q] -= cei * qv[b][q];
+                }
+            }
+    }
+#pragma unroll
+    for (int q = 0; q < RQ; ++q)
+        if (b0 + threadIdx.x + q * kBlock < n) {
+            if (j > 0) U[row[q]] = qo[q];
+            if (!finish) V[row[q]] = no[q];
+        }
 }
 
 // H[j+1][j] = |q|; Givens (GMRES.hpp:603-658); beta; convergence; ++iter.  |q|^2 per
@@ -816,13 +1105,14 @@ __global__ void gm_start_kernel(int m, int k, const double* __restrict__ nn2, do
         hd->succ = conv;
         hd->m = m;
         hd->done = (conv || m <= 0) ? 1 : 0;
+        hd->pend = 0;
     }
 }
 
 // y = H^{-1} beta per column (upper back substitution, iter x iter).  The triangle of
-// H and beta of a chunk of columns are first staged in LDS by the whole workgroup, so
-// the serial substitution of each column reads LDS only; the order of the
-// subtractions is the plain row-oriented one.
+// H and beta of a chunk of columns are first staged in LDS by the whole workgroup; a wave
+// then substitutes a column, a lane per row, column by column of the triangle (one thread
+// per column, row by row, took 22 us for 30 rows: a chain of 450 dependent reads).
 constexpr int kLsqLds = 6144;  // doubles of staged triangle per chunk of columns
 __global__ __launch_bounds__(kBlock) void gm_lsq_kernel(int m, int k, double* __restrict__ small, GmresLayout L,
                                                         const GmresHdr* __restrict__ hd) {
@@ -842,12 +1132,19 @@ __global__ __launch_bounds__(kBlock) void gm_lsq_kernel(int m, int k, double* __
         for (int t = threadIdx.x; t < it * nc; t += blockDim.x)
             sb[(t / nc) * kGmresMaxCols + t % nc] = small[L.beta + (t / nc) * k + c0 + t % nc];
         __syncthreads();
-        for (int cc = threadIdx.x; cc < nc; cc += blockDim.x)
+        // a wave per column, a lane per row: y_i, then every lane above takes t_li y_i off
+        const int lane = threadIdx.x % kWave;
+        for (int cc = threadIdx.x / kWave; cc < nc; cc += kBlock / kWave) {
+            double s = lane < it ? sb[lane * kGmresMaxCols + cc] : 0.0;
+            const double diag = lane < it ? tri[tix(lane, lane) * nc + cc] : 1.0;
             for (int i = it - 1; i >= 0; --i) {
-                double s = sb[i * kGmresMaxCols + cc];
-                for (int j = i + 1; j < it; ++j) s -= tri[tix(i, j) * nc + cc] * sb[j * kGmresMaxCols + cc];
-                sb[i * kGmresMaxCols + cc] = s / tri[tix(i, i) * nc + cc];
+                const double t = lane < i ? tri[tix(lane, i) * nc + cc] : 0.0;
+                const double y = __shfl(s, i, kWave) / __shfl(diag, i, kWave);
+                if (lane < i) s -= t * y;
+                if (lane == i) s = y;
             }
+            if (lane < it) sb[lane * kGmresMaxCols + cc] = s;
+        }
         __syncthreads();
         for (int t = threadIdx.x; t < it * nc; t += blockDim.x)
             small[L.y + (t / nc) * k + c0 + t % nc] = sb[(t / nc) * kGmresMaxCols + t % nc];
@@ -867,7 +1164,19 @@ __global__ __launch_bounds__(kBlock) void gm_synth_kernel(int n, int k, const T*
     for (int64_t e = blockIdx.x * (int64_t)kBlock + threadIdx.x; e < total; e += (int64_t)gridDim.x * kBlock) {
         const int c = (int)(e % k);
         T zv = T(0);
-        for (int j = 0; j < it; ++j) zv += (T)small[L.y + j * k + c] * Q[j * qstride + e];
+        constexpr int U = 8;  // vectors in flight (clamped to a valid one)
+        for (int j0 = 0; j0 < it; j0 += U) {
+            T qv[U], yv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int j = min(j0 + u, it - 1);
+                qv[u] = Q[j * qstride + e];
+                yv[u] = (T)small[L.y + j * k + c];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (j0 + u < it) zv += yv[u] * qv[u];
+        }
         if (d_right) zv = d_right[e / k] * zv;
         sol[e] = implicit_zero ? -zv : sol[e] - zv;
     }
@@ -967,22 +1276,6 @@ template <typename T, int NQMAX>
 static void launch_ddots(hipStream_t s, int gb, int n, int k, int kpad, int j, int finish, const T* Q, int64_t qs,
                          const T* z, const T* d, T* v, double* partial, const GmresHdr* hd) {
     const size_t lds = (size_t)(kBlock / kWave) * (2 * j + 2) * k * sizeof(double);
-    if constexpr (NQMAX == 32) {
-        // FP64 on 2^19 rows and more: the unsplit pass (1e6 rows: 210 against 214 ms)
-        if (k == 1 && g_gmres_split_dots && (sizeof(T) == 4 || n < (1 << 19))) {
-            bool two = false;
-            if constexpr (sizeof(T) == 4) two = n >= (1 << 19);
-            if (two) {
-                if constexpr (sizeof(T) == 4)
-                    hipLaunchKernelGGL((gm_ddots_split_kernel<T, NQMAX, 2>), dim3(gb), dim3(kBlock), lds, s, n, j,
-                                       finish, Q, qs, z, d, v, partial, hd);
-            } else {
-                hipLaunchKernelGGL((gm_ddots_split_kernel<T, NQMAX, 1>), dim3(gb), dim3(kBlock), lds, s, n, j, finish,
-                                   Q, qs, z, d, v, partial, hd);
-            }
-            return;
-        }
-    }
     hipLaunchKernelGGL((gm_ddots_kernel<T, NQMAX>), dim3(gb), dim3(kBlock), lds, s, n, k, kpad, j, finish, Q, qs, z,
                        d, v, partial, hd);
 }
@@ -1004,11 +1297,41 @@ static void dupdate(hipStream_t s, int gb, int n, int k, int kpad, int j, T* Q, 
     else if (j <= 16)
         hipLaunchKernelGGL((gm_dupdate_kernel<T, 16>), dim3(gb), dim3(kBlock), 0, s, n, k, kpad, j, Q, qs, small, L,
                            hd);
-    else if (sizeof(T) == 4 && k == 1 && g_gmres_split_dots)  // FP64: the unsplit pass measured faster
-        hipLaunchKernelGGL((gm_dupdate_split_kernel<T, 32>), dim3(gb), dim3(kBlock), 0, s, n, j, Q, qs, small, L, hd);
     else
         hipLaunchKernelGGL((gm_dupdate_kernel<T, 32>), dim3(gb), dim3(kBlock), 0, s, n, k, kpad, j, Q, qs, small, L,
                            hd);
+}
+
+// The one-column dots kernel: NB vectors per wave by the basis size, 512 threads (two
+// groups of 256 rows, 16 waves per CU with kGB workgroups) where tiles of 256 rows would make
+// more than kGB of them.
+template <typename T, typename RP, bool SPMV>
+static int one_dots(hipStream_t s, int n, int j, int finish, const CsrView* A, const T* dl, const T* dr, const T* Q,
+                    int64_t qs, const T* z, T* v, double* partial, GmresHdr* hd) {
+    const RP* rp = SPMV ? (const RP*)A->rp : nullptr;
+    const int32_t* ci = SPMV ? A->ci : nullptr;
+    const T* a = SPMV ? (const T*)A->val : nullptr;
+    const bool big = n > kGB * kOneRows;
+    const int th = big ? 2 * kOneRows : kOneRows;
+    const int B = std::min(kGB, (n + th - 1) / th);
+#define TG_ONE(NB)                                                                                              \
+    if (big)                                                                                                    \
+        hipLaunchKernelGGL((gm_one_dots_kernel<T, RP, NB, 2 * kOneRows, SPMV>), dim3(B), dim3(2 * kOneRows), 0, s, \
+                           n, j, finish, rp, ci, a, dl, dr, Q, qs, z, v, partial, hd);                          \
+    else                                                                                                        \
+        hipLaunchKernelGGL((gm_one_dots_kernel<T, RP, NB, kOneRows, SPMV>), dim3(B), dim3(kOneRows), 0, s, n, j, \
+                           finish, rp, ci, a, dl, dr, Q, qs, z, v, partial, hd)
+    if (j <= kOneVecs) {
+        TG_ONE(1);
+    } else if (j <= 2 * kOneVecs) {
+        TG_ONE(2);
+    } else if (j <= 4 * kOneVecs) {
+        TG_ONE(4);
+    } else {
+        TG_ONE(8);
+    }
+#undef TG_ONE
+    return B;
 }
 
 static int grid_elems(int64_t count) {
@@ -1175,9 +1498,43 @@ int gmres_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d,
     // step per cycle.  Used where its partial sums fit the LDS (2m + 2 values of k columns)
     // and its registers (m <= 32).
     const bool delayed = g_gmres_delayed && mm <= kDdMaxM && (2 * mm + 2) * k <= 2048;
+    // One column: two or three kernels a step, the product among them for a CSR operator of
+    // short rows (mean length up to 16; its row sums are a thread per row).
+    const bool one = delayed && k == 1 && g_gmres_split_dots;
+    const CsrView* Ao = Aop.csr;
+    const bool one_spmv = one && !host_ops && Ao && Ao->m == n && Ao->n == n && Ao->nnz <= 16 * (int64_t)n && Ao->rp &&
+                          (Ao->nnz == 0 || Ao->ci) && !Ao->longr &&
+                          (Ao->rp_type == TG_I32 || Ao->rp_type == TG_I64) &&
+                          Ao->val_type == (sizeof(T) == 8 ? TG_F64 : TG_F32);
+    auto one_step = [&](hipStream_t st, int j, bool finish, T* V) -> int {
+        const int f = finish ? 1 : 0, nv = 2 * j + 2;
+        const T* dl = side == 0 && !finish ? dd : nullptr;
+        const T* dr = side == 1 && !finish ? dd : nullptr;
+        int B;
+        if (one_spmv)
+            B = Ao->rp_type == TG_I64
+                    ? one_dots<T, int64_t, true>(st, n, j, f, Ao, dl, dr, Q, qstride, z, V, w.partial, w.hd)
+                    : one_dots<T, int32_t, true>(st, n, j, f, Ao, dl, dr, Q, qstride, z, V, w.partial, w.hd);
+        else
+            B = one_dots<T, int32_t, false>(st, n, j, f, nullptr, dl, nullptr, Q, qstride, z, V, w.partial, w.hd);
+        const bool direct = B * nv <= kDirectTotals;
+        if (!direct)
+            hipLaunchKernelGGL(gm_total_kernel, dim3(nv), dim3(kBlock), 0, st, nv, 1, B, (const double*)w.partial, w.tot,
+                               (const GmresHdr*)w.hd);
+        if (n <= kOneRowUpdate)
+            hipLaunchKernelGGL((gm_one_update_kernel<T, 1, 32>), dim3((n + kBlock - 1) / kBlock + 1), dim3(kBlock), 0, st,
+                               n, j, mm, f, Q, qstride, direct ? B : 0, (const double*)w.partial, (const double*)w.tot,
+                               w.small, L, w.hd);
+        else
+            hipLaunchKernelGGL((gm_one_update_kernel<T, 4, 8>), dim3((n + 4 * kBlock - 1) / (4 * kBlock) + 1),
+                               dim3(kBlock), 0, st, n, j, mm, f, Q, qstride, direct ? B : 0, (const double*)w.partial,
+                               (const double*)w.tot, w.small, L, w.hd);
+        return TG_OK;
+    };
     auto delayed_step = [&](hipStream_t st, int j, bool finish) -> int {
         T* U = Q + (int64_t)j * qstride;
         T* V = finish ? U : Q + (int64_t)(j + 1) * qstride;
+        if (one_spmv) return one_step(st, j, finish, V);
         if (!finish) {
             int rc;
             if (side == 0) {
@@ -1190,6 +1547,7 @@ int gmres_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d,
             }
             if (rc) return rc;
         }
+        if (one) return one_step(st, j, finish, V);
         const int nv = 2 * j + 2;
         ddots<T>(st, gb, n, k, kpad, j, finish ? 1 : 0, (const T*)Q, qstride, (const T*)z,
                  (side == 0 && !finish) ? dd : nullptr, V, w.partial, (const GmresHdr*)w.hd);
@@ -1271,7 +1629,7 @@ int gmres_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d,
                 TG_LAUNCH_CHECK();
                 TG_HIP(hipMemcpyAsync(&hh, w.hd, sizeof(hh), hipMemcpyDeviceToHost, s));
                 TG_HIP(hipStreamSynchronize(s));
-                if (hh.done) break;
+                if (hh.done || hh.pend) break;
                 if (!host_ops) batch = std::min(batch * 2, 16);
             }
             int rcf = finish_cycle(s);  // returns at once on the device when the cycle stopped early

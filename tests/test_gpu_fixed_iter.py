@@ -214,6 +214,49 @@ def test_gmres_fixed_cycles_match_oracle(cuda, gmres_delayed, m, cycles, side, p
     assert rel_err(gm.GetHessenbergMatrix().cpu().numpy(), H_o) <= TOL
 
 
+@pytest.mark.parametrize("n,m,per_row", [(3, 4, 1), (255, 12, 4), (257, 5, 9), (1031, 9, 14), (2000, 12, 30), (5003, 17, 3),
+                                         (131071, 12, 4), (131073, 10, 4), (262147, 6, 12)])
+@pytest.mark.parametrize("side,prec", [(0, False), (0, True), (1, True)], ids=["plain", "left", "right"])
+def test_gmres_one_column_shapes(cuda, n, m, per_row, side, prec):
+    """The one-column step (product, dots and totals in a kernel; the update and the scalar
+    work in another) around the sizes where its launch changes: tiles of 256 and 512 rows and
+    their remainders, one and four rows per thread of the update, totals added by every
+    workgroup or by their own kernel, basis sizes of every bucket, a row longer than a chunk
+    of the product, rows too long for the fused product (mean 30), both row-pointer types.
+    Two cycles against the oracle at the bar of this file; A = 2 I + W with |W| <= 1, whose
+    cycles of at most 17 steps stay above rounding (each step takes off a factor of about 4;
+    17 steps 1e-10, so the last columns are compared at 1e-12 of the first)."""
+    rng = np.random.default_rng(n + m)
+    cnt = n * per_row
+    i, j = rng.integers(0, n, cnt), rng.integers(0, n, cnt)
+    if n > 1000:
+        i[: min(3000, n)] = n // 3  # one long row
+    W = sp.coo_matrix((rng.uniform(-1, 1, cnt), (i, j)), shape=(n, n)).tocsr()
+    r, c = (np.asarray(abs(W).sum(a)).ravel() for a in (1, 0))
+    W = sp.diags(1.0 / np.sqrt(np.maximum(r, 1e-3))) @ W @ sp.diags(1.0 / np.sqrt(np.maximum(c, 1e-3)))
+    A = (W + 2.0 * sp.identity(n)).tocsr()
+    A.sort_indices()
+    rp, ci, val = A.indptr.astype(np.int64), A.indices.astype(np.int32), A.data
+    d = rng.uniform(0.9, 1.1, n) if prec else None
+    B = gen.uniform(5600 + n, n).reshape(n, 1)
+    Xo = np.zeros((n, 1))
+    ok_o, it_o, rs_o, rr_o, Q_o, H_o, beta_o, sol_o = oracle.gmres_ex(
+        n, rp, ci, val, B, Xo, 1, m, 0.0, 1, prec_diag=d, side=side)
+    gm = GMRES(n, m, 1, side=side)
+    Xd = torch.zeros(n, 1, dtype=torch.float64, device=cuda)
+    gm(MatrixCSR(rp if n % 2 else rp.astype(np.int32), ci, val, n, n), None if d is None else dev(d, cuda), 1.0,
+       dev(B, cuda), 0.0, Xd, 0.0, 1)
+    if n == 3:  # the Krylov space is used up: only the solution is determined
+        assert rel_err(Xd.cpu().numpy(), np.linalg.solve(A.toarray(), B)) <= TOL
+        return
+    assert gm.IterationCount() == it_o == m and gm.RestartCount() == rs_o == 1
+    assert rel_err(Xd.cpu().numpy(), Xo) <= TOL
+    assert res_err(gm.RelativeResiduals(), rr_o) <= TOL
+    scale = max(1.0, 1e-2 / float(rr_o[0]) ** 0.5)  # the second cycle starts from the first's residual
+    assert rel_err(gm.GetBasis().cpu().numpy(), Q_o) <= TOL * scale
+    assert rel_err(gm.GetHessenbergMatrix().cpu().numpy(), H_o) <= TOL * scale
+
+
 @pytest.mark.parametrize("k", [2, 8, 16])
 def test_gmres_fixed_cycles_wide_blocks(cuda, gmres_delayed, k):
     """Blocks of 2, 8 and 16 right-hand sides (two, eight and sixteen column lanes in the

@@ -8,9 +8,11 @@ import subprocess
 import numpy as np
 import pytest
 import scipy.sparse as sp
+import torch
 
 import oracle
 from helpers import rel_err
+from tensors_amd import TensorsError
 from tensors_amd import structure as st
 
 pytestmark = pytest.mark.gpu
@@ -57,6 +59,90 @@ def test_from_triples_float_values_and_empty(cuda):
     assert np.max(np.abs(gval - A.data)) <= 1e-14 * np.max(np.abs(A.data))
     rp0, ci0, v0 = st.from_triples(np.zeros(0, np.int32), np.zeros(0, np.int32), np.zeros(0), 7, 7)
     assert np.all(rp0 == 0) and len(ci0) == 0
+
+
+def numpy_triples(I, J, V, m, compress, symmetrize):
+    """Stable sort by (row, column); duplicates added one by one in input order."""
+    if symmetrize:
+        off = I != J
+        I, J, V = np.r_[I, J[off]], np.r_[J, I[off]], np.r_[V, V[off]]
+    order = np.lexsort((J, I))
+    I, J, V = I[order], J[order], V[order]
+    head = np.ones(len(I), bool)
+    if compress:
+        head[1:] = (I[1:] != I[:-1]) | (J[1:] != J[:-1])
+    at = np.flatnonzero(head)
+    val = V[at].copy()
+    end = np.r_[at[1:], len(I)]
+    for step in range(1, int((end - at).max()) if len(at) else 0):
+        more = at + step < end
+        val[more] += V[at[more] + step]
+    rp = np.zeros(m + 1, np.int64)
+    np.cumsum(np.bincount(I[head], minlength=m), out=rp[1:])
+    return rp, J[at].astype(np.int32), val
+
+
+@pytest.mark.parametrize("case", ["edge", "one_bucket", "mesh", "few_rows", "many_rows", "duplicates", "long_row",
+                                  "crowded_rows", "wide"])
+@pytest.mark.parametrize("compress,symmetrize", [(True, False), (False, False), (True, True)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, None])
+def test_from_triples_forms_agree(cuda, case, compress, symmetrize, dtype):
+    """The bucket form and the radix form, on both sides of every line between them (4095
+    and 4096 triples, rows of at most / more than 512 triples, a bucket that overflows, more
+    columns than a word holds stay out), against a stable sort with the duplicates added in
+    input order: structure and values bit for bit, FP64 / FP32 / none, both row-pointer
+    types."""
+    from tensors_amd import _capi as capi
+    import ctypes
+
+    rng = np.random.default_rng(len(case) * 7 + compress * 2 + symmetrize)
+    m, n, cnt = {"edge": (900, 900, 4096), "one_bucket": (50, 50, 4095), "mesh": (30011, 30011, 200003),
+                 "few_rows": (40, 40, 5000), "many_rows": (60001, 60001, 5003), "duplicates": (2500, 2500, 60007),
+                 "long_row": (4001, 4001, 30011), "crowded_rows": (20011, 20011, 40009),
+                 "wide": (3001, 2000003, 50021)}[case]
+    if symmetrize and m != n:
+        n = m
+    I, J = rng.integers(0, m, cnt), rng.integers(0, n, cnt)
+    if case == "mesh":  # runs of neighbouring rows, as elements give them
+        I = np.sort(I)
+        J = np.minimum(I + rng.integers(0, 5, cnt), n - 1)
+    if case == "duplicates":
+        J = I // 16 * 16 + rng.integers(0, 3, cnt)
+        J = np.minimum(J, n - 1)
+    if case == "long_row":
+        I[::37] = 77  # more than 512 triples: the radix form
+    if case == "crowded_rows":
+        I[::3] = rng.integers(500, 540, len(I[::3]))  # 40 rows of about 330: a bucket of more than it holds
+    I, J = I.astype(np.int32), J.astype(np.int32)
+    V = rng.uniform(-1, 1, cnt).astype(dtype or np.float64)
+    orp, oci, oval = numpy_triples(I, J, V, m, compress, symmetrize)
+    T = lambda a: torch.from_numpy(a).to(cuda)
+    dI, dJ, dV = T(I), T(J), T(V)
+    cap = cnt * (2 if symmetrize else 1)
+    nb = capi.lib().tg_csr_from_triples_workspace_bytes(cnt, m, int(symmetrize))
+    ws = torch.empty(nb, dtype=torch.uint8, device=cuda)
+    for rpt, tt in ((capi.I64, torch.int64), (capi.I32, torch.int32)):
+        rp = torch.full((m + 2,), -7, dtype=tt, device=cuda)
+        ci = torch.full((cap + 1,), -7, dtype=torch.int32, device=cuda)
+        va = torch.full((cap + 1,), -7.0, dtype=dV.dtype, device=cuda)
+        nnz = ctypes.c_int64(0)
+        capi.call("tg_csr_from_triples", cnt, dI.data_ptr(), dJ.data_ptr(), dV.data_ptr() if dtype else None,
+                  capi.F32 if dtype == np.float32 else capi.F64, m, n, int(compress), int(symmetrize), rp.data_ptr(),
+                  rpt, ci.data_ptr(), va.data_ptr(), cap, ws.data_ptr(), nb, ctypes.byref(nnz), None)
+        k = nnz.value
+        assert k == len(oci) and np.array_equal(rp[:-1].cpu().numpy(), orp) and rp[-1].item() == -7
+        assert np.array_equal(ci[:k].cpu().numpy(), oci) and ci[cap].item() == -7
+        if dtype:
+            assert np.array_equal(va[:k].cpu().numpy(), oval) and va[cap].item() == -7.0
+
+
+def test_from_triples_rejects_out_of_range_in_buckets(cuda):
+    rng = np.random.default_rng(3)
+    for bad in (-1, 3000):
+        I, J = rng.integers(0, 3000, 9000).astype(np.int32), rng.integers(0, 3000, 9000).astype(np.int32)
+        I[4321] = bad
+        with pytest.raises(TensorsError):
+            st.from_triples(I, J, np.ones(9000), 3000, 3000)
 
 
 def test_from_triples_rejects_out_of_range(cuda):

@@ -42,6 +42,9 @@
 //            them (Hc, H, cs, sn, the carried right-hand side beta, G, the state)
 //            into arrays no workgroup reads in the same launch; then q_j =
 //            (u - Q a) / rho and the next vector (v - Q t) / rho on the tile's rows.
+// Systems of one right-hand side and m <= 32 take the same two launches in the form of
+// the single-system solver's one-column step (gb_one_dots / gb_one_update, onecol.hpp);
+// a step launches each pair only where the batch holds such systems.
 // Every workgroup of a system sums that system's tile partials itself, in one
 // fixed order, so all of them see bitwise the same scalars, and no workgroup
 // reads what another writes in the same launch.  A system's arithmetic depends
@@ -57,6 +60,7 @@
 
 #include "common.hpp"
 #include "krylov.hpp"
+#include "onecol.hpp"
 
 namespace tg {
 
@@ -86,6 +90,7 @@ struct GbSys {
     int n, k, kpad, tiles, tile_rows, m;
     int big;       // more than g_gb_big_tiles tiles: the totals come from gb_totals_kernel
     int delayed;   // delayed second pass (p1 holds 2m + 2 values per tile, beta the carried rhs)
+    int one;       // delayed, one column, m <= kDdMaxM: the gb_one_* kernels take its steps
 };
 
 struct GbState {
@@ -484,7 +489,7 @@ __global__ __launch_bounds__(kBlock, 2) void gb_dstep1_kernel(const GbTile* __re
                                                            const GbSys* __restrict__ sys,
                                                            const GbState* __restrict__ st, int j) {
     GB_TILE_PROLOGUE
-    if (s->done || !s->active || j > S.m) return;
+    if (S.one || s->done || !s->active || j > S.m) return;
     const bool fin = j == S.m;
     const int64_t N = (int64_t)S.n * k;
     const double* __restrict__ U = S.Q + j * N;
@@ -527,7 +532,7 @@ __global__ __launch_bounds__(kBlock) void gb_dstep2_kernel(const GbTile* __restr
                                                            const GbSys* __restrict__ sys, GbState* __restrict__ st,
                                                            int j) {
     GB_TILE_PROLOGUE
-    if (s->done || !s->active || j > S.m) return;
+    if (S.one || s->done || !s->active || j > S.m) return;
     const int m = S.m, nv = 2 * j + 2, jj = j - 1;
     const bool fin = j == m;
     const int64_t N = (int64_t)S.n * k;
@@ -664,6 +669,147 @@ __global__ __launch_bounds__(kBlock) void gb_dstep2_kernel(const GbTile* __restr
     }
 }
 
+// dstep1 / dstep2 of one-column systems: the basis vectors dealt over the waves, the
+// product through LDS (one_dots_rows), and in the second kernel only the coefficients of
+// the vectors in every workgroup; tile 0 does the scalars (one_scalar_core) after its rows.
+// A system that stops here gets a q_j and a next vector it does not need: the other tiles
+// do not know.  Each reads its basis vectors once; what bounds them is the chain of memory
+// round trips in a tile (the product's entries, u at the columns, the vectors, the totals) more
+// than the bytes, which lie in the Infinity Cache: 64 systems of 50^2..150^2 (6e5 rows),
+// 17 to 30 vectors: 34 + 17 us a step (dstep1 and dstep2 before: 43 + 43).
+// 512 threads per workgroup take a tile's 1024 rows in two sub-tiles.  Of 256 and 1024,
+// cycles of the 64 systems: 47.2 ms / 45.9 / 49.3 (one workgroup of 1024 per CU has
+// nothing to run while it waits); of 8 systems 12.5 / 10.9 / 10.9, where tiles are few.
+constexpr int kOneDotsBlock = 512;
+
+template <int NB>
+__global__ __launch_bounds__(kOneDotsBlock, 4) void gb_one_dots_kernel(const GbTile* __restrict__ tiles,
+                                                                       const GbSys* __restrict__ sys,
+                                                                       const GbState* __restrict__ st, int j) {
+    const GbTile T = tiles[blockIdx.x];
+    const GbSys S = sys[T.slot];
+    const GbState* __restrict__ s = st + T.slot;
+    if (!S.one || s->done || !s->active || j > S.m) return;
+    constexpr int R = 2 * NB + 2, VB = NB > 4 ? 4 : NB, GROUPS = kOneDotsBlock / kOneRows, W = 2 * kDdMaxM + 2;
+    __shared__ OneDotsLds<double, int32_t, kOneDotsBlock, true> lds;
+    __shared__ double sums[GROUPS * W];
+    double acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.0;
+    const int fin = j == S.m ? 1 : 0;
+    for (int r0 = T.r0; r0 < T.r1; r0 += kOneDotsBlock)
+        one_dots_rows<double, int32_t, NB, VB, kOneDotsBlock, true>(
+            r0, min(kOneDotsBlock, T.r1 - r0), j, fin, S.rp, S.ci, S.val, S.d, nullptr, S.Q, S.n, nullptr,
+            S.Q + (int64_t)(j + 1 - fin) * S.n, lds, acc);
+    wave_sums<R>(acc, [&](int r) { return one_place<NB>(r, j); }, sums + threadIdx.x / kOneRows * W);
+    __syncthreads();
+    double* out = S.p1 + (int64_t)T.t * (2 * S.m + 2);
+    for (int i = threadIdx.x; i < 2 * j + 2; i += kOneDotsBlock) {
+        double v = sums[i];
+#pragma unroll
+        for (int g = 1; g < GROUPS; ++g) v += sums[g * W + i];
+        out[i] = v;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void gb_one_update_kernel(const GbTile* __restrict__ tiles,
+                                                               const GbSys* __restrict__ sys,
+                                                               GbState* __restrict__ st, int j) {
+    const GbTile T = tiles[blockIdx.x];
+    const GbSys S = sys[T.slot];
+    const GbState* __restrict__ s = st + T.slot;
+    if (!S.one || s->done || !s->active || j > S.m) return;
+    const int m = S.m, nv = 2 * j + 2, jj = j - 1;
+    const bool fin = j == m;
+    if (fin && T.t != 0) return;
+    constexpr int RQ = kGbTileRows / kBlock, VB = 8;  // rows per thread, vectors in flight
+    __shared__ OneScalarLds lds;
+    __shared__ double tv[(2 * kDdMaxM + 2) * kGbMaxK], sh[kBlock], ca[kDdMaxM], ce[kDdMaxM];
+    const int64_t N = S.n;
+    double* U = S.Q + j * N + T.r0;
+    double* V = S.Q + (j + 1) * N + T.r0;
+    unsigned row[RQ];  // within the tile, clamped
+    double uv[RQ], vv[RQ], qv[VB][RQ];
+    auto load_q = [&](int i0) {
+#pragma unroll
+        for (int b = 0; b < VB; ++b) {
+            const double* qb = S.Q + (int64_t)max(0, min(i0 + b, j - 1)) * N + T.r0;
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) qv[b][q] = qb[row[q]];
+        }
+    };
+    if (!fin) {  // the first loads are on their way during the totals
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            row[q] = (unsigned)min((int)threadIdx.x + q * kBlock, T.r1 - T.r0 - 1);
+            uv[q] = U[row[q]];
+            vv[q] = V[row[q]];
+        }
+        load_q(0);
+    }
+    if (T.t == 0) {
+        for (int t = threadIdx.x; t < j * (j + 1); t += kBlock) {
+            const int r = t / j, c = t % j;
+            lds.hm[r * kOneW + c] = c == jj ? (r < j ? S.G[(int64_t)r * m + jj] : 0.0)
+                                    : r <= c + 1 ? S.Hc[(int64_t)r * m + c] : 0.0;
+        }
+        for (int t = threadIdx.x; t < jj; t += kBlock) {
+            lds.rot[t] = S.cs[t];
+            lds.rot[kDdMaxM + t] = S.sn[t];
+        }
+    }
+    gb_totals(S, S.p1, 2 * m + 2, nv, tv, sh);
+    for (int i = threadIdx.x; i < nv; i += kBlock) lds.sv[i] = tv[i * kGbMaxK];
+    __syncthreads();
+    if (!fin) {
+        double ir, cj;
+        one_coefs<double>(j, lds.sv, ca, ce, ir, cj);
+        double qo[RQ], no[RQ];
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            qo[q] = uv[q] * ir;
+            no[q] = vv[q] * ir - cj * uv[q];
+        }
+        for (int i0 = 0; i0 < j; i0 += VB) {
+            if (i0 > 0) load_q(i0);
+#pragma unroll
+            for (int b = 0; b < VB; ++b)
+                if (i0 + b < j) {
+                    const double cai = ca[i0 + b], cei = ce[i0 + b];
+#pragma unroll
+                    for (int q = 0; q < RQ; ++q) {
+                        qo[q] -= cai * qv[b][q];
+                        no[q] -= cei * qv[b][q];
+                    }
+                }
+        }
+#pragma unroll
+        for (int q = 0; q < RQ; ++q)
+            if ((int)threadIdx.x + q * kBlock < T.r1 - T.r0) {
+                if (j > 0) U[row[q]] = qo[q];
+                V[row[q]] = no[q];
+            }
+    }
+    if (T.t != 0) return;
+    // beta holds the carried right-hand side; column j - 1 goes to Hc and H, column j to G
+    one_scalar_core(j, fin ? 1 : 0, S.beta + (jj < 0 ? 0 : jj), s->TOL, lds);
+    const bool stop = fin || (j > 0 && lds.conv);
+    if (j > 0 && (int)threadIdx.x <= j) {
+        S.Hc[(int64_t)threadIdx.x * m + jj] = lds.hm[threadIdx.x * kOneW + jj];
+        S.H[(int64_t)threadIdx.x * m + jj] = lds.col[threadIdx.x];
+    }
+    if (!stop && (int)threadIdx.x <= j) S.G[(int64_t)threadIdx.x * m + j] = lds.g[threadIdx.x];
+    if (j > 0 && threadIdx.x == 0) {
+        S.cs[jj] = lds.co;
+        S.sn[jj] = lds.si;
+        S.beta[j] = lds.carry;
+        GbState& w = st[T.slot];
+        w.iters = j;
+        w.conv = lds.conv;
+        if (stop) w.active = 0;
+    }
+}
+
 // Totals of one reduction of each big system, one workgroup per system (grid: the
 // big active systems): phase 0 after start1 (|Q_0|^2), 1 after step1 (first-pass
 // dots), 2 after the first step23 (second-pass dots), 3 after the second (|q|^2),
@@ -699,7 +845,7 @@ __global__ __launch_bounds__(kBlock) void gb_lsq_kernel(const GbTile* __restrict
     if (s->done || s->iters == 0) return;
     const int it = s->iters, m = S.m, k = S.k;
     // the triangle of H and the right-hand side staged in LDS (chunks of columns), then
-    // the serial substitution per column from LDS; plain row-oriented order
+    // the substitution from LDS, column by column of the triangle
     constexpr int kTri = 6144;
     __shared__ double tri[kTri];
     __shared__ double sb[(kGbMaxM + 1) * kGbMaxK];
@@ -718,12 +864,19 @@ __global__ __launch_bounds__(kBlock) void gb_lsq_kernel(const GbTile* __restrict
             sb[i * kGbMaxK + t % nc] = S.delayed ? S.cs[i * k + c] * S.beta[i * k + c] : S.beta[i * k + c];
         }
         __syncthreads();
-        for (int cc = threadIdx.x; cc < nc; cc += blockDim.x)
+        // a wave per column, a lane per row: y_i, then every lane above takes t_li y_i off
+        const int lane = threadIdx.x % kWave;
+        for (int cc = threadIdx.x / kWave; cc < nc; cc += kBlock / kWave) {
+            double v = lane < it ? sb[lane * kGbMaxK + cc] : 0.0;
+            const double diag = lane < it ? tri[tix(lane, lane) * nc + cc] : 1.0;
             for (int i = it - 1; i >= 0; --i) {
-                double v = sb[i * kGbMaxK + cc];
-                for (int jj = i + 1; jj < it; ++jj) v -= tri[tix(i, jj) * nc + cc] * sb[jj * kGbMaxK + cc];
-                sb[i * kGbMaxK + cc] = v / tri[tix(i, i) * nc + cc];
+                const double t = lane < i ? tri[tix(lane, i) * nc + cc] : 0.0;
+                const double y = __shfl(v, i, kWave) / __shfl(diag, i, kWave);
+                if (lane < i) v -= t * y;
+                if (lane == i) v = y;
             }
+            if (lane < it) sb[lane * kGbMaxK + cc] = v;
+        }
         __syncthreads();
         for (int t = threadIdx.x; t < it * nc; t += blockDim.x) S.y[(t / nc) * k + c0 + t % nc] = sb[(t / nc) * kGbMaxK + t % nc];
         __syncthreads();
@@ -743,7 +896,19 @@ __global__ __launch_bounds__(kBlock) void gb_update_kernel(const GbTile* __restr
         for (int row = T.r0 + ro; row < T.r1; row += rows) {
             const int64_t e = (int64_t)row * k + c;
             double z = 0.0;
-            for (int jj = 0; jj < it; ++jj) z += S.y[jj * k + c] * S.Q[jj * N + e];
+            constexpr int U = 8;  // vectors in flight (clamped to a valid one)
+            for (int j0 = 0; j0 < it; j0 += U) {
+                double q[U], y[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int jj = min(j0 + u, it - 1);
+                    q[u] = S.Q[jj * N + e];
+                    y[u] = S.y[jj * k + c];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (j0 + u < it) z += y[u] * q[u];
+            }
             S.x[e] = zero ? -z : S.x[e] - z;
         }
 }
@@ -871,6 +1036,7 @@ class GmresBatch {
         S.Hc = take((size_t)(m + 1) * m * k * 8);
         S.big = S.tiles > g_gb_big_tiles ? 1 : 0;
         S.delayed = delayed_;
+        S.one = delayed_ && k == 1 && m <= kDdMaxM ? 1 : 0;
         mem_[slot] = mem;
         bytes_[slot] = bytes;
         used_[slot] = 1;
@@ -898,7 +1064,7 @@ class GmresBatch {
             if (rc) return rc;
         }
         if (ntiles_ == 0) return TG_OK;
-        const GraphKey key{dtiles_, dsys_, dst_, dbig_, ntiles_, nbig_, mmax_, cycles};
+        const GraphKey key{dtiles_, dsys_, dst_, dbig_, ntiles_, nbig_, none_, nwide_, mmax_, cycles};
         if (!gexec_ || !(key == gkey_)) {
             if (gexec_) (void)hipGraphExecDestroy(gexec_);
             gexec_ = nullptr;
@@ -963,10 +1129,26 @@ class GmresBatch {
         hipLaunchKernelGGL(gb_start2_kernel, g, b, 0, s, dtiles_, dsys_, dst_);
         // delayed form: steps 0 .. m (m: the finishing step), two launches each
         for (int j = 0; delayed_ && j <= mmax_; ++j) {
-#define TG_GB_DSTEPS(NQ)                                                                     \
-    hipLaunchKernelGGL((gb_dstep1_kernel<NQ>), g, b, 0, s, dtiles_, dsys_, dst_, j);       \
-    totals(4, j);                                                                          \
-    hipLaunchKernelGGL((gb_dstep2_kernel<NQ>), g, b, 0, s, dtiles_, dsys_, dst_, j);
+            // one-column systems and the others, each where there are any
+#define TG_GB_ONE(NB)                                                                              \
+    hipLaunchKernelGGL((gb_one_dots_kernel<NB>), g, dim3(kOneDotsBlock), 0, s, dtiles_, dsys_,     \
+                       (const GbState*)dst_, j)
+            if (none_ > 0 && j <= kDdMaxM) {
+                if (j <= kOneVecs) {
+                    TG_GB_ONE(1);
+                } else if (j <= 2 * kOneVecs) {
+                    TG_GB_ONE(2);
+                } else if (j <= 4 * kOneVecs) {
+                    TG_GB_ONE(4);
+                } else {
+                    TG_GB_ONE(8);
+                }
+            }
+#undef TG_GB_ONE
+#define TG_GB_DSTEPS(NQ)                                                                       \
+    if (nwide_ > 0) hipLaunchKernelGGL((gb_dstep1_kernel<NQ>), g, b, 0, s, dtiles_, dsys_, dst_, j); \
+    totals(4, j);                                                                              \
+    if (nwide_ > 0) hipLaunchKernelGGL((gb_dstep2_kernel<NQ>), g, b, 0, s, dtiles_, dsys_, dst_, j);
             if (j <= 4) {
                 TG_GB_DSTEPS(4)
             } else if (j <= 8) {
@@ -979,6 +1161,8 @@ class GmresBatch {
                 TG_GB_DSTEPS(64)
             }
 #undef TG_GB_DSTEPS
+            if (none_ > 0 && j <= kDdMaxM)
+                hipLaunchKernelGGL(gb_one_update_kernel, g, b, 0, s, dtiles_, dsys_, dst_, j);
         }
         for (int j = 0; !delayed_ && j < mmax_; ++j) {
             const int nq = j + 1;
@@ -1038,7 +1222,7 @@ class GmresBatch {
         if (rc) return rc;
         std::vector<GbTile> tl;
         std::vector<int> bl;  // big active systems
-        int mmax = 0;
+        int mmax = 0, none = 0, nwide = 0;
         for (int i = 0; i < (int)used_.size(); ++i)
             if (used_[i] && !states[i].done) {
                 const GbSys& S = host_[i];
@@ -1046,6 +1230,7 @@ class GmresBatch {
                     tl.push_back(GbTile{i, t * S.tile_rows, std::min(S.n, (t + 1) * S.tile_rows), t});
                 if (S.big) bl.push_back(i);
                 mmax = std::max(mmax, S.m);
+                (S.one ? none : nwide) += 1;
             }
         if (tl.size() > tiles_cap_) {
             if (dtiles_) TG_HIP(hipFreeAsync(dtiles_, s_));
@@ -1064,6 +1249,8 @@ class GmresBatch {
         ntiles_ = (int)tl.size();
         nbig_ = (int)bl.size();
         mmax_ = mmax;
+        none_ = none;
+        nwide_ = nwide;
         dirty_ = false;
         return TG_OK;
     }
@@ -1089,10 +1276,10 @@ class GmresBatch {
         const void* sys;
         const void* st;
         const void* big;
-        int ntiles, nbig, mmax, cycles;
+        int ntiles, nbig, none, nwide, mmax, cycles;
         bool operator==(const GraphKey& o) const {
             return tiles == o.tiles && sys == o.sys && st == o.st && big == o.big && ntiles == o.ntiles &&
-                   nbig == o.nbig && mmax == o.mmax && cycles == o.cycles;
+                   nbig == o.nbig && none == o.none && nwide == o.nwide && mmax == o.mmax && cycles == o.cycles;
         }
     };
     hipStream_t cap_s_ = nullptr;
@@ -1113,6 +1300,7 @@ class GmresBatch {
     int* dbig_ = nullptr;  // slots of the big active systems
     size_t big_cap_ = 0;
     int nbig_ = 0;
+    int none_ = 0, nwide_ = 0;  // active systems of the one-column steps, and the others
     int mmax_ = 0;
     bool dirty_ = true;
 };

@@ -34,6 +34,7 @@
 
 #include "common.hpp"
 #include "krylov.hpp"
+#include "onecol.hpp"
 
 namespace tg {
 
@@ -360,7 +361,6 @@ __global__ __launch_bounds__(kBlock) void gm_ddots_kernel(int n, int k, int kpad
 // The totals, column j - 1 of H and the rotations are staged in LDS; the per-column
 // serial part (|a|^2, a.b, the Givens chain) reads only LDS, everything else is
 // spread over (row, column) pairs.
-constexpr int kDdMaxM = 32;  // restart length limit of the delayed form
 __global__ __launch_bounds__(kBlock) void gm_dscalar_kernel(int j, int m, int k, int finish,
                                                             const double* __restrict__ tot, double* __restrict__ small,
                                                             GmresLayout L, GmresHdr* __restrict__ hd) {
@@ -551,25 +551,10 @@ __global__ __launch_bounds__(kBlock) void gm_dupdate_kernel(int n, int k, int kp
 // A stop is found in gm_one_update, whose other workgroups must not see it: it goes to
 // hd->pend, which the next gm_one_dots reads; that one's first workgroup sets hd->done.
 // ---------------------------------------------------------------------------
-constexpr int kOneVecs = 4;        // the waves that share a tile's rows
-constexpr int kOneRows = 256;      // rows of such a group of waves
 // Values of partials that every workgroup of the update adds itself (32 KB; 9e4 rows with up
 // to 8192: 31.9 -> 25.4 ms a solve, 19.5 so), above that a kernel does.
 constexpr int kDirectTotals = 4096;
 constexpr int kOneRowUpdate = 1 << 17;  // rows up to which the update takes one row per thread: 512 workgroups
-
-// Sums R values per lane over the wave and writes value r to out[at(r)] (at(r) < 0: none).
-template <int R, typename At>
-__device__ __forceinline__ void wave_sums(double (&v)[R], At at, double* out) {
-    const ScatterOut o = wave_scatter_sum<R>(v, 1);
-    if (threadIdx.x % o.low == 0)
-#pragma unroll
-        for (int i = 0; i < ScatterSizes<R>::A; ++i)
-            if (i < o.count) {
-                const int t = at(o.base + i);
-                if (t >= 0) out[t] = v[i];
-            }
-}
 
 template <typename T, typename RP, int NB, int TH, bool SPMV>
 __global__ __launch_bounds__(TH, TH == kOneRows ? 1 : 4) void gm_one_dots_kernel(int n, int j, int finish, const RP* __restrict__ rp,
@@ -578,154 +563,50 @@ __global__ __launch_bounds__(TH, TH == kOneRows ? 1 : 4) void gm_one_dots_kernel
                                                          const T* __restrict__ Q, int64_t qstride,
                                                          const T* __restrict__ z, T* __restrict__ vslot,
                                                          double* __restrict__ partial, GmresHdr* __restrict__ hd) {
-    constexpr int EL = 8;  // nonzeros per thread and chunk
-    constexpr int CAP = TH * EL;
-    constexpr int GROUPS = TH / kOneRows;
-    constexpr int RQ = kOneRows / kWave;        // rows per lane
-    constexpr int VB = NB > 4 && TH > kOneRows ? (sizeof(T) == 8 ? 2 : 4) : NB;  // vectors in flight
-    constexpr int R = 2 * NB + 2;
-    __shared__ T prod[SPMV ? CAP : 1];
-    __shared__ RP srp[SPMV ? TH + 1 : 1];
-    __shared__ T sv[TH], su[TH];
-    __shared__ double sums[GROUPS > 1 ? GROUPS * (2 * kDdMaxM + 2) : 1];
+    __shared__ OneDotsLds<T, RP, TH, SPMV> lds;
+    __shared__ double sums[TH > kOneRows ? TH / kOneRows * (2 * kDdMaxM + 2) : 1];
     if (hd->done) return;
     if (hd->pend) {
         if (blockIdx.x == 0 && threadIdx.x == 0) hd->done = 1;
         return;
     }
-    // wave ids in scalar registers: a basis vector's address is one scalar pair and a lane offset
-    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int w = wave % kOneVecs, grp = wave / kOneVecs;
+    // vectors in flight: all of a wave's, on their way during the product, where registers allow
+    constexpr int VB = NB > 4 && TH > kOneRows ? (sizeof(T) == 8 ? 2 : 4) : NB;
+    constexpr int R = 2 * NB + 2;
     const int B = gridDim.x, lb = xcd_swizzle(blockIdx.x, B);
     const int tiles = (n + TH - 1) / TH;
-    const T* U = Q + (int64_t)j * qstride;
     double acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.0;
-    for (int t = (int)((int64_t)tiles * lb / B); t < (int)((int64_t)tiles * (lb + 1) / B); ++t) {
-        const int base = t * TH, nr = min(TH, n - base);
-        const int row = base + min((int)threadIdx.x, nr - 1);
-        const T uown = U[row];
-        T qv[VB][RQ];
-        unsigned off[RQ];  // clamped rows
-#pragma unroll
-        for (int q = 0; q < RQ; ++q) off[q] = (unsigned)min(grp * kOneRows + lane + q * kWave, nr - 1);
-        auto load_q = [&](int b0) {  // at clamped vectors
-#pragma unroll
-            for (int b = 0; b < VB; ++b) {
-                const T* qb = Q + (int64_t)max(0, min(w + kOneVecs * (b0 + b), j - 1)) * qstride + base;
-#pragma unroll
-                for (int q = 0; q < RQ; ++q) qv[b][q] = qb[off[q]];
-            }
-        };
-        if constexpr (VB == NB) load_q(0);  // on their way during the product
-        T vown = uown;
-        if (SPMV && !finish) {
-            for (int i = threadIdx.x; i <= nr; i += TH) srp[i] = rp[base + i];
-            __syncthreads();
-            const RP l0 = srp[0], l1 = srp[nr];
-            T sum = T(0);
-            const RP rb = threadIdx.x < nr ? srp[threadIdx.x] : l0, re = threadIdx.x < nr ? srp[threadIdx.x + 1] : l0;
-            for (RP cs = l0; cs < l1; cs += CAP) {
-                const int cnt = (int)((l1 - cs) < (RP)CAP ? (l1 - cs) : (RP)CAP);
-                int32_t c[EL];
-                T av[EL], xv[EL];
-#pragma unroll
-                for (int e = 0; e < EL; ++e) {  // clamped to the chunk's last nonzero
-                    const RP at = cs + min((int)threadIdx.x + e * TH, cnt - 1);
-                    c[e] = __builtin_nontemporal_load(ci + at);
-                    av[e] = a ? __builtin_nontemporal_load(a + at) : T(1);
-                }
-#pragma unroll
-                for (int e = 0; e < EL; ++e) xv[e] = dr ? dr[c[e]] * U[c[e]] : U[c[e]];
-#pragma unroll
-                for (int e = 0; e < EL; ++e) {
-                    const int at = threadIdx.x + e * TH;
-                    if (at < cnt) prod[at] = av[e] * xv[e];
-                }
-                __syncthreads();
-                const int b0 = (int)((rb > cs ? rb : cs) - cs), b1 = (int)((re < cs + cnt ? re : cs + cnt) - cs);
-                for (int l = b0; l < b1; ++l) sum += prod[l];
-                __syncthreads();
-            }
-            vown = dl ? dl[row] * sum : sum;
-            if (threadIdx.x < nr) vslot[row] = vown;
-        } else if (!finish) {
-            if (dl) {
-                vown = dl[row] * z[row];
-                if (threadIdx.x < nr) vslot[row] = vown;
-            } else {
-                vown = vslot[row];
-            }
-        }
-        su[threadIdx.x] = threadIdx.x < nr ? uown : T(0);
-        sv[threadIdx.x] = threadIdx.x < nr ? vown : T(0);
-        __syncthreads();
-        T uv[RQ], vv[RQ];
-#pragma unroll
-        for (int q = 0; q < RQ; ++q) {
-            uv[q] = su[grp * kOneRows + lane + q * kWave];
-            vv[q] = sv[grp * kOneRows + lane + q * kWave];
-        }
-#pragma unroll
-        for (int b0 = 0; b0 < NB; b0 += VB) {
-            if constexpr (VB != NB) load_q(b0);
-#pragma unroll
-            for (int b = 0; b < VB; ++b)
-#pragma unroll
-                for (int q = 0; q < RQ; ++q) {
-                    acc[b0 + b] += (double)qv[b][q] * (double)uv[q];
-                    acc[NB + b0 + b] += (double)qv[b][q] * (double)vv[q];
-                }
-        }
-        if (w == kOneVecs - 1)
-#pragma unroll
-            for (int q = 0; q < RQ; ++q) {
-                acc[2 * NB] += (double)uv[q] * (double)uv[q];
-                acc[2 * NB + 1] += (double)uv[q] * (double)vv[q];
-            }
-        __syncthreads();
-    }
+    for (int t = (int)((int64_t)tiles * lb / B); t < (int)((int64_t)tiles * (lb + 1) / B); ++t)
+        one_dots_rows<T, RP, NB, VB, TH, SPMV>(t * TH, min(TH, n - t * TH), j, finish, rp, ci, a, dl, dr, Q, qstride, z,
+                                               vslot, lds, acc);
     const int nv = 2 * j + 2;
-    auto at = [&](int r) {  // place of register r among the 2j + 2 values
-        if (r >= 2 * NB) return w == kOneVecs - 1 ? 2 * j + (r - 2 * NB) : -1;
-        const int i = w + kOneVecs * (r < NB ? r : r - NB);
-        return i < j ? (r < NB ? i : j + i) : -1;
-    };
     double* out = partial + (int64_t)lb * nv;
-    if constexpr (GROUPS == 1) {
+    auto at = [&](int r) { return one_place<NB>(r, j); };
+    if constexpr (TH == kOneRows) {
         wave_sums<R>(acc, at, out);
     } else {
-        wave_sums<R>(acc, at, sums + grp * (2 * kDdMaxM + 2));
+        wave_sums<R>(acc, at, sums + threadIdx.x / kOneRows * (2 * kDdMaxM + 2));
         __syncthreads();
         for (int i = threadIdx.x; i < nv; i += TH) {
             double s = 0.0;
 #pragma unroll
-            for (int g = 0; g < GROUPS; ++g) s += sums[g * (2 * kDdMaxM + 2) + i];
+            for (int g = 0; g < TH / kOneRows; ++g) s += sums[g * (2 * kDdMaxM + 2) + i];
             out[i] = s;
         }
     }
 }
 
-struct OneScalarLds {
-    double sv[2 * kDdMaxM + 2];                  // the totals
-    double hm[(kDdMaxM + 1) * (kDdMaxM + 1)];    // Hraw, rows 0..j, columns 0..j-1
-    double rot[2 * kDdMaxM];                     // cs, sn of rotations 0..j-2
-    double col[kDdMaxM + 1];                     // column j - 1, rotated
-    double g[kDdMaxM + 1];                       // column j, first pass
-    int conv;
-};
-
 // What gm_dscalar_kernel does, for one column, by a workgroup of kBlock threads.  `stage`
-// runs before the totals are known (its loads are in flight with theirs), `finish_step`
-// after lds.sv holds them and the workgroup has synchronised; it returns whether the cycle
-// stops here.  Wave 0 rotates column j - 1 while the others form column j.
+// runs before the totals are known (its loads are in flight with theirs), the step after
+// lds.sv holds them and the workgroup has synchronised; it returns whether the cycle stops
+// here.
 __device__ __forceinline__ void one_scalar_stage(int j, int m, const double* __restrict__ small, const GmresLayout& L,
                                                  OneScalarLds& lds) {
-    constexpr int W = kDdMaxM + 1;
     for (int t = threadIdx.x; t < j * (j + 1); t += kBlock) {
         const int r = t / j, c = t % j;
-        lds.hm[r * W + c] = r <= c + 1 ? small[L.Hraw + (int64_t)r * m + c] : 0.0;
+        lds.hm[r * kOneW + c] = r <= c + 1 ? small[L.Hraw + (int64_t)r * m + c] : 0.0;
     }
     for (int t = threadIdx.x; t < j - 1; t += kBlock) {
         lds.rot[t] = small[L.cs + t];
@@ -736,79 +617,21 @@ __device__ __forceinline__ void one_scalar_stage(int j, int m, const double* __r
 __device__ __forceinline__ bool one_scalar_step(int j, int m, int finish, double* __restrict__ small,
                                                 const GmresLayout& L, const GmresHdr* __restrict__ hd,
                                                 OneScalarLds& lds) {
-    constexpr int W = kDdMaxM + 1;
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave, jj = j - 1;
+    const int jj = j - 1;
     double* H = small + L.H;
     double* Hr = small + L.Hraw;
-    // |a|^2 and a.b, by every wave alike
-    double aa = 0.0, ab = 0.0;
-    const double alane = lane < j ? lds.sv[lane] : 0.0;
-    if (lane < j) {
-        aa = alane * alane;
-        ab = alane * lds.sv[j + lane];
-    }
-    aa = group_sum<kWave>(aa);
-    ab = group_sum<kWave>(ab);
-    const double alpha = lds.sv[2 * j], beta = lds.sv[2 * j + 1];
-    // |u - Q a|; at a breakdown (u in the span of Q to rounding) at least 2^-52 |u|
-    const double rho = j > 0 ? sqrt(fmax(alpha - aa, 0x1p-104 * alpha)) : 1.0;
-    const double irho = 1.0 / rho;
-    if (j > 0) {
-        // column jj completed: its second pass and |u - Q a|
-        if (wave == 0 && lane <= j) {
-            const double v = lane < j ? lds.hm[lane * W + jj] + alane : rho;
-            lds.hm[lane * W + jj] = v;
-            lds.col[lane] = v;
-            Hr[(int64_t)lane * m + jj] = v;
-        }
-        __syncthreads();
-    }
-    if (wave == 0) {
-        if (lane == 0 && j > 0) {
-            // Givens on column jj (GMRES.hpp:603-658)
-            const double bj = small[L.beta + jj], lim = small[L.TOL];
-            double xi = lds.col[0];
-#pragma unroll 4
-            for (int i = 0; i < jj; ++i) {
-                const double eta = lds.col[i + 1], co = lds.rot[i], si = lds.rot[kDdMaxM + i];
-                lds.col[i] = co * xi + si * eta;
-                xi = -si * xi + co * eta;
-            }
-            const double eta = lds.col[j];
-            const double r = sqrt(xi * xi + eta * eta);
-            double co, si;
-            if (fabs(xi) <= 2.220446049250313e-16 * r) {
-                co = 0.0;
-                si = 1.0;
-            } else {
-                const double rinv = 1.0 / r;
-                co = fabs(xi) * rinv;
-                si = (xi / fabs(xi)) * eta * rinv;
-            }
-            lds.col[jj] = co * xi + si * eta;
-            lds.col[j] = 0.0;
-            small[L.cs + jj] = co;
-            small[L.sn + jj] = si;
-            small[L.beta + j] = -si * bj;
-            small[L.beta + jj] = co * bj;
-            lds.conv = fabs(-si * bj) <= lim ? 1 : 0;
-        }
-        if (lane == 0 && j == 0) lds.conv = 0;
-    } else if (!finish) {
-        // column j, first pass: g_l = (t_l - (Hraw a)_l) / rho, four lanes to a row
-        const double tj = j > 0 ? (beta - ab) * irho : beta;
-        const int t = threadIdx.x - kWave, part = t % 4;
-        for (int l = t / 4; l <= j; l += (kBlock - kWave) / 4) {
-            double ha = 0.0;
-            for (int i = part; i < j; i += 4) ha += lds.hm[l * W + i] * lds.sv[i];
-            ha += shfl_xor(ha, 1);
-            ha += shfl_xor(ha, 2);
-            if (part == 0) lds.g[l] = ((l < j ? lds.sv[j + l] : tj) - ha) * irho;
-        }
-    }
-    __syncthreads();
+    one_scalar_core(j, finish, small + L.beta + (jj < 0 ? 0 : jj), small + L.TOL, lds);
     const bool stop = j > 0 && (lds.conv || j >= hd->m);
-    if (j > 0 && threadIdx.x <= j) H[(int64_t)threadIdx.x * m + jj] = lds.col[threadIdx.x];
+    if (j > 0 && threadIdx.x <= j) {
+        Hr[(int64_t)threadIdx.x * m + jj] = lds.hm[threadIdx.x * kOneW + jj];
+        H[(int64_t)threadIdx.x * m + jj] = lds.col[threadIdx.x];
+    }
+    if (j > 0 && threadIdx.x == 0) {
+        small[L.cs + jj] = lds.co;
+        small[L.sn + jj] = lds.si;
+        small[L.beta + j] = lds.carry;
+        small[L.beta + jj] = lds.kept;
+    }
     if (!finish && !stop && threadIdx.x <= j) {
         Hr[(int64_t)threadIdx.x * m + j] = lds.g[threadIdx.x];
         H[(int64_t)threadIdx.x * m + j] = lds.g[threadIdx.x];
@@ -898,26 +721,8 @@ __global__ __launch_bounds__(kBlock) void gm_one_update_kernel(int n, int j, int
         }
         return;
     }
-    // rho and a.b as in one_scalar_step, by every wave alike
-    const int lane = threadIdx.x % kWave;
-    double aa = 0.0, ab = 0.0;
-    if (lane < j) {
-        const double ai = lds.sv[lane];
-        aa = ai * ai;
-        ab = ai * lds.sv[j + lane];
-    }
-    aa = group_sum<kWave>(aa);
-    ab = group_sum<kWave>(ab);
-    const double alpha = lds.sv[2 * j], beta = lds.sv[2 * j + 1];
-    const double irho = j > 0 ? 1.0 / sqrt(fmax(alpha - aa, 0x1p-104 * alpha)) : 1.0;
-    const double tj = j > 0 ? (beta - ab) * irho : beta;
-    const double cjd = tj * irho * irho;
-    if (threadIdx.x < j) {
-        ca[threadIdx.x] = (T)(lds.sv[threadIdx.x] * irho);
-        ce[threadIdx.x] = (T)(lds.sv[j + threadIdx.x] * irho - cjd * lds.sv[threadIdx.x]);
-    }
-    __syncthreads();
-    const T ir = (T)irho, cj = (T)cjd;
+    T ir, cj;
+    one_coefs<T>(j, lds.sv, ca, ce, ir, cj);
     T qo[RQ], no[RQ];
 #pragma unroll
     for (int q = 0; q < RQ; ++q) {

@@ -188,3 +188,36 @@ def test_batch_gmres_big_system_totals_are_bitwise_neutral(cuda, big_tiles_knob)
     B = sysl[-1][4]
     assert rl["succeeded"]
     assert np.max(np.linalg.norm(B - A @ Xl, axis=0) / np.linalg.norm(B, axis=0)) <= 1.5e-9
+
+
+@pytest.mark.parametrize("n,m", [(7, 4), (255, 5), (256, 8), (511, 9), (513, 16), (1023, 17), (1025, 32), (2049, 31),
+                                 (1025, 33)])
+def test_batch_gmres_one_column_shapes(cuda, n, m):
+    """One-column systems (their own step kernels up to m = 32) at the edges of the tiles and of
+    the dealing of vectors to waves, with empty rows of W and a row longer than what is staged,
+    with and without a diagonal, next to a wider system and a longer cycle: two cycles against
+    the oracle, and bitwise what the system gives alone.  A = 2 I + W with ||W||_2 <= 1 has a
+    condition number of at most 3, so the solution carries the rounding of the cycles (about
+    sqrt(n) eps a step, 33 steps: 4e-13) and no more; later vectors of a cycle that has
+    reached rounding are noise, so the solution is what is compared."""
+    rng = np.random.default_rng(n * 100 + m)
+    cnt = 5 * n
+    i, j = rng.integers(0, n, cnt), rng.integers(0, n, cnt)
+    if n > 1000:
+        i[:3000] = n // 3
+    W = sp.coo_matrix((rng.uniform(-1, 1, cnt), (i, j)), shape=(n, n)).tocsr()
+    r, c = (np.asarray(abs(W).sum(a)).ravel() for a in (1, 0))
+    W = sp.diags(1.0 / np.sqrt(np.maximum(r, 1e-3))) @ W @ sp.diags(1.0 / np.sqrt(np.maximum(c, 1e-3)))
+    A = (W + 2.0 * sp.identity(n)).tocsr()
+    A.sort_indices()
+    csr = (A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data)
+    d = rng.uniform(0.9, 1.1, n) if n % 2 else None
+    B = gen.uniform(7 * n + m, 4 * n).reshape(n, 4)
+    sysl = [(*csr, d, B[:, :1], n, 1, m), (*csr, d, B[:, 1:], n, 3, min(m, 7)), (*csr, None, B[:, :1], n, 1, min(n, 40))]
+    X, res = run(sysl, cuda, 0.0, 1)
+    for i, (rp, ci, val, dd, b, _, k, mm) in enumerate(sysl):
+        Xo = np.zeros((n, k))
+        oracle.gmres(n, rp, ci, val, np.ascontiguousarray(b), Xo, k, mm, 0.0, 1, prec_diag=dd)
+        assert res[i]["finished"] and rel_err(X[i], Xo) <= 1e-12, i
+    alone, ra = run(sysl[:1], cuda, 0.0, 1)
+    assert np.array_equal(alone[0], X[0]) and np.array_equal(ra[0]["rel_res"], res[0]["rel_res"])

@@ -38,7 +38,8 @@
 namespace tg {
 
 constexpr int kBatchMaxK = 8;
-constexpr int kTileRows = 1024;  // default rows per tile (tg_tune_set "batch_tile_rows")
+constexpr int kTileRows = 1024;  // default rows per tile (tg_tune_set "batch_tile_rows"); 256 / 512 / 1024 rows,
+                                 // 64 mixed systems: 209 / 154 / 147 ms (the partials to add grow)
 constexpr int kMinTileRows = 256;
 static int g_batch_tile_rows = kTileRows;
 static int g_batch_stream = 0;  // SpMM kernel of the engine: 0 = a row per lane (measured faster), 1 = streaming chunks
@@ -74,6 +75,7 @@ template <typename T> struct SysDev {
     double* prz[2];  // tiles * k partials of r.z, by parity
     int* xit;        // per tile: the iteration whose deferred x update the tile has applied
     int n, k, kpad, tiles, tile_rows;
+    int vec, gs;      // columns per lane of the iteration's kernels, log2 of the lanes per row
     int check_every;  // > 0: pause at every multiple of this many iterations for the host
 };
 
@@ -137,6 +139,150 @@ __device__ __forceinline__ double sys_total(const double* partial, int tiles, in
     const double v = sh[c];
     __syncthreads();
     return v;
+}
+
+// Totals of NT partial arrays of a system at once (tot[a * kBatchMaxK + c], for every thread
+// after the call): each column over the lanes of a wave by shuffles, then over the waves, in
+// one fixed order.  sh: NT * kWaves * kBatchMaxK doubles.  The totals stand at the front of
+// every direction and update pass, where nothing else can run: two barriers for all of
+// them, against nine to eleven for each with sys_total.
+constexpr int kWaves = kBlock / kWave;
+template <int NT>
+__device__ __forceinline__ void sys_totals(const double* const (&part)[NT], int tiles, int k, int kpad, double* sh,
+                                           double* tot) {
+    const int c = threadIdx.x & (kpad - 1), j = threadIdx.x / kpad, J = kBlock / kpad;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    double s[NT];
+#pragma unroll
+    for (int a = 0; a < NT; ++a) s[a] = 0.0;
+    constexpr int U = 2;  // tiles of a lane in flight (clamped to a valid one; 4 cost the registers of a wave)
+    if (c < k)
+        for (int t = j; t < tiles; t += U * J) {
+            double w[NT][U];
+#pragma unroll
+            for (int a = 0; a < NT; ++a)
+#pragma unroll
+                for (int q = 0; q < U; ++q)
+                    w[a][q] = ((gptr<const double>)part[a])[(int64_t)min(t + q * J, tiles - 1) * k + c];
+#pragma unroll
+            for (int q = 0; q < U; ++q)
+                if (t + q * J < tiles) {
+#pragma unroll
+                    for (int a = 0; a < NT; ++a) s[a] += w[a][q];
+                }
+        }
+    for (int off = kWave / 2; off >= kpad; off >>= 1) {
+#pragma unroll
+        for (int a = 0; a < NT; ++a) s[a] += __shfl_xor(s[a], off, kWave);
+    }
+    if (lane < kpad) {
+#pragma unroll
+        for (int a = 0; a < NT; ++a) sh[(a * kWaves + wave) * kBatchMaxK + lane] = s[a];
+    }
+    __syncthreads();
+    if (threadIdx.x < NT * kBatchMaxK) {
+        const int a = threadIdx.x / kBatchMaxK, cc = threadIdx.x % kBatchMaxK;
+        double v = 0.0;
+        if (cc < k) {
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) v += sh[(a * kWaves + w) * kBatchMaxK + cc];
+        }
+        tot[threadIdx.x] = v;
+    }
+    __syncthreads();
+}
+
+// ---- the lanes of a row -------------------------------------------------------------
+// The iteration's kernels give a lane V neighbouring columns of a row (16 bytes where there
+// are that many; V the largest power of two up to min(k, 16 / sizeof(T))) and a row
+// ceil(k / V) lanes, rounded up to a power of two.  Where V does not divide k the last lane's
+// columns start at k - V: it loads columns of the lane before as well, but writes and
+// counts only its own.  Against a lane per column a tile of 8 FP32 columns takes 8 passes over
+// its workgroup in place of 32, with a quarter of the loads.  What bounds a launch: with many
+// tiles the bytes (2 039 tiles of 64 mixed systems of 1e3 to 2e5 rows and 1 to 8 columns,
+// FP32: direction 196 MB in 48 -> 44 us, product 160 MB in 64 -> 53, update 118 MB in
+// 30 us), with few the longest tile's passes (850 tiles: 19, 38, 14 -> 17, 21, 14 us; 182
+// tiles: 8.4, 14, 6.2 -> 6.2, 7.4, 4.3).  64 systems to 1e-8: 170 -> 147 ms.
+struct Cols {
+    int c0;   // first column loaded
+    int own;  // columns c0 + own ... c0 + V - 1 are this lane's (V: none, the lane is idle)
+    int ro, rows;
+};
+
+template <int V, typename T> __device__ __forceinline__ Cols cols_of(const SysDev<T>& S) {
+    const int c = ((int)threadIdx.x & ((1 << S.gs) - 1)) * V, c0 = min(c, S.k - V);
+    return Cols{c0, c < S.k ? c - c0 : V, (int)threadIdx.x >> S.gs, kBlock >> S.gs};
+}
+
+inline int lane_columns(int k, int most) {
+    int v = most;
+    while (v > k) v /= 2;
+    return v;
+}
+
+// f(the system's columns per lane as a constant)
+template <typename T, typename F> __device__ __forceinline__ void by_vec(int vec, F&& f) {
+    if constexpr (sizeof(T) == 4) {
+        if (vec == 4) {
+            f(std::integral_constant<int, 4>{});
+            return;
+        }
+    }
+    if (vec == 2)
+        f(std::integral_constant<int, 2>{});
+    else
+        f(std::integral_constant<int, 1>{});
+}
+
+template <typename T, int V> __device__ __forceinline__ void gload(gptr<const T> p, T (&out)[V]) {
+    if constexpr (V == 1) {
+        out[0] = *p;
+    } else {
+        using VT = typename VecAt<T, V>::type;
+        const VT v = *(gptr<const VT>)p;
+#pragma unroll
+        for (int i = 0; i < V; ++i) out[i] = v[i];
+    }
+}
+
+template <typename T, int V> __device__ __forceinline__ void gstore(gptr<T> p, const T (&in)[V], int own) {
+    if constexpr (V == 1) {
+        *p = in[0];
+    } else if (own == 0) {
+        using VT = typename VecAt<T, V>::type;
+        VT v;
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[i] = in[i];
+        *(gptr<VT>)p = v;
+    } else {
+#pragma unroll
+        for (int i = 1; i < V; ++i)
+            if (i >= own) p[i] = in[i];
+    }
+}
+
+// The tile's partial of every column, written to partial[t * k + c]: over the lanes of a wave
+// by shuffles, then over the waves.  sh: kWaves * kBatchMaxK doubles.  All threads call it.
+template <int V>
+__device__ __forceinline__ void tile_partial_cols(double (&acc)[V], const Cols& C, int gs, int k, double* partial, int t,
+                                                  double* sh) {
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    for (int off = kWave / 2; off >= (1 << gs); off >>= 1) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += __shfl_xor(acc[v], off, kWave);
+    }
+    if (lane < (1 << gs)) {
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (v >= C.own) sh[wave * kBatchMaxK + C.c0 + v] = acc[v];
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < k) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) s += sh[w * kBatchMaxK + threadIdx.x];
+        partial[(int64_t)t * k + threadIdx.x] = s;
+    }
 }
 
 // ---- setup: r = b, z = P r, x = 0, partial r.z (parity 0) -------------------------
@@ -353,9 +499,9 @@ __global__ __launch_bounds__(kBlock) void bk_delta16_kernel(int n, int64_t nnz, 
 // template arguments, so the compiler issues all loads of a chunk before the first
 // wait (branches inside the unrolled body split it into blocks that each wait for
 // their loads).  The sum runs in nonzero order.
-template <typename T, bool HAS_D, bool FIRST>
-__device__ __forceinline__ double k1_rows(const SysDev<T>& S, const Tile& tl, int c, int ro, int rows, T be,
-                                          const T* __restrict__ pold_, T* __restrict__ pnew_) {
+template <typename T, int V, bool HAS_D, bool FIRST>
+__device__ __forceinline__ void k1_rows(const SysDev<T>& S, const Tile& tl, const Cols& C, const T (&be)[V],
+                                        const T* __restrict__ pold_, T* __restrict__ pnew_, double (&acc)[V]) {
     // global-address-space views: the pointers come from a table in memory, so the
     // compiler cannot tell them from LDS pointers and would use flat accesses
     const gptr<const T> pold = (gptr<const T>)pold_;
@@ -367,13 +513,12 @@ __device__ __forceinline__ double k1_rows(const SysDev<T>& S, const Tile& tl, in
     const gptr<const T> val = (gptr<const T>)S.val;
     const gptr<T> u = (gptr<T>)S.u;
     const int k = S.k;
-    double acc = 0.0;
-    for (int i = tl.r0 + ro; i < tl.r1; i += rows) {
+    for (int i = tl.r0 + C.ro; i < tl.r1; i += C.rows) {
         const int lb = rp[i], le = rp[i + 1];
-        T sum = T(0);
+        T sum[V] = {};
         for (int l0 = lb; l0 < le; l0 += kGather) {
             int32_t jj[kGather];
-            T vv[kGather], pj[kGather];
+            T vv[kGather], pj[kGather][V];
 #pragma unroll
             for (int q = 0; q < kGather; ++q) {
                 const int lq = min(l0 + q, le - 1);
@@ -385,31 +530,50 @@ __device__ __forceinline__ double k1_rows(const SysDev<T>& S, const Tile& tl, in
             }
 #pragma unroll
             for (int q = 0; q < kGather; ++q) {
-                const int64_t f = (int64_t)jj[q] * k + c;
-                T zj = r[f];
-                if constexpr (HAS_D) zj = d[jj[q]] * zj;
-                if constexpr (FIRST)
-                    pj[q] = zj;
-                else
-                    pj[q] = fma_t(be, pold[f], zj);
+                const int64_t f = (int64_t)jj[q] * k + C.c0;
+                T zj[V];
+                gload<T, V>(r + f, zj);
+                if constexpr (HAS_D) {
+                    const T dj = d[jj[q]];
+#pragma unroll
+                    for (int v = 0; v < V; ++v) zj[v] = dj * zj[v];
+                }
+                if constexpr (!FIRST) gload<T, V>(pold + f, pj[q]);
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    if constexpr (FIRST)
+                        pj[q][v] = zj[v];
+                    else
+                        pj[q][v] = fma_t(be[v], pj[q][v], zj[v]);
+                }
             }
 #pragma unroll
-            for (int q = 0; q < kGather; ++q) sum += (l0 + q < le) ? vv[q] * pj[q] : T(0);
+            for (int q = 0; q < kGather; ++q) {
+#pragma unroll
+                for (int v = 0; v < V; ++v) sum[v] += (l0 + q < le) ? vv[q] * pj[q][v] : T(0);
+            }
         }
-        const int64_t e = (int64_t)i * k + c;
-        T zi = r[e];
-        if constexpr (HAS_D) zi = d[i] * zi;
-        T pi;
-        if constexpr (FIRST)
-            pi = zi;
-        else
-            pi = fma_t(be, pold[e], zi);
-        pnew[e] = pi;
-        u[e] = sum;
-        acc += (double)pi * (double)sum;
+        const int64_t e = (int64_t)i * k + C.c0;
+        T pi[V], po[V];
+        gload<T, V>(r + e, pi);
+        if constexpr (!FIRST) gload<T, V>(pold + e, po);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            if constexpr (HAS_D) pi[v] = d[i] * pi[v];
+            if constexpr (!FIRST) pi[v] = fma_t(be[v], po[v], pi[v]);
+            acc[v] += (double)pi[v] * (double)sum[v];
+        }
+        gstore<T, V>(pnew + e, pi, C.own);
+        gstore<T, V>(u + e, sum, C.own);
     }
-    return acc;
 }
+
+// Scalars of a pass, from the totals: beta, alpha and the stop test.
+template <typename T> struct PassLds {
+    double sh[3 * kWaves * kBatchMaxK], tot[3 * kBatchMaxK];
+    T al[kBatchMaxK], be[kBatchMaxK];
+    int conv, xdo;
+};
 
 // ---- K1: direction + SpMM + partial p.u -----------------------------------------
 template <typename T>
@@ -418,16 +582,22 @@ __global__ __launch_bounds__(kBlock) void bk_dir_spmm_kernel(const Tile* __restr
     const Tile tl = tiles[xcd_swizzle(blockIdx.x, gridDim.x)];
     SysState& ss = st[tl.slot];
     const SysDev<T>& S = sys[tl.slot];
-    const int it = ss.it_b;
-    const int c = threadIdx.x % S.kpad, ro = threadIdx.x / S.kpad, rows = kBlock / S.kpad;
-    const double rz = sys_total(pick(S.prz, it), S.tiles, S.k, S.kpad, c, ro, rows);
-    const double rz_prev = it > 0 ? sys_total(pick(S.prz, it + 1), S.tiles, S.k, S.kpad, c, ro, rows) : 1.0;
-    __shared__ int conv;
-    if (threadIdx.x == 0) conv = 1;
+    const int it = ss.it_b, k = S.k;
+    __shared__ PassLds<T> L;
+    const double* const parts[2] = {pick(S.prz, it), pick(S.prz, it + 1)};
+    sys_totals<2>(parts, S.tiles, k, S.kpad, L.sh, L.tot);
+    if (threadIdx.x < kWave) {
+        const int c = threadIdx.x;
+        const double rz = c < k ? L.tot[c] : 0.0;
+        const unsigned long long bad = __ballot(c < k && !(fabs(rz) <= ss.TOL[c]));
+        if (c < k) {
+            L.be[c] = (T)(rz / (it > 0 ? L.tot[kBatchMaxK + c] : 1.0));
+            if (tl.t == 0) ss.rho[c] = rz;  // current r.z, read by the host between polls
+        }
+        if (c == 0) L.conv = bad == 0;
+    }
     __syncthreads();
-    if (ro == 0 && c < S.k && !(fabs(rz) <= ss.TOL[c])) conv = 0;
-    __syncthreads();
-    if (tl.t == 0 && ro == 0 && c < S.k) ss.rho[c] = rz;  // current r.z, read by the host between polls
+    const int conv = L.conv;
     // Checkpoints depend only on the system's own iteration count, so the host's
     // decisions there do not depend on when it polls or what else runs.
     const bool pause = S.check_every > 0 && it > 0 && it % S.check_every == 0 && it != ss.resumed;
@@ -441,22 +611,37 @@ __global__ __launch_bounds__(kBlock) void bk_dir_spmm_kernel(const Tile* __restr
         return;
     }
     if (tl.t == 0 && threadIdx.x == 0) ss.it_a = it;
-    double acc = 0.0;
+    const bool first = it == 0 || it == ss.restart;
+    const T* pold = pick(S.p, it + 1);
+    T* pnew = pick(S.p, it);
     if (streaming) {
-        acc = k1_stream<T>(S, tl, c, ro, rows, it == 0 || it == ss.restart, (T)(rz / rz_prev), pick(S.p, it + 1),
-                           pick(S.p, it));
-    } else if (c < S.k) {
-        const T be = (T)(rz / rz_prev);
-        const T* pold = pick(S.p, it + 1);
-        T* pnew = pick(S.p, it);
-        if (S.d)
-            acc = (it == 0 || it == ss.restart) ? k1_rows<T, true, true>(S, tl, c, ro, rows, be, pold, pnew)
-                          : k1_rows<T, true, false>(S, tl, c, ro, rows, be, pold, pnew);
-        else
-            acc = (it == 0 || it == ss.restart) ? k1_rows<T, false, true>(S, tl, c, ro, rows, be, pold, pnew)
-                          : k1_rows<T, false, false>(S, tl, c, ro, rows, be, pold, pnew);
+        const int c = threadIdx.x % S.kpad, ro = threadIdx.x / S.kpad, rows = kBlock / S.kpad;
+        const double acc = k1_stream<T>(S, tl, c, ro, rows, first, c < k ? L.be[c] : T(0), pold, pnew);
+        tile_partial(acc, k, S.kpad, S.ppu, tl.t);
+        return;
     }
-    tile_partial(acc, S.k, S.kpad, S.ppu, tl.t);
+    by_vec<T>(S.vec, [&](auto vc) {
+        constexpr int V = decltype(vc)::value;
+        const Cols C = cols_of<V>(S);
+        double acc[V] = {};
+        if (C.own < V) {
+            T be[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v) be[v] = L.be[C.c0 + v];
+            if (S.d) {
+                if (first)
+                    k1_rows<T, V, true, true>(S, tl, C, be, pold, pnew, acc);
+                else
+                    k1_rows<T, V, true, false>(S, tl, C, be, pold, pnew, acc);
+            } else {
+                if (first)
+                    k1_rows<T, V, false, true>(S, tl, C, be, pold, pnew, acc);
+                else
+                    k1_rows<T, V, false, false>(S, tl, C, be, pold, pnew, acc);
+            }
+        }
+        tile_partial_cols<V>(acc, C, S.gs, k, S.ppu, tl.t, L.sh);
+    });
 }
 
 // ---- split form: Kdir (direction) + Kspmm (u = A p, partial p.u) ----------------
@@ -466,64 +651,13 @@ __global__ __launch_bounds__(kBlock) void bk_dir_spmm_kernel(const Tile* __restr
 // for one more launch per iteration.  The arithmetic of p, u and the partials is
 // the same as the fused form's (p = fma(beta, p_prev, z) per entry; the row sums
 // in nonzero order), so both forms give bitwise the same iterates.
-// XUPD: also x += alpha p_old, the x update of the previous iteration that the
-// update kernel leaves to this pass (which reads p_old anyway).
-template <typename T, bool HAS_D, bool FIRST, bool XUPD>
-__device__ __forceinline__ void dir_rows(const SysDev<T>& S, const Tile& tl, int c, int ro, int rows, T be, T al,
-                                         const T* __restrict__ pold_, T* __restrict__ pnew_) {
-    const gptr<const T> pold = (gptr<const T>)pold_;
-    const gptr<T> pnew = (gptr<T>)pnew_;
-    const gptr<const T> r = (gptr<const T>)S.r;
-    const gptr<const T> d = (gptr<const T>)S.d;
-    const gptr<T> x = (gptr<T>)S.x;
-    const int k = S.k;
-    for (int i0 = tl.r0 + ro; i0 < tl.r1; i0 += kRowUnroll * rows) {
-        T rv[kRowUnroll], pv[kRowUnroll], dv[kRowUnroll], xv[kRowUnroll];
-#pragma unroll
-        for (int q = 0; q < kRowUnroll; ++q) {
-            const int i = min(i0 + q * rows, tl.r1 - 1);  // clamped: always a valid row
-            const int64_t e = (int64_t)i * k + c;
-            rv[q] = r[e];
-            if constexpr (!FIRST) pv[q] = pold[e];
-            if constexpr (HAS_D) dv[q] = d[i];
-            if constexpr (XUPD) xv[q] = x[e];
-        }
-#pragma unroll
-        for (int q = 0; q < kRowUnroll; ++q) {
-            const int i = i0 + q * rows;
-            if (i < tl.r1) {
-                const int64_t e = (int64_t)i * k + c;
-                T z = rv[q];
-                if constexpr (HAS_D) z = dv[q] * z;
-                T pi;
-                if constexpr (FIRST)
-                    pi = z;
-                else
-                    pi = fma_t(be, pv[q], z);
-                pnew[e] = pi;
-                if constexpr (XUPD) x[e] = fma_t(al, pv[q], xv[q]);
-            }
-        }
-    }
-}
-
-// x += alpha p_old alone: the deferred x update of a system that stops or pauses here.
-template <typename T>
-__device__ __forceinline__ void x_rows(const SysDev<T>& S, const Tile& tl, int c, int ro, int rows, T al,
-                                       const T* __restrict__ pold_) {
-    const gptr<const T> pold = (gptr<const T>)pold_;
-    const gptr<T> x = (gptr<T>)S.x;
-    const int k = S.k;
-    for (int i = tl.r0 + ro; i < tl.r1; i += rows) {
-        const int64_t e = (int64_t)i * k + c;
-        x[e] = fma_t(al, pold[e], x[e]);
-    }
-}
+// With it goes x += alpha p_old, the x update of the previous iteration that the update
+// kernel leaves to this pass (which reads p_old anyway).
 
 // IDX16: column indices from the 16-bit offsets (2 bytes per nonzero instead of 4).
-template <typename T, bool IDX16>
-__device__ __forceinline__ double spmm_dot_rows(const SysDev<T>& S, const Tile& tl, int c, int ro, int rows,
-                                                const T* __restrict__ p_, double acc = 0.0) {
+template <typename T, int V, bool IDX16>
+__device__ __forceinline__ void spmm_dot_rows(const SysDev<T>& S, const Tile& tl, const Cols& C,
+                                              const T* __restrict__ p_, double (&acc)[V]) {
     const gptr<const T> p = (gptr<const T>)p_;
     const gptr<const int32_t> rp = (gptr<const int32_t>)S.rp;
     const gptr<const int32_t> ci = (gptr<const int32_t>)S.ci;
@@ -531,14 +665,14 @@ __device__ __forceinline__ double spmm_dot_rows(const SysDev<T>& S, const Tile& 
     const gptr<const T> val = (gptr<const T>)S.val;
     const gptr<T> u = (gptr<T>)S.u;
     const int k = S.k;
-    for (int i = tl.r0 + ro; i < tl.r1; i += rows) {
+    for (int i = tl.r0 + C.ro; i < tl.r1; i += C.rows) {
         const int lb = rp[i], le = rp[i + 1];
-        const int64_t e = (int64_t)i * k + c;
-        const T pi = p[e];  // issued with the index loads
-        T sum = T(0);
+        const int64_t e = (int64_t)i * k + C.c0;
+        T pi[V], sum[V] = {};
+        gload<T, V>(p + e, pi);  // issued with the index loads
         for (int l0 = lb; l0 < le; l0 += kGather) {
             int32_t jj[kGather];
-            T vv[kGather], pj[kGather];
+            T vv[kGather], pj[kGather][V];
 #pragma unroll
             for (int q = 0; q < kGather; ++q) {
                 const int lq = min(l0 + q, le - 1);
@@ -553,14 +687,17 @@ __device__ __forceinline__ double spmm_dot_rows(const SysDev<T>& S, const Tile& 
                 vv[q] = ok ? vq : T(0);
             }
 #pragma unroll
-            for (int q = 0; q < kGather; ++q) pj[q] = p[(int64_t)jj[q] * k + c];
+            for (int q = 0; q < kGather; ++q) gload<T, V>(p + ((int64_t)jj[q] * k + C.c0), pj[q]);
 #pragma unroll
-            for (int q = 0; q < kGather; ++q) sum += (l0 + q < le) ? vv[q] * pj[q] : T(0);
+            for (int q = 0; q < kGather; ++q) {
+#pragma unroll
+                for (int v = 0; v < V; ++v) sum[v] += (l0 + q < le) ? vv[q] * pj[q][v] : T(0);
+            }
         }
-        u[e] = sum;
-        acc += (double)pi * (double)sum;
+        gstore<T, V>(u + e, sum, C.own);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += (double)pi[v] * (double)sum[v];
     }
-    return acc;
 }
 
 // The software-pipelined form of spmm_dot_rows.  The row pointers of a segment of
@@ -598,109 +735,93 @@ __device__ __forceinline__ void row_chunk_indices(const SysDev<T>& S, int i, int
     }
 }
 
-template <typename T, bool IDX16>
-__device__ __forceinline__ double spmm_dot_rows_pipe(const SysDev<T>& S, int s0, int s1, const int* rps, int c,
-                                                     int ro, int rows, const T* __restrict__ p_, double acc) {
+template <typename T, int V, bool IDX16>
+__device__ __forceinline__ void spmm_dot_rows_pipe(const SysDev<T>& S, int s0, int s1, const int* rps, const Cols& C,
+                                                   const T* __restrict__ p_, double (&acc)[V]) {
     const gptr<const T> p = (gptr<const T>)p_;
-    const gptr<const int32_t> ci = (gptr<const int32_t>)S.ci;
-    const gptr<const int16_t> cid = (gptr<const int16_t>)S.cid;
-    const gptr<const T> val = (gptr<const T>)S.val;
     const gptr<T> u = (gptr<T>)S.u;
     const int k = S.k;
-    int i = s0 + ro;
-    if (i >= s1) return acc;
+    int i = s0 + C.ro;
+    if (i >= s1) return;
     int32_t jA[kGather];
     T vA[kGather];
     row_chunk_indices<T, IDX16>(S, i, rps[i - s0], rps[i - s0 + 1], jA, vA);
-    for (; i < s1; i += rows) {
-        const int in = i + rows;
+    for (; i < s1; i += C.rows) {
+        const int in = i + C.rows;
         int32_t jB[kGather];
         T vB[kGather];
         if (in < s1) row_chunk_indices<T, IDX16>(S, in, rps[in - s0], rps[in - s0 + 1], jB, vB);
         const int lb = rps[i - s0], le = rps[i - s0 + 1];
-        const int64_t e = (int64_t)i * k + c;
-        const T pi = p[e];
-        T pj[kGather];
+        const int64_t e = (int64_t)i * k + C.c0;
+        T pi[V], sum[V] = {};
+        gload<T, V>(p + e, pi);
+        for (int l0 = lb; l0 < le; l0 += kGather) {  // a row longer than one chunk: the rest as it comes
+            if (l0 > lb) row_chunk_indices<T, IDX16>(S, i, l0, le, jA, vA);
+            T pj[kGather][V];
 #pragma unroll
-        for (int q = 0; q < kGather; ++q) pj[q] = p[(int64_t)jA[q] * k + c];
-        T sum = T(0);
-#pragma unroll
-        for (int q = 0; q < kGather; ++q) sum += (lb + q < le) ? vA[q] * pj[q] : T(0);
-        for (int l0 = lb + kGather; l0 < le; l0 += kGather) {  // rows longer than one chunk
-            int32_t jj[kGather];
-            T vv[kGather];
+            for (int q = 0; q < kGather; ++q) gload<T, V>(p + ((int64_t)jA[q] * k + C.c0), pj[q]);
 #pragma unroll
             for (int q = 0; q < kGather; ++q) {
-                const int lq = min(l0 + q, le - 1);
-                int32_t cq;
-                if constexpr (IDX16)
-                    cq = i + (int32_t)cid[lq];
-                else
-                    cq = ci[lq];
-                const T vq = val[lq];
-                const bool ok = l0 + q < le;
-                jj[q] = ok ? cq : i;
-                vv[q] = ok ? vq : T(0);
+#pragma unroll
+                for (int v = 0; v < V; ++v) sum[v] += (l0 + q < le) ? vA[q] * pj[q][v] : T(0);
             }
-#pragma unroll
-            for (int q = 0; q < kGather; ++q) pj[q] = p[(int64_t)jj[q] * k + c];
-#pragma unroll
-            for (int q = 0; q < kGather; ++q) sum += (l0 + q < le) ? vv[q] * pj[q] : T(0);
         }
-        u[e] = sum;
-        acc += (double)pi * (double)sum;
+        gstore<T, V>(u + e, sum, C.own);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += (double)pi[v] * (double)sum[v];
 #pragma unroll
         for (int q = 0; q < kGather; ++q) {
             jA[q] = jB[q];
             vA[q] = vB[q];
         }
     }
-    return acc;
 }
 
 constexpr int kPipeSeg = 2048;  // rows per LDS segment of row pointers in the pipelined SpMM
-constexpr int kLdsRows = 256;   // rows per segment of the LDS-staged SpMM (a multiple of every kBlock / kpad)
-constexpr int kLdsNnz = 1792;   // nonzeros of a segment that fit the staging buffers (7 per row)
+constexpr int kLdsRows = 256;   // rows per segment of the LDS-staged SpMM (a multiple of every kBlock >> gs)
+constexpr int kLdsNnz = 7 * kBlock;  // nonzeros of a segment that fit the staging buffers (7 per row)
+constexpr int kLdsTile = 1024;  // rows whose row pointers are staged at a time (a multiple of kLdsRows)
 
 // The rows [s0, s1) of a segment whose 16-bit column offsets and values sit in LDS
 // from nonzero rps[0] on: the gathers and the arithmetic of spmm_dot_rows, the index
 // loads from LDS.  acc continues the lane's partial.
-template <typename T>
-__device__ __forceinline__ double spmm_dot_rows_lds(const SysDev<T>& S, int s0, int s1, const int* rps,
-                                                    const int16_t* cls, const T* vls, int c, int ro, int rows,
-                                                    const T* __restrict__ p_, double acc) {
+template <typename T, int V>
+__device__ __forceinline__ void spmm_dot_rows_lds(const SysDev<T>& S, int s0, int s1, const int* rps, const int16_t* cls,
+                                                  const T* vls, const Cols& C, const T* __restrict__ p_,
+                                                  double (&acc)[V]) {
     const gptr<const T> p = (gptr<const T>)p_;
     const gptr<T> u = (gptr<T>)S.u;
     const int k = S.k;
     const int base = rps[0];
-    for (int i = s0 + ro; i < s1; i += rows) {
+    for (int i = s0 + C.ro; i < s1; i += C.rows) {
         const int lb = rps[i - s0] - base, le = rps[i - s0 + 1] - base;
-        const int64_t e = (int64_t)i * k + c;
-        const T pi = p[e];
-        T sum = T(0);
+        const int64_t e = (int64_t)i * k + C.c0;
+        T pi[V], sum[V] = {};
+        gload<T, V>(p + e, pi);
         for (int l0 = lb; l0 < le; l0 += kGather) {
-            T pj[kGather];
+            T pj[kGather][V];
 #pragma unroll
             for (int q = 0; q < kGather; ++q) {
                 const int lq = min(l0 + q, le - 1);
                 const int32_t jj = l0 + q < le ? i + (int32_t)cls[lq] : i;
                 // 32-bit byte offset from the block-uniform base (n k sizeof(T) < 4 GiB is
                 // checked at add): one address register per gather instead of two
-                const uint32_t off = ((uint32_t)jj * (uint32_t)k + (uint32_t)c) * (uint32_t)sizeof(T);
-                pj[q] = *(gptr<const T>)((gptr<const char>)p + off);
+                const uint32_t off = ((uint32_t)jj * (uint32_t)k + (uint32_t)C.c0) * (uint32_t)sizeof(T);
+                gload<T, V>((gptr<const T>)((gptr<const char>)p + off), pj[q]);
             }
             // the values only now, from LDS: fewer registers live across the gathers
 #pragma unroll
             for (int q = 0; q < kGather; ++q) {
                 const bool ok = l0 + q < le;
                 const T vv = ok ? vls[min(l0 + q, le - 1)] : T(0);
-                sum += ok ? vv * pj[q] : T(0);
+#pragma unroll
+                for (int v = 0; v < V; ++v) sum[v] += ok ? vv * pj[q][v] : T(0);
             }
         }
-        u[e] = sum;
-        acc += (double)pi * (double)sum;
+        gstore<T, V>(u + e, sum, C.own);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += (double)pi[v] * (double)sum[v];
     }
-    return acc;
 }
 
 // The rows of spmm_dot_rows one nonzero at a time, with few registers: the rare paths
@@ -710,9 +831,9 @@ __device__ __forceinline__ double spmm_dot_rows_lds(const SysDev<T>& S, int s0, 
 // masked product through a select, which the compiler does not contract); it only
 // skips the +0 that loop adds for masked slots, which changes no value but the sign
 // of a zero sum.
-template <typename T, bool IDX16>
-__device__ __attribute__((noinline)) double spmm_dot_rows_lean(const SysDev<T>& S, int r0, int r1, int c, int ro,
-                                                               int rows, const T* __restrict__ p_, double acc) {
+template <typename T, int V, bool IDX16>
+__device__ __forceinline__ void spmm_dot_rows_lean(const SysDev<T>& S, int r0, int r1, const Cols& C,
+                                                   const T* __restrict__ p_, double (&acc)[V]) {
     const gptr<const T> p = (gptr<const T>)p_;
     const gptr<const int32_t> rp = (gptr<const int32_t>)S.rp;
     const gptr<const int32_t> ci = (gptr<const int32_t>)S.ci;
@@ -720,84 +841,125 @@ __device__ __attribute__((noinline)) double spmm_dot_rows_lean(const SysDev<T>& 
     const gptr<const T> val = (gptr<const T>)S.val;
     const gptr<T> u = (gptr<T>)S.u;
     const int k = S.k;
-    for (int i = r0 + ro; i < r1; i += rows) {
-        const int64_t e = (int64_t)i * k + c;
-        const T pi = p[e];
-        T sum = T(0);
+    for (int i = r0 + C.ro; i < r1; i += C.rows) {
+        const int64_t e = (int64_t)i * k + C.c0;
+        T pi[V], sum[V] = {};
+        gload<T, V>(p + e, pi);
         for (int l = rp[i], le = rp[i + 1]; l < le; ++l) {
 #pragma clang fp contract(off)
             const int32_t j = IDX16 ? i + (int32_t)cid[l] : ci[l];
-            sum += val[l] * p[(int64_t)j * k + c];
+            T pj[V];
+            gload<T, V>(p + ((int64_t)j * k + C.c0), pj);
+#pragma unroll
+            for (int v = 0; v < V; ++v) sum[v] += val[l] * pj[v];
         }
-        u[e] = sum;
-        acc += (double)pi * (double)sum;
+        gstore<T, V>(u + e, sum, C.own);
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += (double)pi[v] * (double)sum[v];
     }
-    return acc;
 }
 
 // Kdir: beta, the stop test and the checkpoint pause as in K1; then p for the own
 // rows, together with the previous iteration's x += alpha p (deferred from the
 // update kernel).  A tile applies that x update once per iteration (xit), also
 // when the system stops or pauses here; before a checkpoint the update kernel has
-// done it already.  So x is whole whenever the host reads it.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void bk_dir_kernel(const Tile* __restrict__ tiles, const SysDev<T>* __restrict__ sys,
-                                                        SysState* __restrict__ st) {
-    const Tile tl = tiles[xcd_swizzle(blockIdx.x, gridDim.x)];
-    SysState& ss = st[tl.slot];
-    const SysDev<T>& S = sys[tl.slot];
-    const int it = ss.it_b;
-    const int c = threadIdx.x % S.kpad, ro = threadIdx.x / S.kpad, rows = kBlock / S.kpad;
-    const double rz = sys_total(pick(S.prz, it), S.tiles, S.k, S.kpad, c, ro, rows);
-    const double rz_prev = it > 0 ? sys_total(pick(S.prz, it + 1), S.tiles, S.k, S.kpad, c, ro, rows) : 1.0;
-    __shared__ int conv, xdo;
-    if (threadIdx.x == 0) {
-        conv = 1;
-        xdo = it > 0 && S.xit[tl.t] != it;
+// done it already.  So x is whole whenever the host reads it.  The first rows are
+// loaded before the totals are known.
+template <typename T, int V>
+__device__ __forceinline__ void dir_tile(const SysDev<T>& S, const Tile& tl, SysState& ss, PassLds<T>& L) {
+    const Cols C = cols_of<V>(S);
+    const int it = ss.it_b, k = S.k, c0 = C.c0;
+    const gptr<const T> pold = (gptr<const T>)pick(S.p, it + 1);
+    const gptr<T> pnew = (gptr<T>)pick(S.p, it);
+    const gptr<const T> r = (gptr<const T>)S.r;
+    const gptr<const T> d = (gptr<const T>)S.d;
+    const gptr<T> x = (gptr<T>)S.x;
+    T rv[kRowUnroll][V], pv[kRowUnroll][V], xv[kRowUnroll][V], dv[kRowUnroll];
+    auto load = [&](int i0) {
+#pragma unroll
+        for (int q = 0; q < kRowUnroll; ++q) {
+            const int i = min(i0 + q * C.rows, tl.r1 - 1);  // clamped: always a valid row
+            const int64_t e = (int64_t)i * k + c0;
+            gload<T, V>(r + e, rv[q]);
+            gload<T, V>(pold + e, pv[q]);
+            gload<T, V>((gptr<const T>)x + e, xv[q]);
+            dv[q] = d ? d[i] : T(1);
+        }
+    };
+    const int first_row = tl.r0 + C.ro;
+    load(first_row);
+    if (threadIdx.x == 0) L.xdo = it > 0 && S.xit[tl.t] != it;
+    // alpha of iteration it - 1 from the same partials and sums the update kernel used
+    const double* const parts[3] = {pick(S.prz, it), pick(S.prz, it + 1), S.ppu};
+    sys_totals<3>(parts, S.tiles, k, S.kpad, L.sh, L.tot);
+    const bool xdo = L.xdo;
+    if (threadIdx.x < kWave) {
+        const int c = threadIdx.x;
+        const double rz = c < k ? L.tot[c] : 0.0;
+        const unsigned long long bad = __ballot(c < k && !(fabs(rz) <= ss.TOL[c]));
+        if (c < k) {
+            const double rz_prev = it > 0 ? L.tot[kBatchMaxK + c] : 1.0;
+            L.be[c] = (T)(rz / rz_prev);
+            L.al[c] = (T)(rz_prev / (xdo ? L.tot[2 * kBatchMaxK + c] : 1.0));
+            if (tl.t == 0) ss.rho[c] = rz;
+        }
+        if (c == 0) {
+            L.conv = bad == 0;
+            if (xdo) S.xit[tl.t] = it;
+        }
     }
     __syncthreads();
-    if (threadIdx.x == 0 && xdo) S.xit[tl.t] = it;
-    // alpha of iteration it - 1 from the same partials and sums the update kernel used
-    const double pu = xdo ? sys_total(S.ppu, S.tiles, S.k, S.kpad, c, ro, rows) : 1.0;
-    const T al = (T)(rz_prev / pu);
-    if (ro == 0 && c < S.k && !(fabs(rz) <= ss.TOL[c])) conv = 0;
-    __syncthreads();
-    if (tl.t == 0 && ro == 0 && c < S.k) ss.rho[c] = rz;
+    const int conv = L.conv;
     const bool pause = S.check_every > 0 && it > 0 && it % S.check_every == 0 && it != ss.resumed;
-    const T* pold = pick(S.p, it + 1);
-    if (conv || it >= ss.max_iter || pause) {
-        if (tl.t == 0 && threadIdx.x == 0) {
+    const bool stop = conv || it >= ss.max_iter || pause;
+    if (tl.t == 0 && threadIdx.x == 0) {
+        if (stop) {
             ss.iter = it;
             ss.succ = conv;
             ss.paused = (!conv && it < ss.max_iter) ? 1 : 0;
             ss.done = 1;
+        } else {
+            ss.it_a = it;
         }
-        if (xdo && c < S.k) x_rows<T>(S, tl, c, ro, rows, al, pold);
-        return;
     }
-    if (tl.t == 0 && threadIdx.x == 0) ss.it_a = it;
+    if (C.own >= V || (stop && !xdo)) return;
     // p = z at iteration 0 and where the host restarted the direction (after a pause,
     // so the deferred x update is done: xdo is false there)
     const bool first = it == 0 || (it == ss.restart && !xdo);
-    if (c < S.k) {
-        const T be = (T)(rz / rz_prev);
-        T* pnew = pick(S.p, it);
-        if (S.d) {
-            if (first)
-                dir_rows<T, true, true, false>(S, tl, c, ro, rows, be, al, pold, pnew);
-            else if (xdo)
-                dir_rows<T, true, false, true>(S, tl, c, ro, rows, be, al, pold, pnew);
-            else
-                dir_rows<T, true, false, false>(S, tl, c, ro, rows, be, al, pold, pnew);
-        } else {
-            if (first)
-                dir_rows<T, false, true, false>(S, tl, c, ro, rows, be, al, pold, pnew);
-            else if (xdo)
-                dir_rows<T, false, false, true>(S, tl, c, ro, rows, be, al, pold, pnew);
-            else
-                dir_rows<T, false, false, false>(S, tl, c, ro, rows, be, al, pold, pnew);
+    T be[V], al[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        be[v] = L.be[c0 + v];
+        al[v] = L.al[c0 + v];
+    }
+    for (int i0 = first_row; i0 < tl.r1; i0 += kRowUnroll * C.rows) {
+        if (i0 > first_row) load(i0);
+#pragma unroll
+        for (int q = 0; q < kRowUnroll; ++q) {
+            const int i = i0 + q * C.rows;
+            if (i < tl.r1) {
+                const int64_t e = (int64_t)i * k + c0;
+                T pi[V], xi[V];
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    const T z = d ? dv[q] * rv[q][v] : rv[q][v];
+                    pi[v] = first ? z : fma_t(be[v], pv[q][v], z);
+                    xi[v] = fma_t(al[v], pv[q][v], xv[q][v]);
+                }
+                if (!stop) gstore<T, V>(pnew + e, pi, C.own);
+                if (xdo) gstore<T, V>(x + e, xi, C.own);
+            }
         }
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kBlock) void bk_dir_kernel(const Tile* __restrict__ tiles, const SysDev<T>* __restrict__ sys,
+                                                        SysState* __restrict__ st) {
+    __shared__ PassLds<T> L;
+    const Tile tl = tiles[xcd_swizzle(blockIdx.x, gridDim.x)];
+    const SysDev<T>& S = sys[tl.slot];
+    by_vec<T>(S.vec, [&](auto vc) { dir_tile<T, decltype(vc)::value>(S, tl, st[tl.slot], L); });
 }
 
 // Kspmm: u = A p and the tile partial of p.u (systems stopped by Kdir skip).
@@ -805,17 +967,24 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void bk_spmm_dot_kernel(const Tile* __restrict__ tiles,
                                                              const SysDev<T>* __restrict__ sys,
                                                              SysState* __restrict__ st) {
+    __shared__ double sh[kWaves * kBatchMaxK];
     const Tile tl = tiles[xcd_swizzle(blockIdx.x, gridDim.x)];
     SysState& ss = st[tl.slot];
     if (ss.done) return;
     const SysDev<T>& S = sys[tl.slot];
-    const int it = ss.it_a;
-    const int c = threadIdx.x % S.kpad, ro = threadIdx.x / S.kpad, rows = kBlock / S.kpad;
-    double acc = 0.0;
-    if (c < S.k)
-        acc = S.cid ? spmm_dot_rows<T, true>(S, tl, c, ro, rows, pick(S.p, it))
-                    : spmm_dot_rows<T, false>(S, tl, c, ro, rows, pick(S.p, it));
-    tile_partial(acc, S.k, S.kpad, S.ppu, tl.t);
+    const T* p = pick(S.p, ss.it_a);
+    by_vec<T>(S.vec, [&](auto vc) {
+        constexpr int V = decltype(vc)::value;
+        const Cols C = cols_of<V>(S);
+        double acc[V] = {};
+        if (C.own < V) {
+            if (S.cid)
+                spmm_dot_rows<T, V, true>(S, tl, C, p, acc);
+            else
+                spmm_dot_rows<T, V, false>(S, tl, C, p, acc);
+        }
+        tile_partial_cols<V>(acc, C, S.gs, S.k, S.ppu, tl.t, sh);
+    });
 }
 
 // Kspmm with the column indices and values staged through LDS.  A row per lane
@@ -824,6 +993,8 @@ __global__ __launch_bounds__(kBlock) void bk_spmm_dot_kernel(const Tile* __restr
 // every load instruction touches many lines and each line is touched once per
 // slot; here the workgroup first copies a 256-row segment's nonzeros with
 // consecutive lanes on consecutive nonzeros, then the row loop reads them from LDS.
+// The next segment's nonzeros are loaded into registers during this one's gathers (100
+// VGPRs; held to 96 or 80, for a fifth or sixth wave per SIMD, it measured no faster).
 // Systems with 16-bit column offsets only (the others, and a segment with more than
 // kLdsNnz nonzeros, take the global loads of spmm_dot_rows_lean).  Rows, lanes and
 // arithmetic are those of spmm_dot_rows: bitwise the same u and partials.
@@ -831,46 +1002,72 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void bk_spmm_dot_lds_kernel(const Tile* __restrict__ tiles,
                                                                  const SysDev<T>* __restrict__ sys,
                                                                  SysState* __restrict__ st) {
-    __shared__ int rps[kLdsRows + 1];
+    __shared__ int rps[kLdsTile + 1];
     __shared__ int16_t cls[kLdsNnz];
-    // the staged values; after the last segment the tile partial's reduction buffer
-    __shared__ __align__(16) char vbuf[kLdsNnz * sizeof(T) > kBlock * sizeof(double) ? kLdsNnz * sizeof(T)
-                                                                                      : kBlock * sizeof(double)];
-    T* vls = (T*)vbuf;
+    __shared__ T vls[kLdsNnz];
+    __shared__ double sh[kWaves * kBatchMaxK];
     const Tile tl = tiles[xcd_swizzle(blockIdx.x, gridDim.x)];
     SysState& ss = st[tl.slot];
     if (ss.done) return;
     const SysDev<T>& S = sys[tl.slot];
-    const int it = ss.it_a;
-    const int c = threadIdx.x % S.kpad, ro = threadIdx.x / S.kpad, rows = kBlock / S.kpad;
     const gptr<const int32_t> rp = (gptr<const int32_t>)S.rp;
     const gptr<const int16_t> cid = (gptr<const int16_t>)S.cid;
     const gptr<const T> val = (gptr<const T>)S.val;
-    const T* p = pick(S.p, it);
-    double acc = 0.0;
-    if (!S.cid) {
-        if (c < S.k) acc = spmm_dot_rows_lean<T, false>(S, tl.r0, tl.r1, c, ro, rows, p, acc);
-        tile_partial_in(acc, S.k, S.kpad, S.ppu, tl.t, (double*)vbuf);
-        return;
-    }
-    for (int s0 = tl.r0; s0 < tl.r1; s0 += kLdsRows) {
-        const int s1 = min(s0 + kLdsRows, tl.r1);
-        for (int j = threadIdx.x; j <= s1 - s0; j += kBlock) rps[j] = rp[s0 + j];
-        __syncthreads();
-        const int base = rps[0], cnt = rps[s1 - s0] - base;
-        if (cnt <= kLdsNnz) {
-            for (int t = threadIdx.x; t < cnt; t += kBlock) {
-                cls[t] = cid[base + t];
-                vls[t] = val[base + t];
-            }
-            __syncthreads();
-            if (c < S.k) acc = spmm_dot_rows_lds<T>(S, s0, s1, rps, cls, vls, c, ro, rows, p, acc);
-        } else if (c < S.k) {
-            acc = spmm_dot_rows_lean<T, true>(S, s0, s1, c, ro, rows, p, acc);
+    const T* p = pick(S.p, ss.it_a);
+    by_vec<T>(S.vec, [&](auto vc) {
+        constexpr int V = decltype(vc)::value, PER = kLdsNnz / kBlock;
+        const Cols C = cols_of<V>(S);
+        double acc[V] = {};
+        if (!S.cid) {
+            if (C.own < V) spmm_dot_rows_lean<T, V, false>(S, tl.r0, tl.r1, C, p, acc);
+            tile_partial_cols<V>(acc, C, S.gs, S.k, S.ppu, tl.t, sh);
+            return;
         }
-        __syncthreads();
-    }
-    tile_partial_in(acc, S.k, S.kpad, S.ppu, tl.t, (double*)vbuf);
+        int16_t cn[PER];
+        T vn[PER];
+        // the nonzeros [rps[a], rps[b]) of a segment that fits the buffers (clamped to its last)
+        auto fetch = [&](int a, int b) {
+            const int base = rps[a], cnt = rps[b] - base;
+            if (cnt > 0 && cnt <= kLdsNnz) {
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    const int l = base + min((int)threadIdx.x + q * kBlock, cnt - 1);
+                    cn[q] = cid[l];
+                    vn[q] = val[l];
+                }
+            }
+        };
+        for (int t0 = tl.r0; t0 < tl.r1; t0 += kLdsTile) {
+            const int nr = min(kLdsTile, tl.r1 - t0);
+            for (int j = threadIdx.x; j <= nr; j += kBlock) rps[j] = rp[t0 + j];
+            __syncthreads();
+            fetch(0, min(kLdsRows, nr));
+            for (int a = 0; a < nr; a += kLdsRows) {
+                const int b = min(a + kLdsRows, nr), cnt = rps[b] - rps[a];
+                const bool fits = cnt <= kLdsNnz;
+                if (fits) {
+#pragma unroll
+                    for (int q = 0; q < PER; ++q) {
+                        const int t = threadIdx.x + q * kBlock;
+                        if (t < cnt) {
+                            cls[t] = cn[q];
+                            vls[t] = vn[q];
+                        }
+                    }
+                }
+                __syncthreads();
+                if (b < nr) fetch(b, min(b + kLdsRows, nr));
+                if (C.own < V) {
+                    if (fits)
+                        spmm_dot_rows_lds<T, V>(S, t0 + a, t0 + b, rps + a, cls, vls, C, p, acc);
+                    else
+                        spmm_dot_rows_lean<T, V, true>(S, t0 + a, t0 + b, C, p, acc);
+                }
+                __syncthreads();
+            }
+        }
+        tile_partial_cols<V>(acc, C, S.gs, S.k, S.ppu, tl.t, sh);
+    });
 }
 
 // Kspmm, software-pipelined: the tile's row pointers go through LDS in segments.
@@ -882,98 +1079,122 @@ __global__ __launch_bounds__(kBlock) void bk_spmm_dot_pipe_kernel(const Tile* __
                                                                   const SysDev<T>* __restrict__ sys,
                                                                   SysState* __restrict__ st) {
     __shared__ int rps[kPipeSeg + 1];
+    __shared__ double sh[kWaves * kBatchMaxK];
     const Tile tl = tiles[xcd_swizzle(blockIdx.x, gridDim.x)];
     SysState& ss = st[tl.slot];
     if (ss.done) return;
     const SysDev<T>& S = sys[tl.slot];
-    const int it = ss.it_a;
-    const int c = threadIdx.x % S.kpad, ro = threadIdx.x / S.kpad, rows = kBlock / S.kpad;
     const gptr<const int32_t> rp = (gptr<const int32_t>)S.rp;
-    const T* p = pick(S.p, it);
-    double acc = 0.0;
-    for (int s0 = tl.r0; s0 < tl.r1; s0 += kPipeSeg) {
-        const int s1 = min(s0 + kPipeSeg, tl.r1);
-        for (int j = threadIdx.x; j <= s1 - s0; j += kBlock) rps[j] = rp[s0 + j];
-        __syncthreads();
-        if (c < S.k)  // the lane's partial continues across segments, as in one pass over the tile
-            acc = S.cid ? spmm_dot_rows_pipe<T, true>(S, s0, s1, rps, c, ro, rows, p, acc)
-                        : spmm_dot_rows_pipe<T, false>(S, s0, s1, rps, c, ro, rows, p, acc);
-        __syncthreads();
-    }
-    tile_partial(acc, S.k, S.kpad, S.ppu, tl.t);
+    const T* p = pick(S.p, ss.it_a);
+    by_vec<T>(S.vec, [&](auto vc) {
+        constexpr int V = decltype(vc)::value;
+        const Cols C = cols_of<V>(S);
+        double acc[V] = {};
+        for (int s0 = tl.r0; s0 < tl.r1; s0 += kPipeSeg) {
+            const int s1 = min(s0 + kPipeSeg, tl.r1);
+            for (int j = threadIdx.x; j <= s1 - s0; j += kBlock) rps[j] = rp[s0 + j];
+            __syncthreads();
+            if (C.own < V) {  // the lane's partial continues across segments, as in one pass over the tile
+                if (S.cid)
+                    spmm_dot_rows_pipe<T, V, true>(S, s0, s1, rps, C, p, acc);
+                else
+                    spmm_dot_rows_pipe<T, V, false>(S, s0, s1, rps, C, p, acc);
+            }
+            __syncthreads();
+        }
+        tile_partial_cols<V>(acc, C, S.gs, S.k, S.ppu, tl.t, sh);
+    });
 }
 
-// ---- K2 body: kRowUnroll rows per step, all loads first, then the stores ----------
-// DEFER_X: x is left to the next direction pass (bk_dir_kernel): r and u only.
-template <typename T, bool HAS_D, bool DEFER_X>
-__device__ __forceinline__ double k2_rows(const SysDev<T>& S, const Tile& tl, int c, int ro, int rows, T al,
-                                          const T* __restrict__ p_) {
-    const gptr<const T> p = (gptr<const T>)p_;
+// ---- K2: x, r, z update + partial r.z (next parity) -------------------------------
+// kRowUnroll rows per step, all loads first, then the stores; the first rows are loaded
+// before the totals are known.  DEFER_X: x is left to the next direction pass (dir_tile),
+// r only.
+template <typename T, int V, bool DEFER_X>
+__device__ __forceinline__ void update_tile(const SysDev<T>& S, const Tile& tl, SysState& ss, PassLds<T>& L) {
+    const Cols C = cols_of<V>(S);
+    const int it = ss.it_a, k = S.k, c0 = C.c0;
+    // Before a checkpoint the x update is done here: the host may read x there
+    // without the direction pass having run (a poll that lands on the checkpoint).
+    const bool xnow = !DEFER_X || (S.check_every > 0 && (it + 1) % S.check_every == 0);
+    const gptr<const T> p = (gptr<const T>)pick(S.p, it);
     const gptr<const T> u = (gptr<const T>)S.u;
     const gptr<const T> d = (gptr<const T>)S.d;
     const gptr<T> x = (gptr<T>)S.x;
     const gptr<T> r = (gptr<T>)S.r;
-    const int k = S.k;
-    double acc = 0.0;
-    for (int i0 = tl.r0 + ro; i0 < tl.r1; i0 += kRowUnroll * rows) {
-        T pv[kRowUnroll], xv[kRowUnroll], rv[kRowUnroll], uv[kRowUnroll], dv[kRowUnroll];
+    T rv[kRowUnroll][V], uv[kRowUnroll][V], dv[kRowUnroll];
+    auto load = [&](int i0) {
 #pragma unroll
         for (int q = 0; q < kRowUnroll; ++q) {
-            const int i = min(i0 + q * rows, tl.r1 - 1);  // clamped: always a valid row
-            const int64_t e = (int64_t)i * k + c;
-            if constexpr (!DEFER_X) {
-                pv[q] = p[e];
-                xv[q] = x[e];
-            }
-            rv[q] = r[e];
-            uv[q] = u[e];
-            if constexpr (HAS_D) dv[q] = d[i];
+            const int i = min(i0 + q * C.rows, tl.r1 - 1);  // clamped: always a valid row
+            const int64_t e = (int64_t)i * k + c0;
+            gload<T, V>((gptr<const T>)r + e, rv[q]);
+            gload<T, V>(u + e, uv[q]);
+            dv[q] = d ? d[i] : T(1);
         }
+    };
+    const int first_row = tl.r0 + C.ro;
+    load(first_row);
+    const double* const parts[2] = {pick(S.prz, it), S.ppu};
+    sys_totals<2>(parts, S.tiles, k, S.kpad, L.sh, L.tot);
+    double acc[V] = {};
+    if (C.own < V) {
+        T al[V];
 #pragma unroll
-        for (int q = 0; q < kRowUnroll; ++q) {
-            const int i = i0 + q * rows;
-            if (i < tl.r1) {
-                const int64_t e = (int64_t)i * k + c;
-                if constexpr (!DEFER_X) x[e] = fma_t(al, pv[q], xv[q]);
-                const T rn = rv[q] - al * uv[q];
-                r[e] = rn;
-                T zv = rn;
-                if constexpr (HAS_D) zv = dv[q] * rn;
-                acc += (double)rn * (double)zv;
+        for (int v = 0; v < V; ++v) al[v] = (T)(L.tot[c0 + v] / L.tot[kBatchMaxK + c0 + v]);
+        for (int i0 = first_row; i0 < tl.r1; i0 += kRowUnroll * C.rows) {
+            if (i0 > first_row) load(i0);
+#pragma unroll
+            for (int q = 0; q < kRowUnroll; ++q) {
+                const int i = i0 + q * C.rows;
+                if (i < tl.r1) {
+                    const int64_t e = (int64_t)i * k + c0;
+                    T rn[V];
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        rn[v] = rv[q][v] - al[v] * uv[q][v];
+                        const T zv = d ? dv[q] * rn[v] : rn[v];
+                        acc[v] += (double)rn[v] * (double)zv;
+                    }
+                    gstore<T, V>(r + e, rn, C.own);
+                }
+            }
+        }
+        // (a loop of its own: one iteration in check_every takes it, and its rows would cost
+        // every one the registers)
+        for (int i0 = first_row; xnow && i0 < tl.r1; i0 += kRowUnroll * C.rows) {
+            T pv[kRowUnroll][V], xv[kRowUnroll][V];
+#pragma unroll
+            for (int q = 0; q < kRowUnroll; ++q) {
+                const int64_t e = (int64_t)min(i0 + q * C.rows, tl.r1 - 1) * k + c0;
+                gload<T, V>(p + e, pv[q]);
+                gload<T, V>((gptr<const T>)x + e, xv[q]);
+            }
+#pragma unroll
+            for (int q = 0; q < kRowUnroll; ++q) {
+                const int i = i0 + q * C.rows;
+                T xi[V];
+#pragma unroll
+                for (int v = 0; v < V; ++v) xi[v] = fma_t(al[v], pv[q][v], xv[q][v]);
+                if (i < tl.r1) gstore<T, V>(x + ((int64_t)i * k + c0), xi, C.own);
             }
         }
     }
-    return acc;
+    if (DEFER_X && xnow && threadIdx.x == 0) S.xit[tl.t] = it + 1;  // the direction pass of it + 1 skips it
+    // (the totals are read: their barriers lie before the rows, and sh is not read after them)
+    tile_partial_cols<V>(acc, C, S.gs, k, pick(S.prz, it + 1), tl.t, L.sh);
+    if (tl.t == 0 && threadIdx.x == 0) ss.it_b = it + 1;
 }
 
-// ---- K2: x, r, z update + partial r.z (next parity) -------------------------------
 template <typename T, bool DEFER_X>
 __global__ __launch_bounds__(kBlock) void bk_update_kernel(const Tile* __restrict__ tiles, const SysDev<T>* __restrict__ sys,
                                                            SysState* __restrict__ st) {
+    __shared__ PassLds<T> L;
     const Tile tl = tiles[xcd_swizzle(blockIdx.x, gridDim.x)];
     SysState& ss = st[tl.slot];
     if (ss.done) return;
     const SysDev<T>& S = sys[tl.slot];
-    const int it = ss.it_a;
-    const int c = threadIdx.x % S.kpad, ro = threadIdx.x / S.kpad, rows = kBlock / S.kpad;
-    const double rz = sys_total(pick(S.prz, it), S.tiles, S.k, S.kpad, c, ro, rows);
-    const double pu = sys_total(S.ppu, S.tiles, S.k, S.kpad, c, ro, rows);
-    // Before a checkpoint the x update is done here: the host may read x there
-    // without the direction pass having run (a poll that lands on the checkpoint).
-    const bool xnow = !DEFER_X || (S.check_every > 0 && (it + 1) % S.check_every == 0);
-    double acc = 0.0;
-    if (c < S.k) {
-        const T al = (T)(rz / pu);
-        if (xnow)
-            acc = S.d ? k2_rows<T, true, false>(S, tl, c, ro, rows, al, pick(S.p, it))
-                      : k2_rows<T, false, false>(S, tl, c, ro, rows, al, pick(S.p, it));
-        else
-            acc = S.d ? k2_rows<T, true, true>(S, tl, c, ro, rows, al, pick(S.p, it))
-                      : k2_rows<T, false, true>(S, tl, c, ro, rows, al, pick(S.p, it));
-    }
-    if (DEFER_X && xnow && threadIdx.x == 0) S.xit[tl.t] = it + 1;  // the direction pass of it + 1 skips it
-    tile_partial(acc, S.k, S.kpad, pick(S.prz, it + 1), tl.t);
-    if (tl.t == 0 && threadIdx.x == 0) ss.it_b = it + 1;
+    by_vec<T>(S.vec, [&](auto vc) { update_tile<T, decltype(vc)::value, DEFER_X>(S, tl, ss, L); });
 }
 
 struct Resume {
@@ -1039,6 +1260,9 @@ template <typename T> class CGBatch {
         S.k = k;
         S.check_every = check_every;
         S.kpad = pow2_at_least(k);
+        S.vec = lane_columns(k, 16 / (int)sizeof(T));
+        S.gs = 0;
+        while (S.vec << S.gs < k) ++S.gs;
         S.tile_rows = g_batch_tile_rows;
         S.tiles = ceil_div(n, S.tile_rows);
         const size_t N = (size_t)n * k;

@@ -318,3 +318,38 @@ def test_batch_edge_cases(cuda, mixed):
     assert res[z]["succeeded"] and res[z]["iterations"] == 0 and not np.any(Xs[z])
     assert not res[nb]["succeeded"] and res[nb]["iterations"] == 0
     assert not res[cap]["succeeded"] and res[cap]["iterations"] == 0
+
+
+@pytest.mark.parametrize("k", range(1, 9))
+@pytest.mark.parametrize("n", [5, 255, 257, 1023, 1025, 2305])
+def test_batch_columns_per_lane(cuda, n, k):
+    """1 to 8 right-hand sides (one, two or four columns per lane, whole vectors and shifted last
+    ones) at the edges of tiles and segments, with rows longer than a gather chunk and a segment
+    that does not fit its staging buffer, in both precisions.  A = I + W, |W| <= 1/2 in every row,
+    so the condition number is at most 3.  FP64: 8 fixed iterations against the oracle; their
+    rounding (about sqrt(n) eps an iteration, times the condition number) is below 1e-12.
+    Mixed: stopped on the FP64 residual at 1e-11, so the error is at most 3e-11 of the solution
+    (||x - x*|| <= ||A^-1|| ||r||, ||b|| <= 1.5 ||x*||, ||A^-1|| <= 2)."""
+    rng = np.random.default_rng(100 * n + k)
+    cnt = 3 * n
+    W = sp.coo_matrix((rng.uniform(-1, 1, cnt), (rng.integers(0, n, cnt), rng.integers(0, n, cnt))), shape=(n, n)).tolil()
+    if n > 1000:
+        W[300:310, :260] = 0.01  # ten rows of 260: more than a segment's share
+    W = sp.csr_matrix(W)
+    W = W + W.T
+    A = (sp.identity(n) + W * (0.5 / max(1.0, float(abs(W).sum(1).max())))).tocsr()
+    A.sort_indices()
+    csr = (A.indptr.astype(np.int64), A.indices.astype(np.int32), A.data)
+    B = gen.uniform(31 * n + k, n * k).reshape(n, k)
+    d = 1.0 / A.diagonal()
+    sysl = [(*csr, d, B, n, k)]
+    Xo = np.zeros((n, k))
+    oracle.cg(n, *csr, B, Xo, k, 8, 0.0, prec_diag=d if n % 3 else None)
+    bt = BatchCG()
+    devs = to_dev(sysl[0], cuda)
+    bt.add(*devs[:3], devs[4], devs[5], 0.0, 8, diag=devs[3] if n % 3 else None)
+    bt.run(4)
+    bt.close()
+    assert rel_err(devs[5].cpu().numpy(), Xo) <= 1e-12
+    X, res = run_batch(sysl, cuda, 1, 1e-11)
+    assert res[0]["succeeded"] and rel_err(X[0], np.linalg.solve(A.toarray(), B)) <= 3e-11

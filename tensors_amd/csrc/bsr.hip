@@ -31,7 +31,7 @@ namespace tg {
 enum BsrBeta : int { kBsrBetaZero = 0, kBsrBetaOne = 1, kBsrBetaGeneric = 2 };
 
 // 1: row-major X / Y chunks use bsr_spmm_vec_kernel (lane = block row x V
-// right-hand sides); 0: every storage order uses bsr_spmm_kernel (lane = entry).
+// right-hand sides) or bsr_staged_kernel (blocks through LDS); 0: every storage order uses bsr_spmm_kernel (lane = entry).
 static int g_bsr_vector = 1;
 
 int bsr_tune_set(const char* key, int32_t value, bool* known) {
@@ -198,6 +198,163 @@ __global__ __launch_bounds__(kBlock) void bsr_spmm_vec_kernel(int mb, int R, int
     }
 }
 
+// Square blocks of side 2, 3, 4, 6 or 8 with row-major chunks.  A group of block rows takes
+// its blocks, which lie one after the other in memory, through LDS in chunks of `cap`
+// blocks: coalesced loads, each line touched once.  (The kernel above reads a block's rows
+// where they lie: lanes 72 bytes apart for 3 x 3 doubles, and by the next block the L1 has
+// lost the lines.)  A lane then owns PR rows and V columns of its row's chunk of Y: it loads
+// the B x V piece of X once for PR rows, UB blocks in flight, and A comes from LDS, where
+// blocks are BS elements apart, an odd number, so that the lanes' rows spread over the
+// banks.  Sums in the order of the kernel above.  What bounds it is the chain rp, blocks, X, X
+// of a group against the bytes that lie in LDS meanwhile (about 40 MB on the chip at any LDS per
+// group), so the X of a lane's first blocks is loaded together with the blocks: 96^3 rows of
+// 3 x 3 doubles, k = 4 (637 MB): 191 us before, 193 staged, 158 with that (4.0 TB/s).
+// `rows` block rows a workgroup (blockDim.x >= rows * lanes), lanes = (B / PR) * ceil(k / V);
+// where V does not divide k the last lane's columns start at k - V and it writes its own.
+template <typename T, int B, int V, bool A_RM>
+__global__ __launch_bounds__(kBlock) void bsr_staged_kernel(int mb, int k, const void* __restrict__ rp, int rp64,
+                                                            const int32_t* __restrict__ ci, const T* __restrict__ A,
+                                                            T alpha, const T* __restrict__ X, T beta,
+                                                            T* __restrict__ Y, int rows, int lanes, int cap,
+                                                            int alpha_one, int beta_mode) {
+    constexpr int BB = B * B, BS = BB | 1, PR = B <= 3 ? B : 2, UB = B <= 3 ? 4 : B == 4 ? 2 : 1;
+    constexpr int VA = 16 / sizeof(T), LB = 8;  // elements per staging load, loads in flight
+    extern __shared__ __align__(16) char lds[];
+    T* as = (T*)lds;
+    int32_t* cs = (int32_t*)(as + (int64_t)cap * BS);
+    const auto at = [&](int i) { return rp64 ? ((const int64_t*)rp)[i] : (int64_t)((const int32_t*)rp)[i]; };
+    const int i0 = xcd_swizzle(blockIdx.x, gridDim.x) * rows, i1 = min(i0 + rows, mb);
+    const int kv = (k + V - 1) / V;
+    const int row = threadIdx.x / lanes, part = threadIdx.x % lanes;
+    const int i = i0 + row;
+    const bool on = row < rows && i < i1;
+    const int r0 = part / kv * PR, hv = part % kv * V, h0 = min(hv, k - V), own = hv - h0;
+    const int64_t first = at(i0), end = at(i1);
+    const int64_t lo = on ? at(i) : 0, hi = on ? at(i + 1) : 0;
+    T acc[PR][V] = {};
+    for (int64_t q0 = first; q0 < end; q0 += cap) {
+        const int nq = (int)min((int64_t)cap, end - q0), len = nq * BB;
+        const T* Aq = A + q0 * BB;
+        for (int t = threadIdx.x; t < nq; t += blockDim.x) cs[t] = ci[q0 + t];
+        // the lane's blocks in the chunk; the X of its first ones is on its way with the blocks
+        const int a = on ? (int)(max(lo, q0) - q0) : 0, b = on ? (int)(min(hi, q0 + nq) - q0) : 0;
+        T x[UB][B][V];
+        auto fetch = [&](const int32_t (&j)[UB]) {
+#pragma unroll
+            for (int u = 0; u < UB; ++u) {
+                const T* xp = X + (int64_t)j[u] * B * k + h0;
+#pragma unroll
+                for (int c = 0; c < B; ++c) load_vec_at<T, V>(xp + c * k, x[u][c]);
+            }
+        };
+        int32_t j[UB];
+        if (a < b) {
+#pragma unroll
+            for (int u = 0; u < UB; ++u) j[u] = ci[q0 + min(a + u, b - 1)];
+        }
+        for (int e0 = threadIdx.x * VA; e0 < len; e0 += LB * VA * blockDim.x) {
+            T v[LB][VA];
+#pragma unroll
+            for (int u = 0; u < LB; ++u)  // the last one overlaps (len >= VA)
+                load_vec_at<T, VA>(Aq + min(e0 + u * VA * (int)blockDim.x, len - VA), v[u]);
+            if (e0 == (int)threadIdx.x * VA && a < b) fetch(j);
+#pragma unroll
+            for (int u = 0; u < LB; ++u) {
+                const int e = min(e0 + u * VA * (int)blockDim.x, len - VA);
+#pragma unroll
+                for (int w = 0; w < VA; ++w) as[(e + w) / BB * BS + (e + w) % BB] = v[u][w];
+            }
+        }
+        if ((int)threadIdx.x * VA >= len && a < b) fetch(j);
+        __syncthreads();
+        for (int kb = a; kb < b; kb += UB) {
+            if (kb > a) {
+#pragma unroll
+                for (int u = 0; u < UB; ++u) j[u] = cs[min(kb + u, b - 1)];
+                fetch(j);
+            }
+#pragma unroll
+            for (int u = 0; u < UB; ++u) {
+                const T* ap = as + min(kb + u, b - 1) * BS;
+                const bool have = kb + u < b;
+#pragma unroll
+                for (int r = 0; r < PR; ++r) {
+                    T sum[V] = {};
+#pragma unroll
+                    for (int c = 0; c < B; ++c) {
+                        const T av = ap[A_RM ? (r0 + r) * B + c : c * B + r0 + r];
+#pragma unroll
+                        for (int v = 0; v < V; ++v) sum[v] += av * x[u][c][v];
+                    }
+#pragma unroll
+                    for (int v = 0; v < V; ++v) acc[r][v] += have ? sum[v] : T(0);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (!on) return;
+    T* yp = Y + ((int64_t)i * B + r0) * k + h0;
+#pragma unroll
+    for (int r = 0; r < PR; ++r) {
+        T y[V];
+        if (beta_mode != kBsrBetaZero) load_vec_at<T, V>(yp + r * k, y);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            T out = alpha_one ? acc[r][v] : alpha * acc[r][v];
+            if (hi == lo) out = T(0);  // WriteYZero: Y_i <- beta Y_i
+            if (beta_mode == kBsrBetaOne)
+                out = hi == lo ? y[v] : out + y[v];
+            else if (beta_mode == kBsrBetaGeneric)
+                out = hi == lo ? beta * y[v] : out + beta * y[v];
+            y[v] = out;
+        }
+        if (own == 0) {
+            store_vec_at<T, V>(yp + r * k, y);
+        } else {
+#pragma unroll
+            for (int v = 1; v < V; ++v)
+                if (v >= own) yp[r * k + v] = y[v];
+        }
+    }
+}
+
+// The launch of bsr_staged_kernel: 20 KB of LDS a workgroup (12 / 16 / 20 / 24 / 32 / 40 KB,
+// the case above: 204 / 172 / 158 / 158 / 160 / 163 us; with 12 or 16 too few lanes of a wave
+// have rows), block rows for as many blocks of the mean row (and one more) as that holds, at
+// most 256 lanes, in whole waves where there is more than one.
+template <typename T, int B>
+static int launch_bsr_staged(int mb, int64_t nnzb, int k, const void* rp, int rp64, const int32_t* ci, const T* A,
+                             int a_rm, T alpha, const T* X, T beta, T* Y, int alpha_one, int beta_mode, hipStream_t s) {
+    constexpr int BS = B * B | 1, PR = B <= 3 ? B : 2, bytes = BS * (int)sizeof(T) + 4;
+    int V = (int)(16 / sizeof(T));
+    while (V > k) V /= 2;
+    const int lanes = B / PR * ((k + V - 1) / V);
+    const int64_t mean = (nnzb + mb - 1) / mb + 1;
+    int cap = 20 * 1024 / bytes;
+    int rows = (int)std::max<int64_t>(1, std::min<int64_t>(kBlock / lanes, cap / mean));
+    if (rows * lanes > kWave) rows = rows * lanes / kWave * kWave / lanes;
+    cap = (int)std::min<int64_t>(cap, std::max<int64_t>(rows * mean, 8));
+    const int threads = (rows * lanes + kWave - 1) / kWave * kWave;
+    const dim3 grid((unsigned)((mb + rows - 1) / rows));
+    const size_t shared = (size_t)cap * bytes;
+#define TG_BSRS(VV)                                                                                                      do {                                                                                                                     if (a_rm)                                                                                                                hipLaunchKernelGGL((bsr_staged_kernel<T, B, VV, true>), grid, dim3(threads), shared, s, mb, k, rp, rp64,                                ci, A, alpha, X, beta, Y, rows, lanes, cap, alpha_one, beta_mode);                            else                                                                                                                     hipLaunchKernelGGL((bsr_staged_kernel<T, B, VV, false>), grid, dim3(threads), shared, s, mb, k, rp,                                     rp64, ci, A, alpha, X, beta, Y, rows, lanes, cap, alpha_one, beta_mode);                  } while (0)
+    if constexpr (sizeof(T) == 4) {
+        if (V == 4) {
+            TG_BSRS(4);
+            TG_LAUNCH_CHECK();
+            return TG_OK;
+        }
+    }
+    if (V == 2)
+        TG_BSRS(2);
+    else
+        TG_BSRS(1);
+#undef TG_BSRS
+    TG_LAUNCH_CHECK();
+    return TG_OK;
+}
+
 // Y <- beta Y over `count` entries (beta == 0: zero, NaN-free).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void bsr_scale_kernel(int64_t count, T beta, int beta_mode, T* __restrict__ Y) {
@@ -274,6 +431,35 @@ static int bsr_typed(int32_t mb, int64_t nnzb, int32_t R, int32_t C, const RP* r
         return TG_OK;
     }
     const int alpha_one = alpha_d == 1.0;
+    // Staged blocks where bsr_spmm_vec_kernel reads narrow vectors or leaves lanes of its
+    // groups idle: k % 4 != 0 (200 000 / B rows of 7 blocks, old against staged, factors
+    // 1.1-2.5 for k = 5, 6, 7 and every B; k = 3: FP64 1.2-1.9 up to B = 6 and 0.86 at B = 8, FP32
+    // 1.1-1.4 up to B = 3 and 0.96-1.05 above; k = 1, 2: 0.7-1.0, not taken), three FP64 block
+    // rows (k = 4 1.15, 8 1.3, 16 1.4), B = 6 from k = 8 (1.1-2.1), B = 4 and 8 from k = 16
+    // (1.1-1.7), B = 2 with four FP32 columns (1.15); in the rest it loses (B = 2, k = 16 0.8; B = 4
+    // or 8, k = 4 0.7-0.9).  Rows of 1-2 blocks mean reading past them (0.6-1.2), rows of 27 leave
+    // a workgroup few rows (0.5-1.7), and with fewer than 32768 blocks the chip is not full and the
+    // longer chain shows (300 rows of 27: 0.6-1.1).
+    const bool fp64 = sizeof(T) == 8;
+    const bool narrow = k % 4 != 0 ? k >= 5 || (k == 3 && R <= (fp64 ? 6 : 3))
+                        : R == 2   ? k == 4 && !fp64
+                        : R == 3   ? fp64
+                                   : k >= (R == 6 ? 8 : 16);
+    const bool staged = narrow && k <= 64 && nnzb >= 32768 && nnzb >= 4 * (int64_t)mb && nnzb <= 16 * (int64_t)mb;
+    if (x_rm && y_rm && g_bsr_vector && R == C && staged) {
+#define TG_BSR_STAGED(BB)                                                                                             \
+    case BB:                                                                                                          \
+        return launch_bsr_staged<T, BB>(mb, nnzb, k, rp, sizeof(RP) == 8, ci, A, a_rm, alpha, X, beta, Y, alpha_one, \
+                                        beta_mode, s)
+        switch (R) {
+            TG_BSR_STAGED(2);
+            TG_BSR_STAGED(3);
+            TG_BSR_STAGED(4);
+            TG_BSR_STAGED(6);
+            TG_BSR_STAGED(8);
+        }
+#undef TG_BSR_STAGED
+    }
     if (x_rm && y_rm && g_bsr_vector) {  // lane = (block row r, V right-hand sides)
         const auto aligned = [&](int bytes) {
             return (uintptr_t)X % bytes == 0 && (uintptr_t)Y % bytes == 0;

@@ -140,3 +140,43 @@ def test_fill_lower_matches_oracle(cuda, R):
         K.FillLowerTriangleFromUpperTriangle(Ad)
         exp = Ao if dtype == torch.float64 else Ao.astype(np.float32)
         assert np.array_equal(Ad.cpu().numpy(), exp)
+
+
+@pytest.mark.parametrize("B", [2, 3, 4, 6, 8])
+@pytest.mark.parametrize("k", [3, 4, 5, 8, 16, 61])
+@pytest.mark.parametrize("a_rm", [1, 0])
+def test_bsr_staged_blocks_equal_entry_mapping(cuda, B, k, a_rm):
+    """Blocks through LDS (square blocks, many rows) against the entry mapping (knob bsr_vector =
+    0): integer data, so both are exact and equal bit for bit.  Rows of 0 to 12 blocks and one longer
+    than a chunk, the last group short, k with whole and shifted last vectors, X and Y at odd
+    element offsets, every beta mode, both row-pointer types and value types."""
+    from tensors_amd import _capi as capi
+
+    rng = np.random.default_rng(10 * B + k)
+    mb, nb = 6001, 4000
+    cnt = rng.integers(0, 13, mb)
+    cnt[1234] = 1500
+    rp = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int64)
+    assert rp[-1] >= 32768
+    ci = np.concatenate([np.sort(rng.choice(nb, c, replace=False)) for c in cnt]).astype(np.int32)
+    A = torch.from_numpy(rng.integers(-4, 5, int(rp[-1]) * B * B)).to(cuda)
+    X = torch.from_numpy(rng.integers(-4, 5, nb * B * k)).to(cuda)
+    Y0 = torch.from_numpy(rng.integers(-4, 5, mb * B * k)).to(cuda)
+    K = KernelMatrixCSR(rp if k % 2 else rp.astype(np.int32), ci, mb, nb, B, B, a_rm, 1, 1)
+
+    def odd(t, dtype):
+        return torch.cat([t.new_zeros(1), t]).to(dtype)[1:]
+
+    before = int(capi.lib().tg_tune_get(b"bsr_vector"))
+    try:
+        for dtype in (torch.float64, torch.float32):
+            for alpha, beta in [(1.0, 0.0), (2.0, 1.0), (-1.0, 0.5)]:
+                out = []
+                for form in (1, 0):
+                    capi.call("tg_tune_set", b"bsr_vector", form)
+                    Y = odd(Y0, dtype)
+                    assert K.Dot(odd(A, dtype), alpha, odd(X, dtype), beta, Y, k) == 0
+                    out.append(Y)
+                assert torch.equal(*out), (dtype, alpha, beta)
+    finally:
+        capi.call("tg_tune_set", b"bsr_vector", before)

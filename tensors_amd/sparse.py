@@ -21,8 +21,11 @@ _TORCH_TO_TG = {torch.float64: capi.F64, torch.float32: capi.F32}
 
 
 def stream_handle(stream=None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if torch.cuda.is_initialized():  # the handle alone, no Stream object built: 2.6 of a small product's 9 us
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _eprint(msg: str) -> None:

@@ -340,3 +340,24 @@ def test_narrow_bands_take_no_slices(cuda):
         assert A.Plan().uses_split(v, 2) == sliced and (A.Plan().slices(torch.float64, 2) > 0) == sliced
         want = (np.arange(3 * n) % 5 - 2.0).reshape(n, 3).sum(1)
         assert np.array_equal(Y.cpu().numpy(), np.stack([want, want], 1))
+
+
+def test_stream_handle_is_the_current_stream(cuda):
+    """Products go to torch's current stream: the default one, a `with torch.cuda.stream` block's
+    (nested, and of each thread), or the one passed."""
+    import threading
+
+    from tensors_amd.sparse import stream_handle
+
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    default = torch.cuda.current_stream().cuda_stream
+    assert stream_handle() == default and stream_handle(a) == a.cuda_stream
+    seen = []
+    with torch.cuda.stream(a):
+        t = threading.Thread(target=lambda: seen.append(stream_handle()))
+        t.start()
+        t.join()
+        with torch.cuda.stream(b):
+            assert stream_handle() == b.cuda_stream and stream_handle(a) == a.cuda_stream
+        assert stream_handle() == a.cuda_stream
+    assert stream_handle() == default and seen == [default]

@@ -202,7 +202,7 @@ __device__ __forceinline__ void sys_totals(const double* const (&part)[NT], int 
 // tiles the bytes (2 039 tiles of 64 mixed systems of 1e3 to 2e5 rows and 1 to 8 columns,
 // FP32: direction 196 MB in 48 -> 44 us, product 160 MB in 64 -> 53, update 118 MB in
 // 30 us), with few the longest tile's passes (850 tiles: 19, 38, 14 -> 17, 21, 14 us; 182
-// tiles: 8.4, 14, 6.2 -> 6.2, 7.4, 4.3).  64 systems to 1e-8: 170 -> 147 ms.
+// tiles: 8.4, 14, 6.2 -> 6.2, 7.4, 4.3).  64 systems to 1e-10: 170 -> 147 ms.
 struct Cols {
     int c0;   // first column loaded
     int own;  // columns c0 + own ... c0 + V - 1 are this lane's (V: none, the lane is idle)

@@ -675,11 +675,11 @@ __global__ __launch_bounds__(kBlock) void gb_dstep2_kernel(const GbTile* __restr
 // A system that stops here gets a q_j and a next vector it does not need: the other tiles
 // do not know.  Each reads its basis vectors once; what bounds them is the chain of memory
 // round trips in a tile (the product's entries, u at the columns, the vectors, the totals) more
-// than the bytes, which lie in the Infinity Cache: 64 systems of 50^2..150^2 (6e5 rows),
+// than the bytes, which lie in the Infinity Cache: 64 systems of 100^2 (6.4e5 rows),
 // 17 to 30 vectors: 34 + 17 us a step (dstep1 and dstep2 before: 43 + 43).
-// 512 threads per workgroup take a tile's 1024 rows in two sub-tiles.  Of 256 and 1024,
-// cycles of the 64 systems: 47.2 ms / 45.9 / 49.3 (one workgroup of 1024 per CU has
-// nothing to run while it waits); of 8 systems 12.5 / 10.9 / 10.9, where tiles are few.
+// 512 threads per workgroup take a tile's 1024 rows in two sub-tiles.  With 256 / 512 / 1024
+// threads the 64 systems take 47.2 / 45.9 / 49.3 ms (one workgroup of 1024 per CU has
+// nothing to run while it waits), 8 systems, with few tiles, 12.5 / 10.9 / 10.9.
 constexpr int kOneDotsBlock = 512;
 
 template <int NB>

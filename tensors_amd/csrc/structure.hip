@@ -181,9 +181,9 @@ static size_t triples_ws(int64_t count, int32_t m, int symmetrize, char* base, T
 //               entries to the bucket's place of a temporary, row starts within the bucket
 //   bk_offsets  scan of the merged counts
 //   bk_out      copies each bucket's entries to the result and writes its row pointers
-// The same case takes 380 us: clear and count
-// 36, deal 109 (shuffled triples 273), sort 136, copy 33.  A bucket that does not fit (more than kBkCap triples, or a
-// row of more than kBkRow) raises a flag, and the radix form runs instead.
+// The same case takes 380 us: clear and count 36, deal 109 (shuffled triples 273), sort
+// 136, copy 33.  A bucket that does not fit (more than kBkCap triples, or a row of more than
+// kBkRow) raises a flag, and the radix form runs instead.
 // ---------------------------------------------------------------------------
 constexpr int kBkThreads = 1024;
 constexpr int kBkCap = 3072;        // triples of a bucket (75 KB of LDS: two workgroups a CU)

@@ -333,7 +333,7 @@ static int launch_bsr_staged(int mb, int64_t nnzb, int k, const void* rp, int rp
     const int64_t mean = (nnzb + mb - 1) / mb + 1;
     int cap = 20 * 1024 / bytes;
     int rows = (int)std::max<int64_t>(1, std::min<int64_t>(kBlock / lanes, cap / mean));
-    if (rows * lanes > kWave) rows = rows * lanes / kWave * kWave / lanes;
+    if (rows * lanes > kWave) rows = std::max(1, rows * lanes / kWave * kWave / lanes);
     cap = (int)std::min<int64_t>(cap, std::max<int64_t>(rows * mean, 8));
     const int threads = (rows * lanes + kWave - 1) / kWave * kWave;
     const dim3 grid((unsigned)((mb + rows - 1) / rows));

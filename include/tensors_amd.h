@@ -194,7 +194,9 @@ int tg_csr_spmm_plan(tg_csr_plan_t plan, const void* a, tg_dtype val_type, doubl
  *                  update, SpMM and p.u in one kernel plus one vector kernel and
  *                  nothing between them, 3 = default (form 2 for blocks of up to
  *                  2^20 entries n * nrhs, 2^21 with at most 4 right-hand sides;
- *                  form 1 above).  Results agree to rounding.
+ *                  form 1 above, and for 5 and more right-hand sides, odd numbers
+ *                  first, from about 2^19 entries on where form 2's workgroups
+ *                  would make many passes).  Results agree to rounding.
  *   "cg_panel":    rows of that iteration's SpMM kernel, 1 = panel order where
  *                  the band allows (default: the rows cut into panels of one band,
  *                  every workgroup taking the same offsets of each panel, so a row's

@@ -938,8 +938,9 @@ size_t cg_workspace_bytes(int32_t n, int32_t k, size_t vs, int prec_kind, int sl
 // Iteration form for CSR operators with P = I or Jacobi, short rows (mean length
 // <= 16) and no column slabs ("cg_fused"): 0 = four vector kernels after the
 // SpMM; 1 = p.u in the SpMM epilogue (kSpmmDot); 2 = direction, SpMM and p.u in
-// one kernel (kFormDir); 3 = default (form 2 up to 2^20 entries n * nrhs, and up to 2^21
-// with at most 4 right-hand sides; form 1 above).  On the 128^3 Laplacian with 32 right-hand sides form 1 measured fastest in
+// one kernel (kFormDir); 3 = default (form 2 up to 2^20 entries n * nrhs unless its workgroups
+// would make many passes over the rows, and up to 2^21 with at most 4 right-hand sides; form
+// 1 above).  On the 128^3 Laplacian with 32 right-hand sides form 1 measured fastest in
 // FP64 and FP32: gathering both z and p_prev per nonzero (form 2) cost more than
 // streaming p once; on small blocks form 2's two launches instead of five win.  Other
 // operators always take form 0.
@@ -1031,14 +1032,31 @@ static void dir_shape(int k, size_t vs, int& V, int& G) {
     while (G < 64 && G * V < k) G *= 2;
 }
 
-// Workgroups of form 2's kernels: one pass over the rows each where that gives few
-// enough, and at most 1024 and 8192 / k (each workgroup adds all of the other kernel's
-// partials, B k values, before it starts).
-static int fused_blocks(int n, int k, size_t vs) {
+// Rows that a workgroup of K1 takes in one pass, and the passes that `blocks` of them make
+// (column tiles counted).
+static int dir_rows(int k, size_t vs) {
     int V, G;
     dir_shape(k, vs, V, G);
-    const int per = kBlock / G;
-    const int most = std::min(kFusedBlocks / 2, std::max(256, 4096 / k));
+    return kBlock / G;
+}
+
+static double dir_passes(int n, int k, size_t vs, int blocks) {
+    int V, G;
+    dir_shape(k, vs, V, G);
+    return (double)n / ((double)blocks * dir_rows(k, vs)) * ((k + G * V - 1) / (G * V));
+}
+
+// Workgroups of form 2's kernels: one pass over the rows each where that gives few enough,
+// and at most max(256, 4096 / k), at most 1024: each workgroup adds all of the other
+// kernel's partials, B k values, before it starts.  512 instead of 256 where 256 would make
+// more than k / 4 passes (at least four) over the rows: a pass is a chain of round trips
+// too.  256 / 512 workgroups, us an iteration, FP64: 17 columns, 29791 rows (14 passes) 52 /
+// 43; 16, 64000 (8) 40 / 35, 15625 (2) 20 / 21; 33, 32768 (32) 101 / 78, 4096 (4) 27 / 32;
+// 128, 8000 (8) 53 / 62.
+static int fused_blocks(int n, int k, size_t vs) {
+    const int per = dir_rows(k, vs);
+    const int floor = (double)n / (256.0 * per) > std::max(4.0, k / 4.0) ? 512 : 256;
+    const int most = std::min(kFusedBlocks / 2, std::max(floor, 4096 / k));
     return std::max(1, std::min(most, (n + per - 1) / per));
 }
 
@@ -1119,12 +1137,19 @@ int cg_solve_t(const CsrView& A, const OpRef& Aop, int prec_kind, const T* d, co
                         Ac.val_type == (sizeof(T) == 8 ? TG_F64 : TG_F32);
     // auto: form 2 (two launches per iteration) for small blocks, where an iteration is
     // bound by the kernels' latency; form 1 (five, its SpMM gathers one vector instead of
-    // two) above.  Measured, form 2 / form 1 a solve: 45^3 x 8 16.1 / 18.8 ms, 90^3 x 2
-    // 15.5 / 17.7, 110^3 x 1 22.5 / 27.3, 80^3 x 4 17.7 / 18.0, 64^3 x 8 37.8 / 36.6, 45^3 x 16
-    // 14.9 / 13.0, 128^3 x 1 (2^21 entries) 31.9 / 35.6.
+    // two) above, and from five columns on where form 2's few workgroups would make many
+    // passes over the rows (odd numbers of columns: a lane per column).  Measured, form 2 /
+    // form 1 a solve: 45^3 x 8 16.1 / 18.8 ms, 90^3 x 2 15.5 / 17.7, 110^3 x 1 22.5 / 27.3,
+    // 80^3 x 4 17.7 / 18.0, 64^3 x 8 37.8 / 36.6, 128^3 x 1 (2^21 entries) 31.9 / 35.6; an
+    // iteration in us, FP64, Jacobi, at about 2^20 entries: 5 columns (8 passes) 66 / 52, 9 (14)
+    // 75 / 56, 17 (16) 80 / 62, 19 (13) 74 / 61, 25 (10) 63 / 57, 65 (31) 102 / 99, and at
+    // 2^19: 5 (4) 43 / 40, 9 (7) 46 / 43, 17 (7) 49 / 48, 33 (8) 56 / 62, 65 (16) 65 / 88.
+    // More columns move the line up: form 1's one-workgroup kernels grow with them.
     const int64_t entries = (int64_t)n * k;
     const bool small = entries <= (int64_t(1) << 20) || (k <= 4 && entries <= (int64_t(1) << 21));
-    int form = g_cg_fused == kFormAuto ? (small ? kFormDir : kSpmmDot) : g_cg_fused;
+    const bool few_passes =
+        k <= 4 || dir_passes(n, k, sizeof(T), fused_blocks(n, k, sizeof(T))) <= 4 + k * (k < 16 ? 0.25 : 0.45);
+    int form = g_cg_fused == kFormAuto ? (small && few_passes ? kFormDir : kSpmmDot) : g_cg_fused;
     if (!csr_ok) form = kFourKernels;
     const bool fused = form == kFormDir;
     // deferred x update: form 1 only (form 0's operator reads p at a fixed address, form 2

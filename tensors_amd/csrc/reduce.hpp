@@ -95,25 +95,39 @@ __device__ __forceinline__ double column_total(const double* partial, int B, int
 
 // Totals of B workgroup partials per column, in a fixed order, by a workgroup of kBlock
 // threads that needs them itself: out[0 .. k) in LDS (scratch: kBlock doubles of LDS).
-// Thread (c, j) adds partials j, j + J, ... into four running sums, the lanes of a wave
-// and then the waves are combined in a fixed tree, so every workgroup that calls it gets
-// bitwise the same totals.  Saves the one-workgroup kernel between two passes where B k
-// is small enough (a few thousand values) for every workgroup to read.
+// Thread (c, j) adds partials j, j + J, ... into four or eight running sums, the lanes of a
+// wave and then the waves are combined in a fixed tree, so every workgroup that calls it
+// gets bitwise the same totals.  Saves the one-workgroup kernel between two passes where
+// every workgroup can read the B k values.  What bounds it is the round trips of a thread's
+// B / J partials, so more than four of them are read eight at a time, at clamped places (no
+// branch between the loads): CG iterations of 10^3 rows and 256 columns, B = 250: 103 us
+// with four at a time and branches, 49 so; 12^3 and 192: 105 / 52.  Up to four per thread
+// (one to four columns) the conditional loads are the shorter form (96^3 rows, one column,
+// an iteration 31.4 against 32.4 us).
 __device__ __forceinline__ void block_totals(const double* __restrict__ partial, int B, int k, int kpad, double* out,
                                              double* scratch) {
     const int c = threadIdx.x % kpad, j = threadIdx.x / kpad, J = kBlock / kpad;
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-    if (c < k) {
-        int b = j;
-        for (; b + 3 * J < B; b += 4 * J) {
+    double t = 0.0;
+    if (B > 4 * J) {
+        constexpr int U = 8;
+        double s[U] = {};
+        if (c < k)
+            for (int b = j; b < B; b += U * J) {
+                double w[U];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) s[q] += partial[(int64_t)(b + q * J) * k + c];
-        }
+                for (int q = 0; q < U; ++q) w[q] = partial[(int64_t)min(b + q * J, B - 1) * k + c];
 #pragma unroll
-        for (int q = 0; q < 3; ++q)  // fewer than 4 left
-            if (b + q * J < B) s[q] += partial[(int64_t)(b + q * J) * k + c];
+                for (int q = 0; q < U; ++q)
+                    if (b + q * J < B) s[q] += w[q];
+            }
+        t = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    } else if (c < k) {
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (j + q * J < B) s[q] = partial[(int64_t)(j + q * J) * k + c];
+        t = (s[0] + s[1]) + (s[2] + s[3]);
     }
-    double t = (s[0] + s[1]) + (s[2] + s[3]);
     for (int off = kWave / 2; off >= kpad; off >>= 1) t += shfl_xor(t, off);
     scratch[threadIdx.x] = t;
     __syncthreads();

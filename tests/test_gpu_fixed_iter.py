@@ -132,6 +132,17 @@ def test_cg_two_kernel_form_ragged_rows(cuda, fused_knob, n, k, prec):
     assert res_err(cg.RelativeResiduals(), rr_o) <= TOL
 
 
+@pytest.mark.parametrize("form,n,k", [(2, 1501, 179), (2, 2003, 256), (2, 701, 130), (2, 9001, 17), (2, 17011, 33),
+                                      (3, 90001, 9), (3, 30011, 33)])
+@pytest.mark.parametrize("prec", [False, True], ids=["identity", "jacobi"])
+def test_cg_two_kernel_form_wide_blocks(cuda, fused_knob, form, n, k, prec):
+    """Wide and odd blocks: more than four partials per thread in the totals (read eight at a
+    time, the last ones clamped), twice the workgroups where 256 would make many passes, and
+    default-form blocks on both sides of the line at which many passes send them to the
+    five-launch form.  Same matrices, steps and bar as above."""
+    test_cg_two_kernel_form_ragged_rows(cuda, (lambda _: fused_knob(form)), n, k, prec)
+
+
 @pytest.fixture
 def panel_knob():
     before = int(capi.lib().tg_tune_get(b"cg_panel"))

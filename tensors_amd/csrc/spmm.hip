@@ -123,13 +123,13 @@ __global__ __launch_bounds__(kBlock) void spmv_team_kernel(
         const RP lb = rp[row], le = rpe[row];
         T z = T(0);
         if (a) {
-            for (RP l = lb + lt; l < le; l += TEAM) {
+            for (int64_t l = (int64_t)lb + lt; l < le; l += TEAM) {
                 const int32_t c = __builtin_nontemporal_load(ci + l);
                 const T av = __builtin_nontemporal_load(a + l);
                 z += av * x[(int64_t)c * ldx];
             }
         } else {
-            for (RP l = lb + lt; l < le; l += TEAM) {
+            for (int64_t l = (int64_t)lb + lt; l < le; l += TEAM) {
                 const int32_t c = __builtin_nontemporal_load(ci + l);
                 z += x[(int64_t)c * ldx];
             }
@@ -210,8 +210,10 @@ __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(
         for (int i = threadIdx.x; i < nr * K; i += kBlock) racc[i] = T(0);
         __syncthreads();
         const RP L0 = srp[0], L1 = srp[nr];
-        for (RP cs = L0; cs < L1; cs += CAP) {
+        // (steps by what was done: cs + CAP may lie past 2^31)
+        for (RP cs = L0, step = 0; cs < L1; cs += step) {
             const int cnt = (int)((L1 - cs) < (RP)CAP ? (L1 - cs) : (RP)CAP);
+            step = (RP)cnt;
             int32_t c[ELEMS];
             T av[ELEMS];
 #pragma unroll
@@ -306,15 +308,16 @@ __global__ __launch_bounds__(kBlock) void spmm_wave_kernel(
             T acc[V];
 #pragma unroll
             for (int i = 0; i < V; ++i) acc[i] = T(0);
-            for (RP base = lb; base < le; base += kWave) {
-                const RP e = base + lane;
+            // (steps by what was done: base + kWave may lie past 2^31)
+            for (RP base = lb, step = 0; base < le; base += step) {
+                const int cnt = (int)((le - base) < (RP)kWave ? (le - base) : (RP)kWave);
+                step = (RP)cnt;
                 int32_t myc = 0;
                 T mya = T(0);
-                if (e < le) {
-                    myc = __builtin_nontemporal_load(ci + e);
-                    mya = a ? __builtin_nontemporal_load(a + e) : T(1);
+                if (lane < cnt) {
+                    myc = __builtin_nontemporal_load(ci + base + lane);
+                    mya = a ? __builtin_nontemporal_load(a + base + lane) : T(1);
                 }
-                const int cnt = (int)((le - base) < (RP)kWave ? (le - base) : (RP)kWave);
                 // G steps of S nonzeros cover the 64 loaded pairs.  Steps run in
                 // groups of U without branches inside a group, so the X loads of
                 // a group are all in flight together; the wave-uniform test

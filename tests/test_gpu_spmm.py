@@ -361,3 +361,25 @@ def test_stream_handle_is_the_current_stream(cuda):
             assert stream_handle() == b.cuda_stream and stream_handle(a) == a.cuda_stream
         assert stream_handle() == a.cuda_stream
     assert stream_handle() == default and seen == [default]
+
+
+@pytest.mark.parametrize("m,nrhs,dtype", [(1 << 20, 1, torch.float64), (1 << 20, 3, torch.float64),
+                                          (1 << 20, 8, torch.float32), ((1 << 27) + 3, 2, torch.float32)])
+def test_int32_row_pointers_up_to_the_last_entry(cuda, m, nrhs, dtype):
+    """2^31 - 1 nonzeros under int32 row pointers: the loops over nonzeros step past 2^31 at the
+    end of the last rows unless they count what is left (rows streamed, a row per wave, short
+    rows).  A binary matrix, columns 0 but for the last 3000 entries, integer X: every sum is
+    exact."""
+    nnz = (1 << 31) - 1
+    if torch.cuda.mem_get_info()[0] < (48 << 30):
+        pytest.skip("needs 48 GB of free device memory")
+    rp = torch.arange(m + 1, dtype=torch.int64, device=cuda) * nnz // m
+    ci = torch.zeros(nnz, dtype=torch.int32, device=cuda)
+    ci[nnz - 3000:] = 1
+    X = torch.arange(1, 2 * nrhs + 1, dtype=dtype, device=cuda).reshape(2, nrhs)
+    Y = torch.full((m, nrhs), -1.0, dtype=dtype, device=cuda)
+    print(f"2^31 - 1 nonzeros, {m} rows, {nrhs} columns", flush=True)
+    assert spmm_raw(m, 2, nnz, rp.to(torch.int32), ci, None, 1.0, X, nrhs, 0.0, Y, nrhs, nrhs) == 0
+    ones = (rp[1:] - rp[:-1].clamp(min=nnz - 3000)).clamp_(min=0)  # entries of a row in column 1
+    want = (rp[1:] - rp[:-1] - ones).to(dtype)[:, None] * X[0] + ones.to(dtype)[:, None] * X[1]
+    assert torch.equal(Y, want)

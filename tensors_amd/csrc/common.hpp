@@ -83,6 +83,21 @@ __device__ __forceinline__ void store_vec_at(T* __restrict__ p, const T* in) {
     }
 }
 
+// Sum of p[l K] for l = lb, lb + TEAM, ... < le, in four running sums: four reads in
+// flight, and a rounding error that grows with a quarter of the terms.
+template <typename T, int TEAM, int K>
+__device__ __forceinline__ T lds_sum(const T* p, int lb, int le) {
+    T s[4] = {T(0), T(0), T(0), T(0)};
+    int l = lb;
+    for (; l + 3 * TEAM < le; l += 4 * TEAM)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] += p[(l + j * TEAM) * K];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+        if (l + j * TEAM < le) s[j] += p[(l + j * TEAM) * K];
+    return (s[0] + s[1]) + (s[2] + s[3]);
+}
+
 template <typename T, int V>
 __device__ __forceinline__ void store_vec(T* __restrict__ p, const T (&in)[V]) {
     if constexpr (V == 1) {

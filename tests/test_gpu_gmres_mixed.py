@@ -131,3 +131,27 @@ def test_mixed_gmres_split_dots_agree(cuda, g, side, prec):
     assert ok1 and ok0 and np.all(rr1 <= 1e-8) and np.all(rr0 <= 1e-8)
     assert r1 >= 1 and abs(r1 - r0) <= 1  # the 32-vector bucket ran (a whole cycle of 30 steps)
     assert rel_err(X1, X0) < 1e-6
+
+
+@pytest.mark.parametrize("n", [12011, 140003])
+def test_fp32_cycle_adds_long_rows_in_parts(cuda, n):
+    """One step of the FP32 cycle for I plus a row of ones, from a constant right-hand side: the
+    rotated H_00 is |A q_0|, nearly all of it the sum of n equal FP32 values.  Added in parts (a
+    wave per row and chunk of 2048 or 4096 products: at most 16 in each of four running sums, 2
+    to join them, 6 levels over the lanes, then one addition a chunk) it is off by at most (24 +
+    chunks) 2^-24 of itself; the vectors around it are rounded to FP32 once or twice.  One
+    running sum is off by 1e-4."""
+    r = n // 3
+    A = (sp.identity(n, format="csr") + sp.csr_matrix((np.ones(n - 1), (np.full(n - 1, r), np.delete(np.arange(n), r))),
+                                                      shape=(n, n))).tocsr()
+    A.sort_indices()
+    gm = GMRES(n, 1, 1, dtype=torch.float32)
+    B = torch.ones(n, 1, dtype=torch.float32, device=cuda)
+    X = torch.zeros_like(B)
+    gm(MatrixCSR(A.indptr.astype(np.int32), A.indices, A.data.astype(np.float32), n, n), None, 1.0, B, 0.0, X, 0.0, 0)
+    q0 = gm.GetBasis()[0, :, 0].double().cpu().numpy()
+    want = np.linalg.norm(A @ q0)
+    got = float(gm.GetHessenbergMatrix()[0, 0, 0])
+    chunks = -(-n // 2048)
+    print(f"FP32 long row n {n}: H_00 off by {abs(got / want - 1):.2e}")
+    assert abs(got / want - 1) <= (24 + chunks + 4) * 2.0 ** -24

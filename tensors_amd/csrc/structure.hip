@@ -92,20 +92,19 @@ __global__ void st_write_kernel(int64_t total, const uint64_t* __restrict__ keys
     }
 }
 
-__global__ void st_nnz_kernel(int64_t total, const int64_t* __restrict__ head, const int64_t* __restrict__ pos,
-                              int64_t* __restrict__ nnz) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) nnz[0] = total > 0 ? pos[total - 1] + head[total - 1] : 0;
-}
-
 template <typename RP>
-__global__ void st_rp_kernel(int32_t m, const int64_t* __restrict__ scanned, RP* __restrict__ rp) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= m; i += (int64_t)gridDim.x * blockDim.x)
+__global__ void st_rp_kernel(int32_t m, const int64_t* __restrict__ scanned, RP* __restrict__ rp,
+                             int64_t* __restrict__ nnz) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i <= m; i += (int64_t)gridDim.x * blockDim.x) {
         rp[i] = (RP)scanned[i];
+        if (i == m) *nnz = scanned[i];
+    }
 }
 
-__global__ void st_zero64_kernel(int64_t count, int64_t* __restrict__ a) {
+__global__ void st_zero64_kernel(int64_t count, int64_t* __restrict__ a, int* __restrict__ flag = nullptr) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
         a[i] = 0;
+    if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
 }
 
 // Bits that hold 0 .. count - 1 (at least one).
@@ -168,6 +167,20 @@ static size_t triples_ws(int64_t count, int32_t m, int symmetrize, char* base, T
     return off;
 }
 
+// The number of entries and the two flags, neighbours in the workspace, in one copy;
+// synchronises s.
+static int triples_found(const TriplesWs& w, int64_t* nnz, int* bad, int* unfit, hipStream_t s) {
+    const size_t span = (size_t)((char*)(w.bad + 2) - (char*)w.nnz);
+    char found[512];
+    if (span > sizeof(found)) return fail(TG_ERR_INVALID, "internal: workspace layout");
+    TG_HIP(hipMemcpyAsync(found, w.nnz, span, hipMemcpyDeviceToHost, s));
+    TG_HIP(hipStreamSynchronize(s));
+    std::memcpy(nnz, found, 8);
+    std::memcpy(bad, found + span - 8, 4);
+    std::memcpy(unfit, found + span - 4, 4);
+    return TG_OK;
+}
+
 // ---------------------------------------------------------------------------
 // Bucket form.  The 64-bit radix sort moved 12 bytes a triple through memory eight times
 // (10.5 M triples of a 96^3 grid's edges: eight passes of 99 us, 1353 us in all).  Here a
@@ -181,9 +194,12 @@ static size_t triples_ws(int64_t count, int32_t m, int symmetrize, char* base, T
 //               entries to the bucket's place of a temporary, row starts within the bucket
 //   bk_offsets  scan of the merged counts
 //   bk_out      copies each bucket's entries to the result and writes its row pointers
-// The same case takes 380 us: clear and count 36, deal 109 (shuffled triples 273), sort
-// 136, copy 33.  A bucket that does not fit (more than kBkCap triples, or a row of more than
-// kBkRow) raises a flag, and the radix form runs instead.
+// The same case takes 345 us (shuffled triples deal in 273).  A bucket that does not fit (more than
+// kBkCap triples, or a row of more than kBkRow) raises a flag, and the radix form runs
+// instead: too many triples before any is dealt, with the kernels that follow returning at
+// once.  Radix form alone (64 bits) / with the attempt in front: 1.05e7 triples with a row of
+// 1e4 1851 / 1646 us, 2e6 602 / 558, 3e5 343 / 390; rows of up to kBkRow stay in the buckets
+// (3e5 triples, one row of 700: 246 / 121 us, of 1400 254 / 165).
 // ---------------------------------------------------------------------------
 constexpr int kBkThreads = 1024;
 constexpr int kBkCap = 3072;        // triples of a bucket (75 KB of LDS: two workgroups a CU)
@@ -191,7 +207,8 @@ constexpr int kBkRowBits = 11;
 constexpr int kBkRows = 1 << kBkRowBits;  // rows of a bucket
 constexpr int kBkIdxBits = 24;      // input positions
 constexpr int kBkColBits = 64 - kBkRowBits - kBkIdxBits;
-constexpr int kBkRow = 512;         // triples of a row (ranked against each other)
+constexpr int kBkRow = 1536;        // triples of a row (ranked against each other)
+constexpr int kBkMeanRow = 128;     // ... on average
 constexpr int kBkMost = 8192;       // buckets
 constexpr int kBkTarget = 1536;     // triples of a bucket on average (up to 2048 where kBkMost binds)
 constexpr int kBkPer = 8;           // triples per thread of a tile
@@ -207,10 +224,12 @@ struct BucketPlan {
 // A triple travels as one word: row in its bucket, column, input position.
 static BucketPlan bucket_plan(int64_t total, int32_t m, int32_t cols) {
     BucketPlan P;
-    if (total < 4096 || m < 1 || total / m > kBkRow / 4 || total > ((int64_t)1 << kBkIdxBits) ||
+    if (total < 4096 || m < 1 || total / m > kBkMeanRow || total > ((int64_t)1 << kBkIdxBits) ||
         cols > ((int64_t)1 << kBkColBits))
         return P;
-    const int64_t target = std::min<int64_t>(kBkTarget, std::max<int64_t>(256, total / 512));  // two a CU if few
+    // two a CU if few (small buckets hold denser ranges of rows: 64 triples on average up to 48
+    // times that)
+    const int64_t target = std::min<int64_t>(kBkTarget, std::max<int64_t>(64, total / 512));
     int64_t nb = std::max((total + target - 1) / target, ((int64_t)m + kBkRows - 1) / kBkRows);
     if (nb > kBkMost && total <= (int64_t)kBkMost * 2048 && m <= (int64_t)kBkMost * kBkRows) nb = kBkMost;
     if (nb > kBkMost || nb * 4 > total) return P;  // the bucket arrays live in 8 bytes a triple
@@ -285,11 +304,17 @@ __global__ __launch_bounds__(kBkThreads) void bk_hist_kernel(int64_t count, int6
         if (h[b]) atomicAdd(&hist[b], h[b]);
 }
 
-// off[0 .. nb] = exclusive scan of cnt[0 .. nb), nb <= kBkMost; cursor (if given) = off.
+// Flags of a run that does not fit, in one word: a bucket of more than kBkCap triples, known
+// before any triple is dealt (the kernels after it then return at once), or a row of more
+// than kBkRow, found while sorting.
+constexpr int kBkCrowded = 1, kBkLongRow = 2;
+
+// off[0 .. nb] = exclusive scan of cnt[0 .. nb), nb <= kBkMost; cursor (if given) = off;
+// unfit (if given): kBkCrowded where a count is more than kBkCap.
 __global__ __launch_bounds__(kBkThreads) void bk_offsets_kernel(int nb, const uint32_t* __restrict__ cnt,
                                                                 uint32_t* __restrict__ off,
                                                                 uint32_t* __restrict__ cursor,
-                                                                int64_t* __restrict__ sum) {
+                                                                int64_t* __restrict__ sum, int* __restrict__ unfit) {
     constexpr int PER = kBkMost / kBkThreads;
     __shared__ uint32_t wsum[kBkThreads / kWave];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
@@ -299,6 +324,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_offsets_kernel(int nb, const ui
         const int b = threadIdx.x * PER + q;
         v[q] = b < nb ? cnt[b] : 0;
         tot += v[q];
+        if (unfit && v[q] > (uint32_t)kBkCap) atomicOr(unfit, kBkCrowded);
     }
     uint32_t inc = tot;
 #pragma unroll
@@ -345,7 +371,9 @@ template <typename T>
 __global__ __launch_bounds__(kBkThreads) void bk_deal_kernel(int64_t count, int64_t total, const int32_t* __restrict__ I,
                                                              const int32_t* __restrict__ J, const T* __restrict__ V,
                                                              int32_t m, int32_t n, int rows, int buckets,
-                                                             uint32_t* __restrict__ cursor, void* __restrict__ out) {
+                                                             uint32_t* __restrict__ cursor, void* __restrict__ out,
+                                                             const int* __restrict__ unfit) {
+    const int stop = *unfit;  // (its load is not waited for here)
     __shared__ uint32_t h[kBkMost];
     for (int b = threadIdx.x; b < buckets; b += kBkThreads) h[b] = 0;
     __syncthreads();
@@ -362,6 +390,7 @@ __global__ __launch_bounds__(kBkThreads) void bk_deal_kernel(int64_t count, int6
         r[q] = on ? rr : -1;
         c[q] = cc;
     }
+    if (stop) return;
     __syncthreads();
     for (int b = threadIdx.x; b < buckets; b += kBkThreads)
         if (h[b]) h[b] = atomicAdd(&cursor[b], h[b]);
@@ -421,17 +450,12 @@ __global__ __launch_bounds__(kBkThreads, 8) void bk_sort_kernel(int32_t m, int r
     __shared__ uint16_t first[kBkCap];                // 1 where an entry starts
     __shared__ uint32_t start[kBkRows + 1], head[kBkCap + 1];
     __shared__ int toolong;
+    const int stop = *unfit & kBkCrowded;  // set in an earlier launch: the same for all
     T* vals = (T*)key;  // the words by row are done with when the values are placed
     const int b = blockIdx.x, r0 = b * rows, nr = min(rows, m - r0);
     const uint32_t base = off[b];
-    const int cnt = (int)min(off[b + 1] - base, (uint32_t)kBkCap + 1);
-    if (cnt > kBkCap) {
-        if (threadIdx.x == 0) {
-            atomicOr(unfit, 1);
-            merged[b] = 0;
-        }
-        return;
-    }
+    const int cnt = (int)(off[b + 1] - base);
+    if (stop) return;
     for (int i = threadIdx.x; i < nr; i += kBkThreads) start[i] = 0;
     if (threadIdx.x == 0) toolong = 0;
     __syncthreads();
@@ -464,7 +488,7 @@ __global__ __launch_bounds__(kBkThreads, 8) void bk_sort_kernel(int32_t m, int r
     __syncthreads();
     if (toolong) {  // block-uniform
         if (threadIdx.x == 0) {
-            atomicOr(unfit, 1);
+            atomicOr(unfit, kBkLongRow);
             merged[b] = 0;
         }
         return;
@@ -516,10 +540,13 @@ __global__ __launch_bounds__(256) void bk_out_kernel(int32_t m, int rows, const 
                                                      const uint32_t* __restrict__ moff,
                                                      const uint32_t* __restrict__ rowoff,
                                                      const int32_t* __restrict__ tci, const T* __restrict__ tval,
-                                                     RP* __restrict__ rp, int32_t* __restrict__ ci, T* __restrict__ val) {
+                                                     RP* __restrict__ rp, int32_t* __restrict__ ci, T* __restrict__ val,
+                                                     const int* __restrict__ unfit) {
+    const int stop = *unfit;
     const int b = blockIdx.x, r0 = b * rows, nr = min(rows, m - r0);
     const uint32_t src = off[b], dst = moff[b];
     const int cnt = (int)(moff[b + 1] - dst);
+    if (stop) return;
     for (int i = threadIdx.x; i < nr; i += 256) rp[r0 + i] = (RP)(dst + rowoff[r0 + i]);
     if (b == (int)gridDim.x - 1 && threadIdx.x == 0) rp[m] = (RP)(dst + cnt);
     for (int t = threadIdx.x; t < cnt; t += 256) {
@@ -528,7 +555,7 @@ __global__ __launch_bounds__(256) void bk_out_kernel(int32_t m, int rows, const 
     }
 }
 
-// The bucket form; *unfit = 1 when a bucket did not fit (nothing useful was written).
+// The bucket form; *unfit != 0 when a bucket did not fit (nothing was written).
 template <typename T>
 static int bucket_triples(const BucketPlan& P, int64_t count, int64_t total, const int32_t* I, const int32_t* J,
                           const T* V, int32_t m, int32_t n, int compress, void* rp_out, tg_dtype rp_type,
@@ -547,32 +574,23 @@ static int bucket_triples(const BucketPlan& P, int64_t count, int64_t total, con
     hipLaunchKernelGGL(bk_hist_kernel, dim3(hgrid), dim3(kBkThreads), 0, s, count, total, I, J, m, n, P.rows, nb, hist,
                        w.bad);
     hipLaunchKernelGGL(bk_offsets_kernel, dim3(1), dim3(kBkThreads), 0, s, nb, (const uint32_t*)hist, off, hist,
-                       (int64_t*)nullptr);
+                       (int64_t*)nullptr, w.bad + 1);
     hipLaunchKernelGGL((bk_deal_kernel<T>), dim3((unsigned)((total + kBkTile - 1) / kBkTile)), dim3(kBkThreads), 0, s,
-                       count, total, I, J, V, m, n, P.rows, nb, hist, items);
+                       count, total, I, J, V, m, n, P.rows, nb, hist, items, (const int*)(w.bad + 1));
     hipLaunchKernelGGL((bk_sort_kernel<T>), dim3(nb), dim3(kBkThreads), 0, s, m, P.rows, (const uint32_t*)off,
                        (const void*)items, V ? 1 : 0, compress, tci, tval, rowoff, hist, w.bad + 1);
     hipLaunchKernelGGL(bk_offsets_kernel, dim3(1), dim3(kBkThreads), 0, s, nb, (const uint32_t*)hist, moff,
-                       (uint32_t*)nullptr, w.nnz);
+                       (uint32_t*)nullptr, w.nnz, (int*)nullptr);
     if (rp_type == TG_I64)
         hipLaunchKernelGGL((bk_out_kernel<T, int64_t>), dim3(nb), dim3(256), 0, s, m, P.rows, (const uint32_t*)off,
                            (const uint32_t*)moff, (const uint32_t*)rowoff, (const int32_t*)tci, (const T*)tval,
-                           (int64_t*)rp_out, ci_out, val_out);
+                           (int64_t*)rp_out, ci_out, val_out, (const int*)(w.bad + 1));
     else
         hipLaunchKernelGGL((bk_out_kernel<T, int32_t>), dim3(nb), dim3(256), 0, s, m, P.rows, (const uint32_t*)off,
                            (const uint32_t*)moff, (const uint32_t*)rowoff, (const int32_t*)tci, (const T*)tval,
-                           (int32_t*)rp_out, ci_out, val_out);
+                           (int32_t*)rp_out, ci_out, val_out, (const int*)(w.bad + 1));
     TG_LAUNCH_CHECK();
-    // the count and the two flags, neighbours in the workspace, in one copy
-    const size_t span = (size_t)((char*)(w.bad + 2) - (char*)w.nnz);
-    char found[512];
-    if (span > sizeof(found)) return fail(TG_ERR_INVALID, "internal: workspace layout");
-    TG_HIP(hipMemcpyAsync(found, w.nnz, span, hipMemcpyDeviceToHost, s));
-    TG_HIP(hipStreamSynchronize(s));
-    std::memcpy(nnz, found, 8);
-    std::memcpy(bad, found + span - 8, 4);
-    std::memcpy(unfit, found + span - 4, 4);
-    return TG_OK;
+    return triples_found(w, nnz, bad, unfit, s);
 }
 
 template <typename T>
@@ -600,8 +618,7 @@ static int from_triples_t(int64_t count, const int32_t* I, const int32_t* J, con
             return TG_OK;
         }
     }
-    hipLaunchKernelGGL(st_zero64_kernel, dim3(grid_of(m + 1)), dim3(256), 0, s, (int64_t)m + 1, w.rowcnt);
-    hipLaunchKernelGGL(st_zero64_kernel, dim3(1), dim3(256), 0, s, (int64_t)1, (int64_t*)w.bad);
+    hipLaunchKernelGGL(st_zero64_kernel, dim3(grid_of(m + 1)), dim3(256), 0, s, (int64_t)m + 1, w.rowcnt, w.bad);
     if (total > 0) {
         // columns and, for transposed copies, rows appear in either half
         const int cb = bits_of(symmetrize ? std::max(m, n) : n), rb = bits_of((int64_t)(symmetrize ? std::max(m, n) : m) + 1);
@@ -619,26 +636,24 @@ static int from_triples_t(int64_t count, const int32_t* I, const int32_t* J, con
                            (const uint64_t*)w.keys[1], (const uint32_t*)w.idx[1], (const int64_t*)w.head,
                            (const int64_t*)w.pos, count, cb, V, compress, ci_out, val_out, w.rowcnt);
     }
-    hipLaunchKernelGGL(st_nnz_kernel, dim3(1), dim3(64), 0, s, total, (const int64_t*)w.head, (const int64_t*)w.pos,
-                       w.nnz);
     size_t tb = w.temp_bytes;
     TG_HIP(rocprim::exclusive_scan(w.temp, tb, (const int64_t*)w.rowcnt, w.rowscan, (int64_t)0, (size_t)m + 1,
                                    rocprim::plus<int64_t>(), s));
     if (rp_type == TG_I64)
         hipLaunchKernelGGL((st_rp_kernel<int64_t>), dim3(grid_of(m + 1)), dim3(256), 0, s, m,
-                           (const int64_t*)w.rowscan, (int64_t*)rp_out);
+                           (const int64_t*)w.rowscan, (int64_t*)rp_out, w.nnz);
     else
         hipLaunchKernelGGL((st_rp_kernel<int32_t>), dim3(grid_of(m + 1)), dim3(256), 0, s, m,
-                           (const int64_t*)w.rowscan, (int32_t*)rp_out);
+                           (const int64_t*)w.rowscan, (int32_t*)rp_out, w.nnz);
     TG_LAUNCH_CHECK();
-    int64_t res[2] = {0, 0};
-    TG_HIP(hipMemcpyAsync(&res[0], w.nnz, 8, hipMemcpyDeviceToHost, s));
-    TG_HIP(hipMemcpyAsync(&res[1], w.bad, 8, hipMemcpyDeviceToHost, s));
-    TG_HIP(hipStreamSynchronize(s));
-    if ((int)res[1]) return fail(TG_ERR_INVALID, "from_triples: a row or column index is out of range");
-    if (rp_type == TG_I32 && res[0] > 0x7fffffffll)
+    int64_t nnz = 0;
+    int bad = 0, unfit = 0;
+    const int rc = triples_found(w, &nnz, &bad, &unfit, s);
+    if (rc) return rc;
+    if (bad) return fail(TG_ERR_INVALID, "from_triples: a row or column index is out of range");
+    if (rp_type == TG_I32 && nnz > 0x7fffffffll)
         return fail(TG_ERR_DTYPE, "from_triples: nnz does not fit int32 row pointers");
-    if (nnz_host) *nnz_host = res[0];
+    if (nnz_host) *nnz_host = nnz;
     return TG_OK;
 }
 

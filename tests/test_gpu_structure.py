@@ -87,11 +87,10 @@ def numpy_triples(I, J, V, m, compress, symmetrize):
 @pytest.mark.parametrize("compress,symmetrize", [(True, False), (False, False), (True, True)])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32, None])
 def test_from_triples_forms_agree(cuda, case, compress, symmetrize, dtype):
-    """The bucket form and the radix form, on both sides of every line between them (4095
-    and 4096 triples, rows of at most / more than 512 triples, a bucket that overflows, more
-    columns than a word holds stay out), against a stable sort with the duplicates added in
-    input order: structure and values bit for bit, FP64 / FP32 / none, both row-pointer
-    types."""
+    """The bucket form and the radix form (4095 and 4096 triples, few and many rows, dense
+    ranges of rows, long rows, many columns), against a stable sort with the duplicates added
+    in input order: structure and values bit for bit, FP64 / FP32 / none, both row-pointer
+    types.  The lines between the forms are met in the two tests below."""
     from tensors_amd import _capi as capi
     import ctypes
 
@@ -110,9 +109,9 @@ def test_from_triples_forms_agree(cuda, case, compress, symmetrize, dtype):
         J = I // 16 * 16 + rng.integers(0, 3, cnt)
         J = np.minimum(J, n - 1)
     if case == "long_row":
-        I[::37] = 77  # more than 512 triples: the radix form
+        I[::37] = 77  # a row of more than 800
     if case == "crowded_rows":
-        I[::3] = rng.integers(500, 540, len(I[::3]))  # 40 rows of about 330: a bucket of more than it holds
+        I[::3] = rng.integers(500, 540, len(I[::3]))  # 40 rows of about 330
     I, J = I.astype(np.int32), J.astype(np.int32)
     V = rng.uniform(-1, 1, cnt).astype(dtype or np.float64)
     orp, oci, oval = numpy_triples(I, J, V, m, compress, symmetrize)
@@ -134,6 +133,62 @@ def test_from_triples_forms_agree(cuda, case, compress, symmetrize, dtype):
         assert np.array_equal(ci[:k].cpu().numpy(), oci) and ci[cap].item() == -7
         if dtype:
             assert np.array_equal(va[:k].cpu().numpy(), oval) and va[cap].item() == -7.0
+
+
+def crowd(m, cnt, rows, crowded, seed):
+    """cnt triples over m rows, `crowded` of them in rows 0 .. rows - 1, in random order."""
+    rng = np.random.default_rng(seed)
+    I = np.r_[rng.integers(0, rows, crowded), rng.integers(rows, m, cnt - crowded)]
+    return I[rng.permutation(cnt)].astype(np.int32), rng.integers(0, m, cnt).astype(np.int32)
+
+
+@pytest.mark.parametrize("rows,crowded", [(1, 1535), (1, 1536), (1, 1537), (9, 3071), (9, 3072), (9, 3073), (1, 20000)])
+@pytest.mark.parametrize("compress", [True, False])
+def test_from_triples_crowded_rows(cuda, rows, crowded, compress):
+    """Rows and buckets (here of nine rows) at the sizes that a workgroup just holds and just
+    does not, and a row of two thirds of all triples: the radix form takes over before or
+    after the triples were dealt.  Structure and values bit for bit."""
+    m, cnt = 4001, 30011
+    I, J = crowd(m, cnt, rows, crowded, rows + crowded)
+    V = np.random.default_rng(7).uniform(-1, 1, cnt)
+    rp, ci, val = st.from_triples(I, J, V, m, m, compress, False)
+    orp, oci, oval = numpy_triples(I, J, V, m, compress, False)
+    assert np.array_equal(rp, orp) and np.array_equal(ci, oci) and np.array_equal(val, oval)
+
+
+@pytest.mark.parametrize("m,n,cnt", [(3001, 1 << 29, 50021), (3001, (1 << 29) + 1, 50021),
+                                     (1 << 24, 1 << 24, 40009), ((1 << 24) + 1, (1 << 24) + 1, 40009),
+                                     (1000003, 1000003, 1 << 24), (1000003, 1000003, (1 << 24) + 1)])
+def test_from_triples_at_the_limits_of_a_word(cuda, m, n, cnt):
+    """As many columns, rows (8192 buckets of 2048) and triples (8192 buckets of 2048 triples)
+    as a triple's word and the buckets hold, and one more of each (the radix form), with the
+    last row, column and input position among them.  Integer values: the sums are exact in
+    any order, so the device's own sort serves as the reference."""
+    from tensors_amd import _capi as capi
+    import ctypes
+
+    g = torch.Generator(device=cuda).manual_seed(cnt + n)
+    I = torch.randint(0, m, (cnt,), device=cuda, generator=g, dtype=torch.int32)
+    J = torch.randint(0, n, (cnt,), device=cuda, generator=g, dtype=torch.int32)
+    I[-1], J[-1], I[5], J[5] = m - 1, n - 1, m - 1, n - 1
+    J[1::2] = n - 1 - J[1::2] % 64
+    V = torch.randint(-9, 10, (cnt,), device=cuda, generator=g).double()
+    nb = capi.lib().tg_csr_from_triples_workspace_bytes(cnt, m, 0)
+    ws = torch.empty(nb, dtype=torch.uint8, device=cuda)
+    rp = torch.empty(m + 1, dtype=torch.int32, device=cuda)
+    ci = torch.empty(cnt, dtype=torch.int32, device=cuda)
+    va = torch.empty(cnt, dtype=torch.float64, device=cuda)
+    nnz = ctypes.c_int64(0)
+    print(f"from_triples m {m} n {n} count {cnt}", flush=True)
+    capi.call("tg_csr_from_triples", cnt, I.data_ptr(), J.data_ptr(), V.data_ptr(), capi.F64, m, n, 1, 0,
+              rp.data_ptr(), capi.I32, ci.data_ptr(), va.data_ptr(), cnt, ws.data_ptr(), nb, ctypes.byref(nnz), None)
+    key, where = torch.unique(I.long() * n + J, return_inverse=True)
+    k = key.numel()
+    want = torch.zeros(k, dtype=torch.float64, device=cuda).index_add_(0, where, V)
+    orp = torch.zeros(m + 1, dtype=torch.int64, device=cuda)
+    torch.cumsum(torch.bincount(key // n, minlength=m), 0, out=orp[1:])
+    assert nnz.value == k and torch.equal(rp.long(), orp)
+    assert torch.equal(ci[:k].long(), key % n) and torch.equal(va[:k], want)
 
 
 def test_from_triples_rejects_out_of_range_in_buckets(cuda):

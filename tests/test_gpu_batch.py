@@ -353,3 +353,35 @@ def test_batch_columns_per_lane(cuda, n, k):
     assert rel_err(devs[5].cpu().numpy(), Xo) <= 1e-12
     X, res = run_batch(sysl, cuda, 1, 1e-11)
     assert res[0]["succeeded"] and rel_err(X[0], np.linalg.solve(A.toarray(), B)) <= 3e-11
+
+
+@pytest.mark.parametrize("split", [1, 0], ids=["split", "fused"])
+@pytest.mark.parametrize("mixed", [0, 1, 2], ids=["fp64", "mixed", "fp64_true_residual"])
+def test_steps_after_a_stop_change_nothing(cuda, mixed, split):
+    """7, 23 and 400 steps between polls: systems that stop or pause early sit through hundreds
+    of steps in the last case, without a tile of theirs being touched (x, its deferred
+    update, the iteration count).  Bitwise the same.  (Polls that land on a checkpoint see the
+    residual estimate of the step before it and may replace a residual earlier or later:
+    lengths that divide the 16 steps between checkpoints are left out.)"""
+    from tensors_amd import _capi as capi
+
+    sysl = systems(7, seed=515)
+    before = int(capi.lib().tg_tune_get(b"batch_split"))
+    out = []
+    try:
+        capi.call("tg_tune_set", b"batch_split", split)
+        for steps in (7, 23, 400):
+            bt = BatchCG()
+            devs = [to_dev(s, cuda) for s in sysl]
+            ids = [bt.add(rp, ci, val, B, X, 1e-9, 20000, diag=d, mixed=mixed == 1, true_residual=mixed == 2)
+                   for rp, ci, val, d, B, X in devs]
+            bt.run(steps)
+            res = [bt.result(i) for i in ids]
+            assert all(r["succeeded"] for r in res)
+            out.append(([d[5].cpu() for d in devs], [r["iterations"] for r in res]))
+            bt.close()
+    finally:
+        capi.call("tg_tune_set", b"batch_split", before)
+    for X, its in out[1:]:
+        assert its == out[0][1]
+        assert all(torch.equal(a, b) for a, b in zip(X, out[0][0]))

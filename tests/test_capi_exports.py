@@ -120,3 +120,25 @@ def test_every_documented_knob_reads_back():
         assert L.tg_tune_set(key.encode(), v) == 0, (key, capi.last_error())
         assert int(L.tg_tune_get(key.encode())) == v, key
     assert int(L.tg_tune_get(b"no_such_knob")) == -1
+
+
+def test_stream_handle_without_the_raw_stream_call(monkeypatch):
+    """A torch whose private names for the current stream are gone (either of them): products
+    take the public call."""
+    import importlib.util
+    import types
+
+    import torch
+
+    from tensors_amd import sparse
+
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=4711))
+    for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+        with monkeypatch.context() as gone:
+            gone.delattr(torch._C, name, raising=False)
+            spec = importlib.util.spec_from_file_location("tensors_amd.sparse_of_another_torch", sparse.__file__)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            assert module.stream_handle() == 4711
+            assert module.stream_handle(types.SimpleNamespace(cuda_stream=12)) == 12

@@ -88,10 +88,11 @@ __device__ __forceinline__ void one_dots_rows(int base, int nr, int j, int finis
         const RP l0 = lds.srp[0], l1 = lds.srp[nr];
         T sum = T(0);
         const RP rb = threadIdx.x < nr ? lds.srp[threadIdx.x] : l0, re = threadIdx.x < nr ? lds.srp[threadIdx.x + 1] : l0;
-        // (steps by what was done: cs + CAP may lie past 2^31)
-        for (RP cs = l0, step = 0; cs < l1; cs += step) {
+        // (unsigned: cs + CAP may lie past 2^31)
+        using UP = typename std::make_unsigned<RP>::type;
+        for (UP us = (UP)l0; us < (UP)l1; us += CAP) {
+            const RP cs = (RP)us;
             const int cnt = (int)((l1 - cs) < (RP)CAP ? (l1 - cs) : (RP)CAP);
-            step = (RP)cnt;
             int32_t c[EL];
             T av[EL], xv[EL];
 #pragma unroll

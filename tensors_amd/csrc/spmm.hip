@@ -195,10 +195,11 @@ __global__ __launch_bounds__(kBlock) void spmv_stream_kernel(
         for (int i = threadIdx.x; i < nr * K; i += kBlock) racc[i] = T(0);
         __syncthreads();
         const RP L0 = srp[0], L1 = srp[nr];
-        // (steps by what was done: cs + CAP may lie past 2^31)
-        for (RP cs = L0, step = 0; cs < L1; cs += step) {
+        // (unsigned: cs + CAP may lie past 2^31)
+        using U = typename std::make_unsigned<RP>::type;
+        for (U us = (U)L0; us < (U)L1; us += CAP) {
+            const RP cs = (RP)us;
             const int cnt = (int)((L1 - cs) < (RP)CAP ? (L1 - cs) : (RP)CAP);
-            step = (RP)cnt;
             int32_t c[ELEMS];
             T av[ELEMS];
 #pragma unroll
@@ -293,10 +294,11 @@ __global__ __launch_bounds__(kBlock) void spmm_wave_kernel(
             T acc[V];
 #pragma unroll
             for (int i = 0; i < V; ++i) acc[i] = T(0);
-            // (steps by what was done: base + kWave may lie past 2^31)
-            for (RP base = lb, step = 0; base < le; base += step) {
+            // (unsigned: base + kWave may lie past 2^31)
+            using UP = typename std::make_unsigned<RP>::type;
+            for (UP ub = (UP)lb; ub < (UP)le; ub += kWave) {
+                const RP base = (RP)ub;
                 const int cnt = (int)((le - base) < (RP)kWave ? (le - base) : (RP)kWave);
-                step = (RP)cnt;
                 int32_t myc = 0;
                 T mya = T(0);
                 if (lane < cnt) {

@@ -353,7 +353,14 @@ __global__ __launch_bounds__(kBlock) void spmm_wave_kernel(
 // therefore are ordinary ones (a non-temporal line would be fetched again for each).
 // V columns per lane at any alignment; where V does not divide nrhs the last lane's vector
 // is moved back to end at the last column and stores only its own columns.
-template <typename T, typename RP, int G, int V>
+// FORM: kRowsShort for rows of about one chunk, with a pair per lane from G = 8 on (two pairs
+// of rows of 5-7 are half idle loads: 100^3 grid, k = 16 FP64 118 / 115 us); kRowsStream the
+// same with A past the caches; kRowsLong for rows of several chunks, the next chunk's pairs
+// fetched before this one's gathers (3e5 rows of 12, k = 8 FP64 72 / 65 us; of 8 with one of
+// 7287, k = 5 1181 / 1078: such a row is one chain of round trips).
+enum RowForm : int { kRowPerWave = 0, kRowsShort = 1, kRowsStream = 2, kRowsLong = 3 };
+
+template <typename T, typename RP, int G, int V, int FORM>
 __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(
     int m, const RP* __restrict__ rp, const RP* __restrict__ rpe, const int32_t* __restrict__ ci, const T* __restrict__ a, T alpha,
     const T* __restrict__ X, int64_t ldX, T beta, T* __restrict__ Y, int64_t ldY, int nrhs, int alpha_one,
@@ -363,7 +370,7 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(
     constexpr int KT = G * V;     // columns per tile
     constexpr int WAVES = kBlock / kWave;
     constexpr int U = V * sizeof(T) <= 8 ? 8 : 4;
-    constexpr int PER = G >= 16 ? 1 : G == 8 ? 2 : 8 / G;
+    constexpr int PER = G >= 16 ? 1 : G == 8 ? (FORM == kRowsLong ? 2 : 1) : 8 / G;
     constexpr int CH = G * PER;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int s = lane / G, g = lane % G;
@@ -384,15 +391,32 @@ __global__ __launch_bounds__(kBlock) void spmm_rows_kernel(
             T acc[V];
 #pragma unroll
             for (int i = 0; i < V; ++i) acc[i] = T(0);
+            int32_t nextc[PER];
+            T nexta[PER];
+            auto fetch = [&](int base) {
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    const RP at = max(lb + min(base + g + q * G, len - 1), RP(0));
+                    nextc[q] = ci[at];
+                    nexta[q] = a ? a[at] : T(1);
+                }
+            };
+            if (FORM == kRowsLong && wmax > 0) fetch(0);
             for (int base = 0; base < wmax; base += CH) {
                 int32_t myc[PER];
                 T mya[PER];
 #pragma unroll
                 for (int q = 0; q < PER; ++q) {  // clamped: some row of the wave has a nonzero, so 0 is valid
-                    const RP at = max(lb + min(base + g + q * G, len - 1), RP(0));
-                    myc[q] = ci[at];
-                    mya[q] = a ? a[at] : T(1);
+                    if constexpr (FORM == kRowsLong) {
+                        myc[q] = nextc[q];
+                        mya[q] = nexta[q];
+                    } else {
+                        const RP at = max(lb + min(base + g + q * G, len - 1), RP(0));
+                        myc[q] = FORM == kRowsStream ? __builtin_nontemporal_load(ci + at) : ci[at];
+                        mya[q] = !a ? T(1) : FORM == kRowsStream ? __builtin_nontemporal_load(a + at) : a[at];
+                    }
                 }
+                if (FORM == kRowsLong && base + CH < wmax) fetch(base + CH);
                 const int cnt = min(CH, len - base);  // this group's pairs in the chunk
                 const int wcnt = min(CH, wmax - base);
                 auto round = [&](int u0) {
@@ -679,19 +703,26 @@ static int launch_stream_k(int32_t m, int64_t nnz, const RP* rp, const int32_t* 
 }
 
 template <typename T, typename RP, int V>
-static int launch_spmm_v(int G, bool rows, int32_t m, const RP* rp, const RP* rpe, const int32_t* ci, const T* a,
+static int launch_spmm_v(int G, RowForm rows, int32_t m, const RP* rp, const RP* rpe, const int32_t* ci, const T* a,
                          T alpha,
                          const T* X, int64_t ldX, T beta, T* Y, int64_t ldY, int32_t nrhs, int alpha_one,
                          int beta_mode, const int32_t* job_ptr, int32_t blocks, const int* skip, hipStream_t st) {
-    if (rows && G < kWave) {
+    if (rows != kRowPerWave && G < kWave) {
         // 64/G rows per wave at a time
         const int rpb = (kBlock / G) * rounds_for(m, kBlock / G);
         const int grid = job_ptr ? blocks : (m + rpb - 1) / rpb;
         if (grid <= 0) return TG_OK;
-#define TG_SPMMR(GG)                                                                                          \
-    case GG:                                                                                                  \
-        hipLaunchKernelGGL((spmm_rows_kernel<T, RP, GG, V>), dim3(grid), dim3(kBlock), 0, st, m, rp, rpe, ci, a, alpha, \
-                           X, ldX, beta, Y, ldY, nrhs, alpha_one, beta_mode, job_ptr, rpb, skip);             \
+#define TG_SPMMRF(GG, FF)                                                                                      \
+    hipLaunchKernelGGL((spmm_rows_kernel<T, RP, GG, V, FF>), dim3(grid), dim3(kBlock), 0, st, m, rp, rpe, ci, a, \
+                       alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one, beta_mode, job_ptr, rpb, skip)
+#define TG_SPMMR(GG)                                       \
+    case GG:                                               \
+        if (rows == kRowsLong)                             \
+            TG_SPMMRF(GG, kRowsLong);                      \
+        else if (GG == 8 && rows == kRowsStream)           \
+            TG_SPMMRF(GG, (GG == 8 ? kRowsStream : kRowsShort)); \
+        else                                               \
+            TG_SPMMRF(GG, kRowsShort);                     \
         break;
         switch (G) {
             TG_SPMMR(1)
@@ -703,6 +734,7 @@ static int launch_spmm_v(int G, bool rows, int32_t m, const RP* rp, const RP* rp
             default: return fail(TG_ERR_INVALID, "internal: bad lane group %d", G);
         }
 #undef TG_SPMMR
+#undef TG_SPMMRF
         TG_LAUNCH_CHECK();
         return TG_OK;
     }
@@ -789,16 +821,27 @@ static int spmm_typed(int32_t m, int32_t n, int64_t nnz, int32_t max_row, const 
         }
     }
     const int G = lanes_for(V);
+    // Rows of more than a chunk (mean over 8, or one of over 64 that a plan knows) take the
+    // fetch-ahead form.  In the short form A goes past the caches where X and Y just about fill
+    // the Infinity Cache by themselves (256 MB) and a pass over A would push them out: 1e6 rows
+    // of 5, FP64, cached / streamed: k = 13 (208 + 64 MB) 76 / 80 us, 14 (224 + 64) 82 / 80, 16 (256 +
+    // 64) 91 / 84; k = 10 59 / 74, 32 168 / 172.
+    const int64_t vectors = ((int64_t)m + n) * nrhs * (int64_t)sizeof(T), cache = 256ll << 20;
+    const int64_t all = vectors + nnz * (int64_t)(sizeof(T) + 4) + (int64_t)m * (int64_t)sizeof(RP);
+    const RowForm form = !rows                        ? kRowPerWave
+                         : avg > 8.0 || max_row > 64  ? kRowsLong
+                         : vectors <= cache && all > cache + (cache >> 5) ? kRowsStream
+                                                                         : kRowsShort;
     switch (V) {
         case 1:
-            return launch_spmm_v<T, RP, 1>(G, rows, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
+            return launch_spmm_v<T, RP, 1>(G, form, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
                                            beta_mode, job_ptr, blocks, skip, st);
         case 2:
-            return launch_spmm_v<T, RP, 2>(G, rows, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
+            return launch_spmm_v<T, RP, 2>(G, form, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
                                            beta_mode, job_ptr, blocks, skip, st);
         default:
             if constexpr (sizeof(T) == 4)
-                return launch_spmm_v<T, RP, 4>(G, rows, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
+                return launch_spmm_v<T, RP, 4>(G, form, m, rp, rpe, ci, a, alpha, X, ldX, beta, Y, ldY, nrhs, alpha_one,
                                                beta_mode, job_ptr, blocks, skip, st);
             return fail(TG_ERR_INVALID, "internal: bad vector width");
     }

@@ -383,3 +383,54 @@ def test_int32_row_pointers_up_to_the_last_entry(cuda, m, nrhs, dtype):
     ones = (rp[1:] - rp[:-1].clamp(min=nnz - 3000)).clamp_(min=0)  # entries of a row in column 1
     want = (rp[1:] - rp[:-1] - ones).to(dtype)[:, None] * X[0] + ones.to(dtype)[:, None] * X[1]
     assert torch.equal(Y, want)
+
+
+@pytest.mark.parametrize("dtype,k", [(torch.float64, 15), (torch.float64, 16), (torch.float32, 30), (torch.float32, 32)])
+def test_short_rows_with_vectors_that_fill_the_cache(cuda, dtype, k):
+    """X and Y of 240-256 MB with a matrix of 44-64 MB beside them: the short-row form that
+    streams A.  Five diagonals and X of small integers, so every sum is exact; an update of Y,
+    rows cut off at both ends, a last lane that shares columns with the one before (k = 15, 30)."""
+    n = 1000003
+    i = torch.arange(n, device=cuda)
+    off = (-1000, -1, 0, 1, 1000)
+    cols = torch.stack([i + d for d in off], 1)
+    keep = (cols >= 0) & (cols < n)
+    vals = torch.stack([(i * 7 + 3 * j) % 11 - 5 for j in range(5)], 1).to(dtype)
+    rp = torch.zeros(n + 1, dtype=torch.int64, device=cuda)
+    torch.cumsum(keep.sum(1), 0, out=rp[1:])
+    A = MatrixCSR.from_device(rp.to(torch.int32), cols[keep].to(torch.int32), vals[keep], n, n)
+    X = ((i[:, None] * 5 + torch.arange(k, device=cuda) * 3) % 13 - 6).to(dtype)
+    Y = ((i[:, None] + torch.arange(k, device=cuda)) % 9).to(dtype)
+    want = -Y
+    for j, d in enumerate(off):
+        lo, hi = max(0, -d), min(n, n - d)
+        want[lo:hi] += 2 * vals[lo:hi, j, None] * X[lo + d:hi + d]
+    A.Dot(2.0, X, -1.0, Y)
+    assert torch.equal(Y, want)
+
+
+@pytest.mark.parametrize("longest", [9, 64, 65, 66, 700])
+@pytest.mark.parametrize("dtype,k", [(torch.float64, 5), (torch.float64, 11), (torch.float64, 32), (torch.float32, 7),
+                                     (torch.float32, 18), (torch.float32, 60)])
+def test_short_rows_with_one_long_row(cuda, dtype, k, longest):
+    """Rows of about five nonzeros and one of up to / more than 64, which sends the product to the
+    form that fetches a chunk of pairs ahead: chunks of 8, 16 and 32 pairs and their
+    remainders, empty rows beside the long one.  Integers: every sum is exact."""
+    import scipy.sparse as sp
+
+    m, n = 3001, 2003
+    rng = np.random.default_rng(longest * 100 + k)
+    S = sp.random(m, n, density=5 / n, format="csr", random_state=3)
+    S.data = rng.integers(-4, 5, S.nnz).astype(np.float64)
+    S = S.tolil()
+    S[1000:1040] = 0
+    S[1017, rng.choice(n, longest, replace=False)] = 3
+    S = S.tocsr()
+    S.sort_indices()
+    assert np.diff(S.indptr).max() >= longest
+    X = rng.integers(-3, 4, (n, k)).astype(np.float64)
+    A = MatrixCSR(S.indptr.astype(np.int32), S.indices, S.data.astype(np.float64 if dtype == torch.float64 else np.float32),
+                  m, n)
+    Y = torch.full((m, k), 7.0, dtype=dtype, device=cuda)
+    A.Dot(1.0, torch.from_numpy(X).to(cuda).to(dtype), 0.0, Y)
+    assert np.array_equal(Y.double().cpu().numpy(), S @ X)

@@ -50,7 +50,7 @@ def fused_knob():
     capi.call("tg_tune_set", b"cg_fused", before)
 
 
-@pytest.mark.parametrize("form", [3, 0, 2], ids=["default", "four_kernels", "fused_direction"])
+@pytest.mark.parametrize("form", [3, 0, 1, 2], ids=["default", "four_kernels", "spmm_dot", "fused_direction"])
 @pytest.mark.parametrize("steps", [1, 5, 20])
 @pytest.mark.parametrize("prec", [False, True], ids=["identity", "jacobi"])
 @pytest.mark.parametrize("k", [1, 8])
@@ -150,15 +150,18 @@ def panel_knob():
     capi.call("tg_tune_set", b"cg_panel", before)
 
 
+@pytest.mark.parametrize("form", [1, 2], ids=["spmm_dot", "fused_direction"])
 @pytest.mark.parametrize("panel", [1, 0], ids=["panel_order", "contiguous"])
 @pytest.mark.parametrize("prec", [False, True], ids=["identity", "jacobi"])
-def test_cg_fixed_iterations_panel_order(cuda, panel_knob, panel, prec):
-    """The SpMM of the default iteration with its rows in panel order: the 7-point
-    Laplacian (+ 0.1) of a 128 x 64 x 8 grid, x fastest, has band 8192, so the rows are
-    cut into 8 panels of one plane and every workgroup takes 4 offsets of each (knob
-    cg_panel = 1, the default); the contiguous chunks (cg_panel = 0) for comparison.  Both
-    at 1e-12 from the oracle after 20 steps (a well-conditioned operator, so that 20 steps
-    do not amplify rounding past that bar)."""
+def test_cg_fixed_iterations_panel_order(cuda, fused_knob, panel_knob, form, panel, prec):
+    """The SpMM kernels of both fused forms with their rows in panel order: form 1's, which
+    the large solves take, and form 2's.  The 7-point Laplacian (+ 0.1) of a 128 x 64 x 8
+    grid, x fastest, has band 8192, so the rows are cut into 8 panels of one plane and every
+    workgroup takes a run of offsets of each (4 with form 1's 2048 workgroups; knob
+    cg_panel = 1, the default); the contiguous chunks (cg_panel = 0) for comparison.  All at
+    1e-12 from the oracle after 20 steps (a well-conditioned operator, so that 20 steps do
+    not amplify rounding past that bar)."""
+    fused_knob(form)
     panel_knob(panel)
 
     def path(m):
@@ -179,7 +182,7 @@ def test_cg_fixed_iterations_panel_order(cuda, panel_knob, panel, prec):
     Xd = torch.zeros(n, k, dtype=torch.float64, device=cuda)
     cg(MatrixCSR(rp.astype(np.int32), ci, val, n, n), None if d is None else dev(d, cuda), 1.0, dev(B, cuda), 0.0,
        Xd, 0.0)
-    print(f"CG panel {panel} prec {prec}")
+    print(f"CG form {form} panel {panel} prec {prec}")
     assert cg.IterationCount() == it_o == steps
     assert rel_err(Xd.cpu().numpy(), Xo) <= TOL
     assert res_err(cg.RelativeResiduals(), rr_o) <= TOL

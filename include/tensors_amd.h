@@ -229,9 +229,10 @@ int tg_csr_spmm_plan(tg_csr_plan_t plan, const void* a, tg_dtype val_type, doubl
  *   "bsr_vector":  tg_bsr_spmm with row-major X / Y chunks, 1 = a lane per
  *                  (block row, 1-4 right-hand sides) with vector loads, or for
  *                  many square blocks of side 2, 3, 4, 6 or 8 the blocks through
- *                  LDS where that is faster (default; bitwise the same),
- *                  0 = a lane per output entry (the mapping of the other
- *                  storage orders).
+ *                  LDS where that is faster (default; bitwise the same, but there
+ *                  a block row far longer than the mean is added in parts and
+ *                  agrees to rounding), 0 = a lane per output entry (the mapping
+ *                  of the other storage orders).
  *   "gbatch_big_tiles": systems added to a batched GMRES engine with more than
  *                  this many 1024-row tiles (default 64) get each reduction's totals
  *                  from one workgroup per system instead of every tile workgroup

@@ -211,6 +211,12 @@ __global__ __launch_bounds__(kBlock) void bsr_spmm_vec_kernel(int mb, int R, int
 // 3 x 3 doubles, k = 4 (637 MB): 191 us before, 193 staged, 158 with that (4.0 TB/s).
 // `rows` block rows a workgroup (blockDim.x >= rows * lanes), lanes = (B / PR) * ceil(k / V);
 // where V does not divide k the last lane's columns start at k - V and it writes its own.
+// A workgroup with far more blocks than planned (kLongChunks chunks) holds a long row, which
+// would be one lane group's chain of round trips: it takes its rows one after the other, each
+// row's blocks dealt over all lane groups, whose sums meet in LDS (one of 20000 rows with 8000
+// blocks of side 4, 5 columns FP32: 1.46 ms in chunks, 0.12 so, 0.73 in the kernel above).
+constexpr int kLongChunks = 8;
+
 template <typename T, int B, int V, bool A_RM>
 __global__ __launch_bounds__(kBlock) void bsr_staged_kernel(int mb, int k, const void* __restrict__ rp, int rp64,
                                                             const int32_t* __restrict__ ci, const T* __restrict__ A,
@@ -231,6 +237,66 @@ __global__ __launch_bounds__(kBlock) void bsr_staged_kernel(int mb, int k, const
     const int r0 = part / kv * PR, hv = part % kv * V, h0 = min(hv, k - V), own = hv - h0;
     const int64_t first = at(i0), end = at(i1);
     const int64_t lo = on ? at(i) : 0, hi = on ? at(i + 1) : 0;
+    // Y of the lane's part of row `to`, from its sums
+    auto write = [&](int to, bool none, const T (&sum)[PR][V]) {
+        T* yp = Y + ((int64_t)to * B + r0) * k + h0;
+#pragma unroll
+        for (int r = 0; r < PR; ++r) {
+            T y[V];
+            if (beta_mode != kBsrBetaZero) load_vec_at<T, V>(yp + r * k, y);
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                T out = alpha_one ? sum[r][v] : alpha * sum[r][v];
+                if (none) out = T(0);  // WriteYZero: Y_i <- beta Y_i
+                if (beta_mode == kBsrBetaOne)
+                    out = none ? y[v] : out + y[v];
+                else if (beta_mode == kBsrBetaGeneric)
+                    out = none ? beta * y[v] : out + beta * y[v];
+                y[v] = out;
+            }
+            if (own == 0) {
+                store_vec_at<T, V>(yp + r * k, y);
+            } else {
+#pragma unroll
+                for (int v = 1; v < V; ++v)
+                    if (v >= own) yp[r * k + v] = y[v];
+            }
+        }
+    };
+    if (rows > 1 && end - first > (int64_t)kLongChunks * cap) {
+        constexpr int N = PR * V;  // sums of a lane, in as[]: rows * lanes * N (the host's size covers them)
+        for (int to = i0; to < i1; ++to) {
+            const int64_t from = at(to), till = at(to + 1);
+            T sum[PR][V] = {};
+            for (int64_t q = from + row; row < rows && q < till; q += rows) {
+                const T* xp = X + (int64_t)ci[q] * B * k + h0;
+                const T* ap = A + q * BB;
+#pragma unroll
+                for (int c = 0; c < B; ++c) {
+                    T xv[V];
+                    load_vec_at<T, V>(xp + c * k, xv);
+#pragma unroll
+                    for (int r = 0; r < PR; ++r) {
+                        const T av = ap[A_RM ? (r0 + r) * B + c : c * B + r0 + r];
+#pragma unroll
+                        for (int v = 0; v < V; ++v) sum[r][v] += av * xv[v];
+                    }
+                }
+            }
+            __syncthreads();
+            if (row < rows)
+#pragma unroll
+                for (int e = 0; e < N; ++e) as[(int)threadIdx.x * N + e] = sum[e / V][e % V];
+            __syncthreads();
+            if (row == 0) {
+                for (int g = 1; g < rows; ++g)
+#pragma unroll
+                    for (int e = 0; e < N; ++e) sum[e / V][e % V] += as[(g * lanes + part) * N + e];
+                write(to, till == from, sum);
+            }
+        }
+        return;
+    }
     T acc[PR][V] = {};
     for (int64_t q0 = first; q0 < end; q0 += cap) {
         const int nq = (int)min((int64_t)cap, end - q0), len = nq * BB;
@@ -293,29 +359,60 @@ __global__ __launch_bounds__(kBlock) void bsr_staged_kernel(int mb, int k, const
         }
         __syncthreads();
     }
-    if (!on) return;
-    T* yp = Y + ((int64_t)i * B + r0) * k + h0;
-#pragma unroll
-    for (int r = 0; r < PR; ++r) {
-        T y[V];
-        if (beta_mode != kBsrBetaZero) load_vec_at<T, V>(yp + r * k, y);
-#pragma unroll
-        for (int v = 0; v < V; ++v) {
-            T out = alpha_one ? acc[r][v] : alpha * acc[r][v];
-            if (hi == lo) out = T(0);  // WriteYZero: Y_i <- beta Y_i
-            if (beta_mode == kBsrBetaOne)
-                out = hi == lo ? y[v] : out + y[v];
-            else if (beta_mode == kBsrBetaGeneric)
-                out = hi == lo ? beta * y[v] : out + beta * y[v];
-            y[v] = out;
-        }
-        if (own == 0) {
-            store_vec_at<T, V>(yp + r * k, y);
-        } else {
-#pragma unroll
-            for (int v = 1; v < V; ++v)
-                if (v >= own) yp[r * k + v] = y[v];
-        }
+    if (on) write(i, hi == lo, acc);
+}
+
+// Whether blocks go through LDS.  They do where bsr_spmm_vec_kernel has one column a lane (odd k)
+// or two (k % 4 == 2), or fewer tiles of four columns than its power of two of lanes, and for
+// FP64 blocks of side 4 and 8 from k = 16.  Longer rows (mean over 7) are a longer chain for a
+// staged lane, and a small product does not fill the chip to hide it; factors old / staged:
+//   rows of 4-7 blocks, 8e4 to 4e5 of them: odd k >= 5 1.0-2.7, k % 4 == 2 FP64 1.0-1.5, FP32
+//     1.0-1.7, k = 3 FP64 up to side 6 1.0-1.6 and FP32 up to side 3 1.1-1.4, side 3 FP64 1.0-1.6,
+//     side 6 FP64 k >= 8 1.1-1.9, side 8 1.0-2.8.  Not taken: side 2 k = 4 and, FP64, k % 4 == 2
+//     (0.9), side 4 FP32 k = 16, 64 (0.6-1.1) and FP64 k = 64 (0.9-1.0), side 6 FP32 k = 8 below 2^18
+//     blocks (0.8-1.3), side 8 FP64 k = 6 below 2^17 (0.9).
+//   rows of 7-16, k <= 8: 0.5-1.4 at 8e4, 0.6-1.6 at 1.5e5 but for odd k of side 6 and 8 (0.9-1.5)
+//     and, from 1.5e5, side 4 and 7 columns of side 3 FP64 (1.1-1.4); at 4e5 1.0-2.5 for odd k, FP32
+//     k = 6 from side 3 on, side 3 FP64 but k = 4, k = 3 FP64 of side 6; the same from 2.7e5 on, but
+//     FP32 sides 2 and 3 with rows over 11 (0.8-0.9).  k > 16 1.2-2.3 (side 2 FP32, 7e4: 0.8-1.0);
+//     k = 9-15 1.0-2.0, but below 2^17 blocks side 3 (0.9-1.0) and even k up to side 6 (0.9-1.2), below 2^18
+//     even k of side 3 and FP64 side 6 (0.8-1.0), and rows over 11 of side 2 and 3 (0.5-0.9) and,
+//     below 2^17, FP32 of side 4 and 6 (0.7-0.9).
+//   below 65536 blocks: k >= 24 1.0-3.1, FP64 side 6 and 8 with odd k and side 6 from k = 12 1.0-1.6;
+//     the rest 0.6-1.2 in the kernel (6000 rows of 6, side 6, k = 8 FP32 8.6 against 11.0 us).
+//   Side 3 FP64 with 15 of 16 lanes busy (k = 10, 20) 0.8-0.9 for rows of 4-7.
+// Rows of 1-3 mean reading past them (0.6-1.2), rows of 27 leave a workgroup few rows (0.5-1.7).
+// Other sides (1, 5, 7) keep the mapping above: a staged lane takes one to three whole rows of a
+// block, and sides that its rows do not divide were not written.
+static bool bsr_staged_pays(int side, int k, bool fp64, int64_t nnzb, int64_t mb) {
+    if (k > 64 || nnzb < 32768 || nnzb < 4 * mb || nnzb > 16 * mb) return false;
+    const bool longer = nnzb > 7 * mb, longest = nnzb > 11 * mb, many = nnzb >= (1 << 18), some = nnzb >= (1 << 17);
+    const bool odd = k % 2 && k >= 5;
+    if (nnzb < 65536 && k < 24 && !(fp64 && side >= 6 && (odd || (side == 6 && k >= 12)))) return false;
+    const bool enough = nnzb >= (!fp64 && side <= 3 && k < 9 && longest ? 3 << 17 : 1 << 18);
+    const int tiles = side * k / (k % 4 == 0 ? 4 : k % 2 == 0 ? 2 : 1);
+    int lanes = 1;
+    while (lanes < tiles) lanes *= 2;
+    if (side == 3 && fp64 && k % 2 == 0 && !longer && 8 * tiles > 7 * lanes) return false;
+    if (k % 4) {
+        if (k < 3 || (k == 3 && side > (fp64 ? 6 : 3)) || (k % 4 == 2 && side == 2 && fp64)) return false;
+        if (!longer) return !(k == 6 && side == 8 && fp64) || some;
+        if (enough) return k != 3 ? odd || k > 6 || (fp64 ? side == 3 : side >= 3) : fp64 && side % 3 == 0;
+        if (k > 16) return side > 2 || (longest ? fp64 && some : fp64 || some);
+        if (k >= 9 && !longest)
+            return k % 2 == 0 ? side == 8 || (some && side != 3 && !(side == 6 && fp64)) : side != 3 || some;
+        if (k >= 9) return side == 8 || (side == 6 && (fp64 ? odd : some)) || (side == 4 && (fp64 || some));
+        if (!odd) return false;
+        if (side == 6) return longest ? k == 7 && (fp64 || some) : fp64 || k == 7;
+        return side == 8 || (some && (side == 4 ? fp64 || (k == 7 && !longest) : fp64 && side == 3 && k == 7));
+    }
+    const bool idle = lanes != tiles;
+    switch (side) {
+        case 3: return fp64 && (!longer || k > 8 || (k == 8 && many));
+        case 4: return k >= 16 && (fp64 ? idle || k <= 32 : idle && (!longer || some));
+        case 6: return k > 8 ? fp64 || !longest || some || k > 32 : k == 8 && (fp64 ? !longer || many : !longer && many);
+        case 8: return k >= 16 && (idle || fp64 || k > 32 || !longer || many);
+        default: return false;
     }
 }
 
@@ -337,8 +434,17 @@ static int launch_bsr_staged(int mb, int64_t nnzb, int k, const void* rp, int rp
     cap = (int)std::min<int64_t>(cap, std::max<int64_t>(rows * mean, 8));
     const int threads = (rows * lanes + kWave - 1) / kWave * kWave;
     const dim3 grid((unsigned)((mb + rows - 1) / rows));
-    const size_t shared = (size_t)cap * bytes;
-#define TG_BSRS(VV)                                                                                                      do {                                                                                                                     if (a_rm)                                                                                                                hipLaunchKernelGGL((bsr_staged_kernel<T, B, VV, true>), grid, dim3(threads), shared, s, mb, k, rp, rp64,                                ci, A, alpha, X, beta, Y, rows, lanes, cap, alpha_one, beta_mode);                            else                                                                                                                     hipLaunchKernelGGL((bsr_staged_kernel<T, B, VV, false>), grid, dim3(threads), shared, s, mb, k, rp,                                     rp64, ci, A, alpha, X, beta, Y, rows, lanes, cap, alpha_one, beta_mode);                  } while (0)
+    // (a lane's sums of a long row need less: at most 256 lanes of 6 FP64 or 12 FP32 values)
+    const size_t shared = std::max((size_t)cap * bytes, (size_t)threads * PR * V * sizeof(T));
+#define TG_BSRS(VV)                                                                                             \
+    do {                                                                                                        \
+        if (a_rm)                                                                                               \
+            hipLaunchKernelGGL((bsr_staged_kernel<T, B, VV, true>), grid, dim3(threads), shared, s, mb, k, rp,  \
+                               rp64, ci, A, alpha, X, beta, Y, rows, lanes, cap, alpha_one, beta_mode);         \
+        else                                                                                                    \
+            hipLaunchKernelGGL((bsr_staged_kernel<T, B, VV, false>), grid, dim3(threads), shared, s, mb, k, rp, \
+                               rp64, ci, A, alpha, X, beta, Y, rows, lanes, cap, alpha_one, beta_mode);         \
+    } while (0)
     if constexpr (sizeof(T) == 4) {
         if (V == 4) {
             TG_BSRS(4);
@@ -431,21 +537,7 @@ static int bsr_typed(int32_t mb, int64_t nnzb, int32_t R, int32_t C, const RP* r
         return TG_OK;
     }
     const int alpha_one = alpha_d == 1.0;
-    // Staged blocks where bsr_spmm_vec_kernel reads narrow vectors or leaves lanes of its
-    // groups idle: k % 4 != 0 (200 000 / B rows of 7 blocks, old against staged, factors
-    // 1.1-2.5 for k = 5, 6, 7 and every B; k = 3: FP64 1.2-1.9 up to B = 6 and 0.86 at B = 8, FP32
-    // 1.1-1.4 up to B = 3 and 0.96-1.05 above; k = 1, 2: 0.7-1.0, not taken), three FP64 block
-    // rows (k = 4 1.15, 8 1.3, 16 1.4), B = 6 from k = 8 (1.1-2.1), B = 4 and 8 from k = 16
-    // (1.1-1.7), B = 2 with four FP32 columns (1.15); in the rest it loses (B = 2, k = 16 0.8; B = 4
-    // or 8, k = 4 0.7-0.9).  Rows of 1-2 blocks mean reading past them (0.6-1.2), rows of 27 leave
-    // a workgroup few rows (0.5-1.7), and with fewer than 32768 blocks the chip is not full and the
-    // longer chain shows (300 rows of 27: 0.6-1.1).
-    const bool fp64 = sizeof(T) == 8;
-    const bool narrow = k % 4 != 0 ? k >= 5 || (k == 3 && R <= (fp64 ? 6 : 3))
-                        : R == 2   ? k == 4 && !fp64
-                        : R == 3   ? fp64
-                                   : k >= (R == 6 ? 8 : 16);
-    const bool staged = narrow && k <= 64 && nnzb >= 32768 && nnzb >= 4 * (int64_t)mb && nnzb <= 16 * (int64_t)mb;
+    const bool staged = bsr_staged_pays(R, k, sizeof(T) == 8, nnzb, mb);
     if (x_rm && y_rm && g_bsr_vector && R == C && staged) {
 #define TG_BSR_STAGED(BB)                                                                                             \
     case BB:                                                                                                          \

@@ -145,7 +145,7 @@ def test_fill_lower_matches_oracle(cuda, R):
 @pytest.mark.parametrize("B", [2, 3, 4, 6, 8])
 @pytest.mark.parametrize("k", [3, 4, 5, 8, 16, 61])
 @pytest.mark.parametrize("a_rm", [1, 0])
-def test_bsr_staged_blocks_equal_entry_mapping(cuda, B, k, a_rm):
+def test_bsr_staged_blocks_equal_entry_mapping(cuda, B, k, a_rm, mb=6001, longer=()):
     """Blocks through LDS (square blocks, many rows) against the entry mapping (knob bsr_vector =
     0): integer data, so both are exact and equal bit for bit.  Rows of 0 to 12 blocks and one longer
     than a chunk, the last group short, k with whole and shifted last vectors, X and Y at odd
@@ -153,9 +153,11 @@ def test_bsr_staged_blocks_equal_entry_mapping(cuda, B, k, a_rm):
     from tensors_amd import _capi as capi
 
     rng = np.random.default_rng(10 * B + k)
-    mb, nb = 6001, 4000
+    nb = 4000
     cnt = rng.integers(0, 13, mb)
     cnt[1234] = 1500
+    for row, blocks in longer:
+        cnt[row] = blocks
     rp = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int64)
     assert rp[-1] >= 32768
     ci = np.concatenate([np.sort(rng.choice(nb, c, replace=False)) for c in cnt]).astype(np.int32)
@@ -180,3 +182,14 @@ def test_bsr_staged_blocks_equal_entry_mapping(cuda, B, k, a_rm):
                 assert torch.equal(*out), (dtype, alpha, beta)
     finally:
         capi.call("tg_tune_set", b"bsr_vector", before)
+
+
+@pytest.mark.parametrize("B", [2, 3, 4, 6, 8])
+@pytest.mark.parametrize("k", [3, 4, 5, 6, 7, 8, 9, 12, 16, 61, 64])
+@pytest.mark.parametrize("a_rm", [1, 0])
+def test_bsr_staged_blocks_with_long_rows(cuda, B, k, a_rm):
+    """The same with enough blocks for every staged form, and long rows one after the other, at both
+    ends and of lengths about a chunk: their blocks are dealt over the lane groups of a wave,
+    one to thirty of them, where a row takes a whole chunk."""
+    longer = [(0, 700), (1235, 3999), (1236, 40), (1240, 270), (2000, 860), (2001, 855), (13000, 2222)]
+    test_bsr_staged_blocks_equal_entry_mapping(cuda, B, k, a_rm, 13001, longer)

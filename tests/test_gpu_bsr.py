@@ -189,7 +189,8 @@ def test_bsr_staged_blocks_equal_entry_mapping(cuda, B, k, a_rm, mb=6001, longer
 @pytest.mark.parametrize("a_rm", [1, 0])
 def test_bsr_staged_blocks_with_long_rows(cuda, B, k, a_rm):
     """The same with enough blocks for every staged form, and long rows one after the other, at both
-    ends and of lengths about a chunk: their blocks are dealt over the lane groups of a wave,
-    one to thirty of them, where a row takes a whole chunk."""
-    longer = [(0, 700), (1235, 3999), (1236, 40), (1240, 270), (2000, 860), (2001, 855), (13000, 2222)]
+    ends and of lengths about a chunk: the blocks of a workgroup's rows are dealt over all its lane
+    groups where they come to more than eight chunks (6824 blocks of side 2 FP32, 312 of side 8 FP64),
+    and go chunk by chunk up to there."""
+    longer = [(0, 700), (1235, 3999), (1236, 40), (1237, 3100), (1240, 270), (2000, 860), (2001, 855), (13000, 422)]
     test_bsr_staged_blocks_equal_entry_mapping(cuda, B, k, a_rm, 13001, longer)

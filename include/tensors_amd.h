@@ -218,12 +218,14 @@ int tg_csr_spmm_plan(tg_csr_plan_t plan, const void* a, tg_dtype val_type, doubl
  *                  tg_gmres_solve_mixed), 1 = CGS2 with each vector's second pass
  *                  delayed to the next step and fused with its projection (default
  *                  for restart lengths up to 32 and (2m + 2) * nrhs <= 2048: two
- *                  passes over the basis and five launches per step), 0 = CGS2
+ *                  passes over the basis and five launches per step, two or three
+ *                  with one right-hand side, see "gmres_split_dots"), 0 = CGS2
  *                  (three passes, eight launches).  Results agree to rounding.
  *   "gmres_split_dots": delayed steps with one right-hand side, 1 = the basis
  *                  vectors dealt over the waves of a workgroup, two or three
  *                  kernels a step with the product among them for CSR operators of
- *                  short rows (default); 0 = every vector on every lane, a kernel
+ *                  short rows on average (default; a row far longer is added in
+ *                  parts); 0 = every vector on every lane, a kernel
  *                  each for the product, dots, totals, scalars and update.
  *                  Results agree to rounding.
  *   "bsr_vector":  tg_bsr_spmm with row-major X / Y chunks, 1 = a lane per

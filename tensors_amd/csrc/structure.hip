@@ -194,7 +194,7 @@ static int triples_found(const TriplesWs& w, int64_t* nnz, int* bad, int* unfit,
 //               entries to the bucket's place of a temporary, row starts within the bucket
 //   bk_offsets  scan of the merged counts
 //   bk_out      copies each bucket's entries to the result and writes its row pointers
-// The same case takes 345 us (shuffled triples deal in 273).  A bucket that does not fit (more than
+// The same case takes 348 us (580 shuffled, the deal 239 of it for 74).  A bucket that does not fit (more than
 // kBkCap triples, or a row of more than kBkRow) raises a flag, and the radix form runs
 // instead: too many triples before any is dealt, with the kernels that follow returning at
 // once.  Radix form alone (64 bits) / with the attempt in front: 1.05e7 triples with a row of
